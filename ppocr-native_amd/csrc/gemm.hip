@@ -30,8 +30,12 @@
 
 #include "act.hpp"
 #include "kernels.hpp"
+#include "split.hpp"
 
 namespace ppocr {
+
+// What loads outside an operand read.
+__device__ __attribute__((aligned(16))) float kRingZeros[4];
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -843,26 +847,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
 // then a fused multiply-add per input in order, src/engine/layers.rs:770-776),
 // and takes the first column of their maximum.
 //
-// `tie` bounds how far the two orders can put two columns' logits apart:
-// each order computes bias + sum of ci products with at most n = ci + 1
-// roundings, so each lies within n u T of the exact sum (u = 2^-24, T =
-// |bias| + sum |w_i x_i| <= bias_max + wsum_max * max |x_i|), the two orders
-// within 2 n u T of each other, and two columns' differences within 4 n u T.
-// The test takes twice that (8 n u T, which also covers an accumulation that
-// rounds toward zero), so columns further below the maximum on the GPU are
-// below it in the CPU's order too.
+// `tie` bounds how far the two orders can put two columns' logits apart (u =
+// 2^-24, T = |bias| + sum |w_i x_i| <= bias_max + wsum_max * max |x_i|): the
+// CPU's bias + sum of ci products has n = ci + 1 roundings, each at most u T.
+// The panel's six products of split parts leave out at most 2 u T; its hi
+// accumulator rounds at most ci times, its lo one at most 5 ci times at sums
+// below 2^-6.9 T (0.042 ci u T), and joining them and the bias rounds twice:
+// (1.042 ci + 4) u T. So two columns' differences lie within (4.1 ci + 10)
+// u T of each other. The test takes 8 n u T, which from ci = 4 on also covers
+// accumulations that round toward zero, so columns further below the maximum
+// on the GPU are below it in the CPU's order too.
 constexpr float kCtcUnit = 1.0f / 16777216.0f;  // 2^-24
 
 
-__global__ __launch_bounds__(256) void ctc_merge(const float4 *part, int rows, int ntiles, float *y,
+__global__ __launch_bounds__(256) void ctc_merge(const float4 *part, int rows, int ntiles, int run, float *y,
                                                  long y_lane_stride, int rows_per_lane, CtcExact ex) {
   int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   int lane = threadIdx.x & 63;
   if (row >= rows) return;
   CtcState st{-__builtin_inff(), 0.0f, __builtin_inff()};
   float m2 = -__builtin_inff();
-  for (int t = lane; t < ntiles; t += 64) {
-    float4 p = part[(long)row * ntiles + t];
+  for (int t = lane; t * run < ntiles; t += 64) {
+    // A run's records, joined in column order as a workgroup that walks the
+    // whole run joins them.
+    const float4 *rec = part + (long)row * ntiles + t * run;
+    float4 p = rec[0];
+    for (int q = 1; q < run && t * run + q < ntiles; q++) p = ctc_join_partial(p, rec[q]);
     float n1, n2;
     top2(st.m, m2, p.x, p.w, n1, n2);
     m2 = n2;
@@ -898,7 +908,7 @@ __global__ __launch_bounds__(256) void ctc_merge(const float4 *part, int rows, i
     // the wave joins the lanes once at the end, the same total order.
     float bm = -__builtin_inff(), bb = __builtin_inff();
     int c0s[4] = {0, 0, 0, 0}, c1s[4] = {0, 0, 0, 0}, nq = 0;
-    auto run = [&]() {
+    auto recompute = [&]() {
       float v[4];
       const float *w[4];
       bool ok[4];
@@ -911,7 +921,8 @@ __global__ __launch_bounds__(256) void ctc_merge(const float4 *part, int rows, i
         v[k] = ex.bias[cc];
       }
       int i = 0;
-      for (; i + 4 <= ex.ci; i += 4) {
+#pragma unroll 6
+      for (; i + 4 <= ex.ci; i += 4) {  // six groups' loads in flight (one at a time: 11 us more)
         const float x0 = x[i], x1 = x[i + 1], x2 = x[i + 2], x3 = x[i + 3];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -932,17 +943,21 @@ __global__ __launch_bounds__(256) void ctc_merge(const float4 *part, int rows, i
       }
       nq = 0;
     };
-    for (int t = 0; t < ntiles; t++) {
-      if (part[(long)row * ntiles + t].x < st.m - tie) continue;
-      const int c1 = min((t + 1) * ex.tile_n, ex.vocab);
-      for (int c0 = t * ex.tile_n; c0 < c1; c0 += 64) {
-        // A record over several tiles: only its tiles whose own maximum is close.
-        if (ex.tmax && ex.tmax[(long)(c0 / 64) * rows + row] < st.m - tie) continue;
-        c0s[nq] = c0, c1s[nq] = min(c0 + 64, c1), nq++;
-        if (nq == 4) run();
+    // The 64-column tiles whose own maximum is close, found 64 tiles at a
+    // time (a lane each), in column order.
+    const int units = ex.tmax ? ex.tmax_n : ntiles;
+    for (int u0 = 0; u0 < units; u0 += 64) {
+      const int u = min(u0 + lane, units - 1);
+      const float um = ex.tmax ? ex.tmax[(long)u * rows + row] : part[(long)row * ntiles + u].x;
+      unsigned long long near = __ballot(u0 + lane < units && !(um < st.m - tie));
+      while (near) {
+        const int t = u0 + __builtin_ctzll(near);
+        near &= near - 1;
+        c0s[nq] = t * 64, c1s[nq] = min(t * 64 + 64, ex.vocab), nq++;
+        if (nq == 4) recompute();
       }
     }
-    if (nq) run();
+    if (nq) recompute();
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
       const float ov = __shfl_xor(bm, d, 64), ob = __shfl_xor(bb, d, 64);
@@ -959,130 +974,152 @@ __global__ __launch_bounds__(256) void ctc_merge(const float4 *part, int rows, i
 
 // ------------------------------------------------------------ CTC, panels
 
-// The CTC head's GEMM when the head's input is at most 128 wide. A
-// workgroup keeps 128 rows (eight waves of 16) in its operand registers for
-// the whole launch and walks a run of 64-column tiles: each tile's weights
-// (enc_pack order: four column blocks, 4 KB per group of 16 inputs) come
-// from global memory straight into one of two LDS stages (direct loads, the
-// next tile's in flight while the MFMAs run on this one), and every wave
-// reads its B fragments from there, one 16-byte read per lane per block and
-// group. Each row's partials are joined over runs of kCtcRunTiles tiles
-// (in column order, in registers) and go to ctc_merge as one record per row
-// and run, a sixth of the per-tile records; a workgroup walks one run or
-// more, as many as the row count needs for about kCtcTarget workgroups. The
-// workgroups of one run of columns take one XCD's consecutive slots, so the
-// run's weights meet in that XCD's L2. Reduction order: groups of 16 inputs
-// in order, within a group four steps of one input per lane group.
-// Measured on 1280 x 18385 x 120: 16-row waves, eight a workgroup (96
-// VGPRs, four waves a SIMD with two workgroups a CU; four waves of 32 rows:
-// 71.4 us at two waves a SIMD; of 64 rows: 86 us, their 230 VGPRs leave one
-// wave a SIMD) and about 512 workgroups (256: 88 us, 1024: 74 us, with four
-// waves of 32 rows).
+// The CTC head's GEMM when the head's input is at most 128 wide, its f32
+// products on the bf16 matrix cores (split.hpp). A workgroup of four waves
+// keeps 128 rows (two blocks of 16 a wave), split into their three parts, in
+// its operand registers for the whole launch and walks a run of 64-column
+// tiles in halves of 32 columns: each half's weights (SplitPackArgs'
+// order, three parts) come from global memory straight into one of two LDS
+// stages (direct loads, the next half's in flight while the MFMAs run on
+// this one), and every wave reads its B fragments from there, one 16-byte
+// read per lane, block, group of 32 inputs and part. Each row's partials are
+// joined over runs of kCtcRunTiles tiles (in column order) and go to
+// ctc_merge as one record per row and run, a sixth of the per-tile records;
+// a launch of few rows has a workgroup per tile or two write the single
+// tiles' records, and the merge joins each run's in the same order.
+// The workgroups of one run of columns take one XCD's consecutive slots, so
+// the run's weights meet in that XCD's L2.
+//
+// What bounds it: the matrix cores (the six products of 1280 x 18385 x 120
+// take 17 us at the 2.0 PFLOP/s that bf16 steps reach here) and the epilogue's
+// vector work beside them, two waves a SIMD. Measured on 1280 x 18385 x 120:
+// 45 us; on f32 MFMA 68 us. On 80 rows (one row tile): 11.4 us as 288
+// workgroups of a tile, 38 us on f32 as 48 of a run. Statistics kept per lane
+// over a run and joined across lanes at its end (less epilogue work, 40 us
+// with runs of three tiles) left the few-row launch at 18 us; three stages
+// instead of two took 44 us.
 constexpr int kCtcRows = 128;             // rows a workgroup
-constexpr int kCtcWaves = 8;              // waves a workgroup, 128 / (16 * kCtcWaves) row blocks each
+constexpr int kCtcWaves = 4;              // waves a workgroup, 128 / (16 * kCtcWaves) row blocks each
 constexpr int kCtcTarget = 512;           // workgroups a launch aims at
 constexpr int kCtcRunTiles = 6;           // 64-column tiles a partial record joins
-
-template <int KQ>
-__global__ __launch_bounds__(64 * kCtcWaves) void ctc_panel(CtcDirectArgs a, int row_tiles, int per_run, int runs,
-                                                            int per_group) {
-  constexpr int W = kCtcWaves, MT = kCtcRows / (16 * W), NT = 4, STAGE = NT * KQ * 64 * 4;  // floats
-  constexpr int TPI = NT * KQ * 64 / (64 * W);  // direct loads a thread issues a tile
+constexpr int kCtcFewRuns = 256;          // below so many workgroups of a run each, single tiles
+template <int KG>
+__global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(2))) void ctc_panel(
+    CtcDirectArgs a, int row_tiles, int per_run, int runs, int per_group) {
+  constexpr int W = kCtcWaves, MT = kCtcRows / (16 * W);
+  constexpr int STAGE = 2 * KG * 3 * 64;          // 16-byte groups of a half tile's weights
+  constexpr int TPI = (STAGE + 64 * W - 1) / (64 * W);  // direct loads a thread issues a half
+  static_assert(STAGE % 64 == 0, "whole waves load");
   extern __shared__ __attribute__((aligned(16))) float bs[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lg = lane >> 4;
   const int M = a.rows_per_lane * a.lanes;
-  const int ntn = (a.vocab + 63) / 64, nb = (a.vocab + 15) / 16;
+  const int vocab = a.vocab, ntn = (vocab + 63) / 64, nb = (vocab + 15) / 16;
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int tm = tile % row_tiles, group = tile / row_tiles;
   const int t0 = group * per_group * per_run, t1 = min(ntn, t0 + per_group * per_run);
   const int m0 = tm * kCtcRows + wave * 16 * MT;
   if (t0 >= t1) return;
 
-  // A tile's weights into stage `st`: 8 * KQ 16-byte groups a thread,
-  // blocks past the vocabulary read the last block (their columns are
-  // masked in the epilogue).
-  auto issue = [&](int t, int st) {
-    const f32x4 *src = reinterpret_cast<const f32x4 *>(a.wt);
+  // Half h's weights (columns 32h .. 32h + 31) into stage h & 1; blocks past
+  // the vocabulary read the last block (their columns are masked in the
+  // epilogue).
+  auto issue = [&](int h) {
+    const split_f4 *src = reinterpret_cast<const split_f4 *>(a.wt);
 #pragma unroll
     for (int i = 0; i < TPI; i++) {
-      const int e = i * 64 * W + tid;  // 16-byte group of the tile
-      const int blk = min(t * 4 + e / (KQ * 64), nb - 1);
-      const f32x4 *p = src + (long)blk * KQ * 64 + e % (KQ * 64);
-      __builtin_amdgcn_global_load_lds((const void *)p, (lds_void *)(bs + st * STAGE + (i * 64 * W + wave * 64) * 4),
-                                       16, 0, 0);
+      const int e0 = (i * W + wave) * 64;
+      if (STAGE % (64 * W) && e0 >= STAGE) break;
+      const int e = e0 + lane, blk = min(h * 2 + e / (KG * 192), nb - 1);
+      const split_f4 *p = src + (long)blk * (KG * 192) + e % (KG * 192);
+      __builtin_amdgcn_global_load_lds((const void *)p, (lds_void *)(bs + ((h & 1) * STAGE + e0) * 4), 16, 0, 0);
     }
   };
-  issue(t0, 0);
 
   // This lane's rows (past the last row: the last row, never stored), zero
-  // past the input width.
-  f32x4 av[MT][KQ];
+  // past the input width, as operand parts; the first weights go out after
+  // the rows, so that waiting for the rows does not wait for them.
+  split_f4 x[MT][KG][2];
 #pragma unroll
   for (int i = 0; i < MT; i++) {
     const int m = min(m0 + 16 * i + li, M - 1);
     const int ln = m / a.rows_per_lane;
     const float *row = a.x + ln * a.x_lane_stride + (long)(m - ln * a.rows_per_lane) * a.ci;
 #pragma unroll
-    for (int q = 0; q < KQ; q++) {
-      const int k = 16 * q + 4 * lg;
-      av[i][q] = k < a.ci ? *reinterpret_cast<const f32x4 *>(row + k) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int q = 0; q < KG; q++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int k = 32 * q + 8 * lg + 4 * h;
+        x[i][q][h] = *reinterpret_cast<const split_f4 *>(k < a.ci ? row + k : kRingZeros);
+      }
   }
+  issue(2 * t0);
+  bf16x8 av[KG][MT][3];
+#pragma unroll
+  for (int q = 0; q < KG; q++)
+#pragma unroll
+    for (int i = 0; i < MT; i++) split8(x[i][q][0], x[i][q][1], av[q][i]);
 
   // The run's per-tile records of the workgroup's rows, joined at its end.
-  float4 *recs = reinterpret_cast<float4 *>(bs + 2 * STAGE);
+  float4 *recs = reinterpret_cast<float4 *>(bs + 2 * STAGE * 4);
   for (int t = t0; t < t1; t++) {
-    const int st = (t - t0) & 1;
-    // Every wave is done with the other stage (the tile before last).
-    ring_barrier();
-    if (t + 1 < t1) {
-      issue(t + 1, st ^ 1);
-      ring_wait<TPI>();
-    } else {
+    f32x4 acc[MT][4];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      // This half's weights have landed, from every wave, and every wave is
+      // done with the half before, whose stage the next half's loads take.
       ring_wait<0>();
+      ring_barrier();
+      if (h == 0 || t + 1 < t1) issue(2 * t + h + 1);
+      f32x4 hi[MT][2], lo[MT][2];
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) hi[i][j] = lo[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const bf16x8 *bl = reinterpret_cast<const bf16x8 *>(bs) + h * STAGE + lane;
+#pragma unroll
+      for (int q = 0; q < KG; q++) {
+        bf16x8 bv[2][3];
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+          for (int p = 0; p < 3; p++) bv[j][p] = bl[((j * KG + q) * 3 + p) * 64];
+        split_mma(av[q], bv, hi, lo);
+      }
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][2 * h + j] = hi[i][j] + lo[i][j];
     }
-    ring_barrier();  // this tile's weights have landed, from every wave
-    f32x4 acc[MT][NT];
-#pragma unroll
-    for (int i = 0; i < MT; i++)
-#pragma unroll
-      for (int j = 0; j < NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const f32x4 *bl = reinterpret_cast<const f32x4 *>(bs + st * STAGE) + lane;
-#pragma unroll
-    for (int q = 0; q < KQ; q++) {
-      f32x4 bv[NT];
-#pragma unroll
-      for (int j = 0; j < NT; j++) bv[j] = bl[(j * KQ + q) * 64];
-#pragma unroll
-      for (int e = 0; e < 4; e++)
-#pragma unroll
-        for (int i = 0; i < MT; i++)
-#pragma unroll
-          for (int j = 0; j < NT; j++)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][q][e], bv[j][e], acc[i][j], 0, 0, 0);
-    }
-    const int k = t % per_run;
-    ctc_tile_rows<MT, NT>(acc, t * 64, a.bias, a.vocab, lane, [&](int i, int r, float4 rec) {
+    const int k = t % kCtcRunTiles;
+    ctc_tile_rows<MT, 4>(acc, t * 64, a.bias, vocab, lane, [&](int i, int r, float4 rec) {
       const int row = wave * 16 * MT + i * 16 + lg * 4 + r;
-      if (li == 0) recs[row * per_run + k] = rec;
-      if (li == 0 && a.tmax && m0 + i * 16 + lg * 4 + r < M) a.tmax[(long)t * M + m0 + i * 16 + lg * 4 + r] = rec.x;
+      const int m = tm * kCtcRows + row;
+      if (li != 0) return;
+      if (per_run == 1) {
+        if (m < M) reinterpret_cast<float4 *>(a.part)[(long)m * ntn + t] = rec;
+        return;
+      }
+      recs[row * kCtcRunTiles + k] = rec;
+      if (a.tmax && m < M) a.tmax[(long)t * M + m] = rec.x;
     });
     // A run's last tile: each row's records joined in column order, one
     // record out. (The next tile's stores wait behind its first barrier.)
-    if (k == per_run - 1 || t + 1 == t1) {
+    if (per_run > 1 && (k == kCtcRunTiles - 1 || t + 1 == t1)) {
       __syncthreads();
       const int m = tm * kCtcRows + tid;
       if (tid < kCtcRows && m < M) {
-        float4 run_rec = recs[tid * per_run];
-        for (int q = 1; q <= k; q++) run_rec = ctc_join_partial(run_rec, recs[tid * per_run + q]);
-        reinterpret_cast<float4 *>(a.part)[(long)m * runs + t / per_run] = run_rec;
+        float4 run_rec = recs[tid * kCtcRunTiles];
+        for (int q = 1; q <= k; q++) run_rec = ctc_join_partial(run_rec, recs[tid * kCtcRunTiles + q]);
+        reinterpret_cast<float4 *>(a.part)[(long)m * runs + t / kCtcRunTiles] = run_rec;
       }
     }
   }
 }
 
 bool ctc_direct_supported(int ci) { return ci > 0 && ci <= 128 && ci % 4 == 0; }
+int ctc_direct_kpad(int ci) { return ci <= 32 ? 32 : (ci <= 64 ? 64 : 128); }
 
 CtcRuns ctc_direct_runs(long rows, int vocab) {
   const int row_tiles = (int)((rows + kCtcRows - 1) / kCtcRows), ntn = (vocab + 63) / 64;
@@ -1090,10 +1127,12 @@ CtcRuns ctc_direct_runs(long rows, int vocab) {
   // The records' grouping of tiles is fixed, so that a row's joins, and so
   // its bits, do not depend on how many rows the launch has; how many
   // records a workgroup walks is what follows the row count: about
-  // kCtcTarget workgroups (two a CU, each holding two 32 KB stages).
-  r.per_run = std::min(kCtcRunTiles, ntn);
-  r.runs = (ntn + r.per_run - 1) / r.per_run;
-  r.columns = 64 * r.per_run;
+  // kCtcTarget workgroups (two a CU). With fewer runs than CUs, each takes a
+  // tile or two and writes single tiles' records.
+  r.run_tiles = std::min(kCtcRunTiles, ntn);
+  const int all = (ntn + r.run_tiles - 1) / r.run_tiles;
+  r.per_run = long(row_tiles) * all < kCtcFewRuns ? 1 : r.run_tiles;
+  r.runs = r.per_run == 1 ? ntn : all;
   r.per_group = std::max(1, int((long(row_tiles) * r.runs + kCtcTarget - 1) / kCtcTarget));
   return r;
 }
@@ -1104,23 +1143,22 @@ hipError_t launch_ctc_direct(const CtcDirectArgs &a, hipStream_t s) {
   if (M <= 0 || M >= (1L << 31)) return hipErrorInvalidValue;
   const int row_tiles = (int)((M + kCtcRows - 1) / kCtcRows);
   const CtcRuns r = ctc_direct_runs(M, a.vocab);
-  const int per_run = r.per_run, runs = r.runs;
-  const unsigned blocks = (unsigned)(row_tiles * ((runs + r.per_group - 1) / r.per_group));
-  const int kq = enc_kpad(a.ci) / 16;
+  const unsigned blocks = (unsigned)(row_tiles * ((r.runs + r.per_group - 1) / r.per_group));
+  const int kg = ctc_direct_kpad(a.ci) / 32;
   // Two weight stages, then the run's per-tile records.
-  const size_t shm = (size_t)2 * 4 * kq * 64 * 16 + size_t(kCtcRows) * per_run * 16;
+  const size_t shm = size_t(2) * 2 * kg * 3 * 64 * 16 + (r.per_run > 1 ? size_t(kCtcRows) * kCtcRunTiles * 16 : 0);
   auto go = [&](auto kernel) {
     if (shm > 64 * 1024) {
       hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), int(shm));
       if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kCtcWaves), shm, s, a, row_tiles, per_run, runs, r.per_group);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kCtcWaves), shm, s, a, row_tiles, r.per_run, r.runs, r.per_group);
     return hipGetLastError();
   };
-  switch (kq) {
+  switch (kg) {
+    case 1: return go(ctc_panel<1>);
     case 2: return go(ctc_panel<2>);
-    case 4: return go(ctc_panel<4>);
-    default: return go(ctc_panel<8>);
+    default: return go(ctc_panel<4>);
   }
 }
 
@@ -1153,8 +1191,6 @@ hipError_t launch_ctc_direct(const CtcDirectArgs &a, hipStream_t s) {
 // Reduction order: chunks of BK channels in order; within a chunk the MFMA
 // chain takes groups of four channels lane group by lane group. Bias,
 // activation, residual and second activation as in conv_mfma's epilogue.
-__device__ __attribute__((aligned(16))) float kRingZeros[4];
-
 static const size_t kMaxLdsBytes = 160 * 1024;
 
 // The chunk width of a windowed convolution on the ring: the packer lays each
@@ -1731,13 +1767,45 @@ hipError_t launch_conv_patch_group(const ConvArgs *as, int n, int wr, int bk, in
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_ctc_merge(const float *part, int rows, int ntiles, float *y, long y_lane_stride,
+// A split operand's packing: a thread one 16-byte group of each part (eight
+// inputs of one column), groups in the output's order.
+__global__ __launch_bounds__(256) void split_pack_kernel(SplitPackArgs a, int kq, long groups) {
+  const long g = (long)blockIdx.x * 256 + threadIdx.x;
+  if (g >= groups) return;
+  const int l = (int)(g & 63);
+  const long b = g >> 6;
+  const int q = (int)(b % kq), j = (int)(b / kq);
+  const int k0 = 32 * q + 8 * (l >> 4), n = 16 * j + (l & 15);
+  const float *col = a.w + (long)(n / a.panel) * a.panel_stride + n % a.panel;
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const bool in = k0 + e < a.k && n < a.n;
+    x[e] = in ? col[(long)(k0 + e) * a.k_stride] : 0.0f;
+  }
+  split_u4 p[3];
+  split8(split_f4{x[0], x[1], x[2], x[3]}, split_f4{x[4], x[5], x[6], x[7]}, p[0], p[1], p[2]);
+  split_u4 *o = reinterpret_cast<split_u4 *>(a.out) + b * 192 + l;
+#pragma unroll
+  for (int s = 0; s < 3; s++) o[s * 64] = p[s];
+}
+
+hipError_t launch_split_pack(const SplitPackArgs &a, hipStream_t s) {
+  if (a.k <= 0 || a.n <= 0 || a.kp % 32 || a.kp < a.k || a.panel <= 0 || (uintptr_t(a.out) & 15)) return hipErrorInvalidValue;
+  const int kq = a.kp / 32;
+  const long groups = (long)kq * ((a.n + 15) / 16) * 64;
+  hipLaunchKernelGGL(split_pack_kernel, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s, a, kq, groups);
+  return hipGetLastError();
+}
+
+hipError_t launch_ctc_merge(const float *part, int rows, int ntiles, int run, float *y, long y_lane_stride,
                             int rows_per_lane, const CtcExact &ex, hipStream_t s) {
   if (rows <= 0) return hipSuccess;
+  if (run < 1) return hipErrorInvalidValue;
   // The recompute reads packed rows as float4.
   if (ex.wt && (ex.wt_k % 4 || (uintptr_t(ex.wt) & 15))) return hipErrorInvalidValue;
   hipLaunchKernelGGL(ctc_merge, dim3((rows + 3) / 4), dim3(256), 0, s,
-                     reinterpret_cast<const float4 *>(part), rows, ntiles, y, y_lane_stride,
+                     reinterpret_cast<const float4 *>(part), rows, ntiles, run, y, y_lane_stride,
                      rows_per_lane, ex);
   return hipGetLastError();
 }

@@ -200,23 +200,26 @@ struct CtcExact {
   long wt_k;
   const float *bias;   // per column
   int vocab;
-  int tile_n;          // columns a partial record covers (a GEMM tile, or a run of tiles)
-  const float *tmax;   // or per 64-column tile and row its maximum, tile t's row m at t * rows + m
-  int tmax_n;          // tiles
+  // Where a record covers more than one 64-column tile: per tile and row its
+  // maximum, tile t's row m at t * rows + m, and the tiles.
+  const float *tmax;
+  int tmax_n;
   // Bounds of a column's terms for the near-tie test: the largest |bias| and
   // the largest sum of a column's |weights|.
   float bias_max, wsum_max;
 };
-hipError_t launch_ctc_merge(const float *part, int rows, int ntiles, float *y, long y_lane_stride,
+// `part`: ntiles records a row; `run` consecutive ones are joined first, in
+// order (1: none).
+hipError_t launch_ctc_merge(const float *part, int rows, int ntiles, int run, float *y, long y_lane_stride,
                             int rows_per_lane, const CtcExact &ex, hipStream_t s);
 
-// The CTC head's GEMM over an input at most 128 wide (a multiple of 4), its
-// operands read straight into MFMA registers: the rows of x (ci floats,
-// rows_per_lane of them per lane) against the weights in enc_pack order
-// (kp = enc_kpad(ci), columns padded to 16), bias per column; per row and
-// run of `columns` columns (ctc_direct_runs) a float4 partial (max, sum of
-// exp, first column of the max, second value), row m's run k at
-// part[m * runs + k], for launch_ctc_merge.
+// The CTC head's GEMM over an input at most 128 wide (a multiple of 4): the
+// rows of x (ci floats, rows_per_lane of them per lane) against the weights
+// in SplitPackArgs' order (kp = ctc_direct_kpad(ci), columns padded to
+// 16), bias per column; per row and run of columns (ctc_direct_runs) a float4
+// partial (max, sum of exp, first column of the
+// max, second value), row m's record k at part[m * runs + k], for
+// launch_ctc_merge.
 struct CtcDirectArgs {
   const float *x;
   long x_lane_stride;
@@ -224,17 +227,34 @@ struct CtcDirectArgs {
   const float *wt, *bias;
   int vocab;
   float *part;
-  float *tmax;  // optional: per 64-column tile and row its maximum, tile t's row m at t * rows + m
+  float *tmax;  // where a record covers more than one: per 64-column tile and row its maximum, tile t's row m at t * rows + m
 };
 bool ctc_direct_supported(int ci);
+int ctc_direct_kpad(int ci);
 struct CtcRuns {
-  int per_run;  // 64-column tiles a workgroup walks
-  int runs;     // runs over the columns: partial records per row
-  int columns;  // columns a record covers (the last run's may be fewer)
-  int per_group; // runs a workgroup walks
+  int run_tiles; // 64-column tiles that are joined together, in the panel or in the merge
+  int per_run;   // tiles a partial record covers: run_tiles, or 1 (few rows)
+  int runs;      // partial records per row
+  int per_group; // records a workgroup makes per row
 };
 CtcRuns ctc_direct_runs(long rows, int vocab);
 hipError_t launch_ctc_direct(const CtcDirectArgs &a, hipStream_t s);
+
+// Packs a layer's weights (k inputs x n outputs) for kernels that multiply on
+// the bf16 matrix cores (split.hpp), in the order of a 16 x 16 x 32 step's
+// second operand: for column block j of 16 and input group q of 32, each of
+// the three parts in turn as 64 x 16 bytes, lane l's holding inputs
+// 32q + 8(l / 16) + e, e = 0..7, of column 16j + l % 16; zero past k and n.
+// Input i of column c lies at w[(c / panel) * panel_stride + c % panel + i * k_stride].
+struct SplitPackArgs {
+  const float *w;
+  int k, n, kp;  // kp: k padded to a multiple of 32
+  int panel;
+  long panel_stride, k_stride;
+  float *out;    // split_pack_floats(kp, n) floats, 16-byte aligned
+};
+inline size_t split_pack_floats(int kp, int n) { return size_t(kp / 32) * size_t((n + 15) / 16) * 768; }
+hipError_t launch_split_pack(const SplitPackArgs &a, hipStream_t s);
 
 // ---------------------------------------------------------------- depthwise
 

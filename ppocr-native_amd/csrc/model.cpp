@@ -112,6 +112,7 @@ struct Step {
   size_t wt_off = 0, wt_k = 0;
   size_t se_w1 = 0, se_w2 = 0;  // S_MEAN with an SE: the 1x1 weights, 16-byte aligned in the packed arena
   float ctc_bias_max = 0, ctc_wsum_max = 0;  // S_CTC: the largest |bias| and sum of a column's |weights|
+  size_t split_w = 0;  // where the bf16 parts of its weights lie in dsplit
   size_t enc_w1 = 0, enc_w2 = 0, enc_w3 = 0;  // encoder steps: their 1x1 weights in enc_pack order
 };
 
@@ -192,6 +193,7 @@ struct Model {
   std::vector<float> weights;     // host copy of the plan's weights
   float *dweights = nullptr;      // the plan's weights on the device
   float *dpacked = nullptr;       // GEMM-packed weights
+  float *dsplit = nullptr;        // the bf16 parts of the layers that run on them
   std::vector<Step> steps;
   std::vector<std::unique_ptr<Batch>> batches;
   std::vector<std::pair<size_t, size_t>> lane_at;  // lane -> (batch, index in batch)
@@ -251,6 +253,7 @@ Model::~Model() {
   }
   if (dweights) hipFree(dweights);
   if (dpacked) hipFree(dpacked);
+  if (dsplit) hipFree(dsplit);
   if (stream) hipStreamDestroy(stream);
 }
 
@@ -793,6 +796,16 @@ static RingTile ring_tile(const std::vector<ConvArgs> &as, long M) {
 // latencies in sequence, which is what small layers wait on.
 bool Model::pack(std::string &err) {
   std::vector<float> packed;
+  std::vector<SplitPackArgs> split_jobs;
+  std::vector<size_t> split_off;  // where each one's parts lie in `dsplit`
+  size_t split_floats = 0;
+  auto split_job = [&](const SplitPackArgs &a) {
+    const size_t at = split_floats;
+    split_floats += round_up(split_pack_floats(a.kp, a.n), 64);
+    split_jobs.push_back(a);
+    split_off.push_back(at);
+    return at;
+  };
   const auto &ops = plan.ops;
   for (Step &s : steps) {
     if (s.kind == S_MEAN && s.fc1 >= 0) {
@@ -950,22 +963,11 @@ bool Model::pack(std::string &err) {
       s.ctc_bias_max = std::nextafter(float(bm), INFINITY), s.ctc_wsum_max = std::nextafter(float(wm), INFINITY);
     }
     if (s.kind == S_CTC && ctc_direct_supported(int(op.ic))) {
-      // The same weights in MFMA operand order for ctc_direct (the rows above
-      // serve ctc_merge's exact recomputation of near ties): for column block
-      // j and input group q of 16, lane l's four inputs 16q + 4(l / 16) + e of
-      // column 16j + l % 16, from the plan's panels of 16 columns.
-      const int ci = int(op.ic), kp = enc_kpad(ci), kq = kp / 16, nb = (N + 15) / 16;
-      s.enc_w1 = round_up(packed.size(), 64);
-      packed.resize(s.enc_w1 + enc_pack_floats(kp, N), 0.0f);
-      float *o = packed.data() + s.enc_w1;
-      for (int j = 0; j < nb; j++)
-        for (int q = 0; q < kq; q++)
-          for (int l = 0; l < 64; l++)
-            for (int e = 0; e < 4; e++) {
-              const int kk = 16 * q + 4 * (l >> 4) + e, nn = 16 * j + (l & 15);
-              if (kk < ci && nn < N)
-                o[(((size_t)j * kq + q) * 64 + l) * 4 + e] = w[(size_t(nn) / 16) * ci * 16 + size_t(kk) * 16 + nn % 16];
-            }
+      // The same weights in the panel kernel's operand order (the rows above
+      // serve ctc_merge's exact recomputation of near ties), from the plan's
+      // panels of 16 columns.
+      const int ci = int(op.ic), kp = ctc_direct_kpad(ci);
+      s.split_w = split_job({dweights + op.w0, ci, N, kp, 16, 16L * ci, 16, nullptr});
     }
   }
   // Depthwise layers and the 1x1 convolution that alone reads each: one
@@ -1000,6 +1002,12 @@ bool Model::pack(std::string &err) {
   HIPTRY(hipMalloc(&dpacked, packed.size() * sizeof(float)), "allocating packed weights");
   HIPTRY(hipMemcpy(dpacked, packed.data(), packed.size() * sizeof(float), hipMemcpyHostToDevice),
          "uploading packed weights");
+  // The bf16 parts of the layers that run on them, made on the GPU.
+  if (split_floats) HIPTRY(hipMalloc(&dsplit, split_floats * sizeof(float)), "allocating the weights' parts");
+  for (size_t i = 0; i < split_jobs.size(); i++) {
+    split_jobs[i].out = dsplit + split_off[i];
+    HIPTRY(launch_split_pack(split_jobs[i], stream), "packing the weights");
+  }
   // A 1x1 convolution whose input only the implicit-GEMM convolution just
   // before it writes and nothing else reads: folded into that convolution's
   // epilogue, whose tile holds every output column of its pixels (16-row
@@ -1157,7 +1165,7 @@ bool Model::arrange(Batch &b, std::string &err) {
       need = L * op.iw * ntn * 4;
       if (ctc_direct_supported(int(op.ic))) {  // run records, then the per-tile maxima
         const CtcRuns r = ctc_direct_runs(long(L * op.iw), int(op.n2));
-        need = std::max(need, L * op.iw * (size_t(r.runs) * 4 + (op.n2 + 63) / 64));
+        need = std::max(need, L * op.iw * (size_t(r.runs) * 4 + (r.per_run > 1 ? (op.n2 + 63) / 64 : 0)));
       }
     }
     if (s.kind == S_ATTN) need = attention_scratch_floats(int(op.iw), int(op.oc), int(op.n2), int(L));
@@ -1351,25 +1359,29 @@ void Model::build_launches(Batch &b) {
         a.part = part;
         a.y = Y, a.y_lane_stride = ys;
         GemmTile t = s.tile;
-        int ntn = (a.n + t.bn - 1) / t.bn, tile_n = t.bn;  // partial records per row, columns each
+        int ntn = (a.n + t.bn - 1) / t.bn;  // partial records per row
         int rows = L * int(op.iw), T = int(op.iw);
         float *tmax = nullptr;  // per-tile maxima after a run's records, for the near-tie recheck
-        int tiles = 0;
+        int tiles = 0, run = 1;
         if (ctc_direct_supported(int(op.ic))) {
           const CtcRuns r = ctc_direct_runs(rows, a.vocab);
-          tiles = (a.vocab + 63) / 64;
-          tmax = part + size_t(rows) * r.runs * 4;
-          const CtcDirectArgs d{a.src[0].p, a.src[0].lane_stride, T, L, int(op.ic), dpacked + s.enc_w1, a.bias,
+          if (r.per_run > 1) {
+            tiles = (a.vocab + 63) / 64;
+            tmax = part + size_t(rows) * r.runs * 4;
+          } else {
+            run = r.run_tiles;
+          }
+          const CtcDirectArgs d{a.src[0].p, a.src[0].lane_stride, T, L, int(op.ic), dsplit + s.split_w, a.bias,
                                 a.vocab, part, tmax};
           b.launches.push_back({"ctc_gemm", s.op, [d](hipStream_t st) { return launch_ctc_direct(d, st); }});
-          ntn = r.runs, tile_n = r.columns;
+          ntn = r.runs;
         } else {
           b.launches.push_back({"ctc_gemm", s.op, [a, t](hipStream_t st) { return launch_conv(a, t, st); }});
         }
-        const CtcExact ex{a.src[0].p, a.src[0].lane_stride, int(op.ic), a.wt, a.wt_k, a.bias, a.vocab, tile_n,
+        const CtcExact ex{a.src[0].p, a.src[0].lane_stride, int(op.ic), a.wt, a.wt_k, a.bias, a.vocab,
                           tmax, tiles, s.ctc_bias_max, s.ctc_wsum_max};
-        b.launches.push_back({"ctc_merge", s.op, [part, rows, ntn, Y, ys, T, ex](hipStream_t st) {
-                                return launch_ctc_merge(part, rows, ntn, Y, ys, T, ex, st);
+        b.launches.push_back({"ctc_merge", s.op, [part, rows, ntn, run, Y, ys, T, ex](hipStream_t st) {
+                                return launch_ctc_merge(part, rows, ntn, run, Y, ys, T, ex, st);
                               }});
         break;
       }

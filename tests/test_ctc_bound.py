@@ -73,3 +73,45 @@ def test_merge_bound_covers_column_bounds():
         x = rng.normal(0, 2.0, ci).astype(np.float32)
         T = np.abs(bias.astype(np.float64)) + np.abs(w.astype(np.float64) * x[:, None]).sum(axis=0)
         assert T.max() <= bias_max + wsum_max * float(np.abs(x).max())
+
+
+def parts(v):
+    """The three bf16 parts of a float32, whose sum it is."""
+    out = []
+    for _ in range(3):
+        u = int(np.float32(v).view(np.uint32))
+        u = (u + 0x7FFF + ((u >> 16) & 1)) & 0xFFFF0000
+        out.append(np.uint32(u).view(np.float32))
+        v = np.float32(v) - out[-1]
+    assert v == 0
+    return [float(p) for p in out]
+
+
+@pytest.mark.parametrize("ci", [4, 32, 120])
+def test_split_order_within_bound(ci):
+    """The panel kernel's order: six products of bf16 parts, the five small
+    ones in an accumulator of their own, every addition rounded (to nearest or
+    toward zero): within (1.042 ci + 4) u T, twice that toward zero."""
+    rng = np.random.default_rng(ci)
+    for trial in range(20):
+        x = rng.normal(0, 3, ci).astype(np.float32)
+        w = rng.normal(0, 0.3, ci).astype(np.float32)
+        if trial % 2:  # heavy cancellation
+            w[-1] = np.float32(-(w[:-1].astype(np.float64) * x[:-1]).sum() / float(x[-1]))
+        bias = np.float32(rng.normal(0, 0.5))
+        exact = math.fsum([float(bias)] + [float(a) * float(b) for a, b in zip(w, x)])
+        T = abs(float(bias)) + sum(abs(float(a) * float(b)) for a, b in zip(w, x))
+        for toward_zero in (False, True):
+            def add(v, t):
+                s = np.float32(v + t)
+                if toward_zero and abs(float(s)) > abs(v + t):
+                    s = np.nextafter(s, np.float32(0))
+                return float(s)
+            hi = lo = 0.0
+            for a, b in zip(w, x):
+                p, q = parts(a), parts(b)
+                for i, j in ((2, 0), (0, 2), (1, 1), (1, 0), (0, 1)):
+                    lo = add(lo, p[i] * q[j])
+                hi = add(hi, p[0] * q[0])
+            got = float(np.float32(np.float32(hi + lo) + bias))
+            assert abs(got - exact) <= (1.042 * ci * (1 + toward_zero) + 4) * U * T
