@@ -129,8 +129,10 @@ bool direct_supported(int kh, int kw, int ic) { return kh * kw * ic <= kDirectTa
 // of the threads computes outputs q * OC / QS .. of every pixel, so that a
 // small map still fills the GPU. The block's pixels x OC outputs are one run
 // of memory (within a lane), written back from LDS as whole float4 rows.
-template <int OC, int QS>
-__global__ __launch_bounds__(256) void conv_stem_kernel(DirectArgs a) {
+template <int OC, int QS, int GN>
+__global__ __launch_bounds__(256) void conv_stem_kernel(Group<DirectArgs, GN> grp) {
+  const int prob = group_problem(grp);
+  const DirectArgs &a = grp.a[prob];
   constexpr int K = 27, PB = 256 / QS, OQ = OC / QS;
   static_assert(OQ % 4 == 0 && PB % 64 == 0, "float4 columns, whole waves per part");
   __shared__ __attribute__((aligned(16))) float ws[K * OC];
@@ -139,7 +141,7 @@ __global__ __launch_bounds__(256) void conv_stem_kernel(DirectArgs a) {
   const int pl = threadIdx.x % PB, q = threadIdx.x / PB;
   // Blocks numbered XCD by XCD (xcd_tile): neighbouring output rows, which
   // read the same input rows, meet in one L2.
-  const int g0 = xcd_tile((int)blockIdx.x, (int)gridDim.x) * PB, g = g0 + pl;
+  const int g0 = xcd_tile((int)blockIdx.x - grp.first[prob], grp.first[prob + 1] - grp.first[prob]) * PB, g = g0 + pl;
   // The pixel's patch is requested first, then every weight at once (a
   // rolled staging loop would wait out each load before the next), so that
   // both arrive in one round trip.
@@ -310,7 +312,55 @@ __global__ __launch_bounds__(256) void conv_direct_pix(DirectArgs a) {
 // separate multiply and add, does not (23.6 against 21.9 us).
 bool direct_pix_supported(int kh, int kw, int ic, int oc) { return kh == 2 && kw == 2 && ic == 12 && oc == 24; }
 
-hipError_t launch_conv_direct(const DirectArgs &a, hipStream_t s) {
+// Whether conv_stem_kernel takes the layer.
+static bool stem_layer(const DirectArgs &a) {
+  const long n = (long)a.lanes * a.oh * a.ow;
+  return n > 0 && n <= 0x7fffff00L && a.kh == 3 && a.kw == 3 && a.ic == 3 && a.first_end >= a.ow && a.fused >= a.oc &&
+         (a.oc == 16 || a.oc == 24 || a.oc == 32 || a.oc == 48) && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 &&
+         a.y_lane_stride % 4 == 0;
+}
+
+long direct_group_key(const DirectArgs &a) { return stem_layer(a) ? a.oc : -1; }
+
+hipError_t launch_conv_direct_group(const DirectArgs *as, int count, hipStream_t s) {
+  if (count < 1 || count > kGroupMax) return hipErrorInvalidValue;
+  bool stem = true;
+  long pixels = 0;
+  for (int p = 0; p < count; p++) {
+    stem = stem && stem_layer(as[p]) && as[p].oc == as[0].oc;
+    pixels += (long)as[p].lanes * as[p].oh * as[p].ow;
+  }
+  // The stem: 256 pixels a block, each thread all outputs of one pixel; on
+  // maps too small for that to fill the GPU (under two blocks a CU), 64
+  // pixels a block with a quarter of the outputs a wave, or 128 for 24
+  // outputs (halves of 12).
+  if (stem) {
+    const bool split = (pixels + 255) / 256 < 512;
+    const int pb = !split ? 256 : (as[0].oc == 24 ? 128 : 64);
+    Group<DirectArgs> g{};
+    long blocks = 0;
+    for (int p = 0; p < count; p++) {
+      g.first[p] = (int)blocks, g.a[p] = as[p];
+      blocks += ((long)as[p].lanes * as[p].oh * as[p].ow + pb - 1) / pb;
+      if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    }
+    g.n = count, g.first[count] = (int)blocks;
+    auto go = [&](auto one, auto many) {
+      if (count == 1)
+        hipLaunchKernelGGL(one, dim3((unsigned)blocks), dim3(256), 0, s, group_of<1>(g));
+      else
+        hipLaunchKernelGGL(many, dim3((unsigned)blocks), dim3(256), 0, s, g);
+      return hipGetLastError();
+    };
+#define PPOCR_STEM(OC, QS) return go(conv_stem_kernel<OC, QS, 1>, conv_stem_kernel<OC, QS, kGroupMax>);
+    if (as[0].oc == 16) { if (split) PPOCR_STEM(16, 4) else PPOCR_STEM(16, 1) }
+    if (as[0].oc == 24) { if (split) PPOCR_STEM(24, 2) else PPOCR_STEM(24, 1) }
+    if (as[0].oc == 32) { if (split) PPOCR_STEM(32, 4) else PPOCR_STEM(32, 1) }
+    if (split) PPOCR_STEM(48, 4) else PPOCR_STEM(48, 1)
+#undef PPOCR_STEM
+  }
+  if (count > 1) return hipErrorInvalidValue;
+  const DirectArgs &a = as[0];
   const long n = (long)a.lanes * a.oh * a.ow;
   if (n <= 0 || a.oc <= 0) return hipSuccess;
   const unsigned nb = (unsigned)((n + 255) / 256);
@@ -322,25 +372,7 @@ hipError_t launch_conv_direct(const DirectArgs &a, hipStream_t s) {
   }
   if (!direct_supported(a.kh, a.kw, a.ic) || n > 0x7fffff00L || (a.oc + 7) / 8 > 65535)
     return hipErrorInvalidValue;
-  const bool stem = a.kh == 3 && a.kw == 3 && a.ic == 3 && a.first_end >= a.ow && a.fused >= a.oc &&
-                    (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 && a.y_lane_stride % 4 == 0;
-  const unsigned blocks = (unsigned)((n + 255) / 256);
-  // The stem: 256 pixels a block, each thread all outputs of one pixel; on a
-  // map too small for that to fill the GPU (under two blocks a CU), 64
-  // pixels a block with a quarter of the outputs a wave, or 128 for 24
-  // outputs (halves of 12).
-  if (stem) {
-    const bool split = blocks < 512;
-    const unsigned b64 = (unsigned)((n + 63) / 64), b128 = (unsigned)((n + 127) / 128);
-    auto go = [&](auto kernel, unsigned nb) {
-      hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, s, a);
-      return hipGetLastError();
-    };
-    if (a.oc == 16) return split ? go(conv_stem_kernel<16, 4>, b64) : go(conv_stem_kernel<16, 1>, blocks);
-    if (a.oc == 24) return split ? go(conv_stem_kernel<24, 2>, b128) : go(conv_stem_kernel<24, 1>, blocks);
-    if (a.oc == 32) return split ? go(conv_stem_kernel<32, 4>, b64) : go(conv_stem_kernel<32, 1>, blocks);
-    if (a.oc == 48) return split ? go(conv_stem_kernel<48, 4>, b64) : go(conv_stem_kernel<48, 1>, blocks);
-  }
+  const unsigned blocks = nb;
   dim3 grid(blocks, (a.oc + 7) / 8), block(256);
   if (a.kh == 3 && a.kw == 3 && a.ic == 3)
     hipLaunchKernelGGL((conv_direct_kernel<3, 3, 3>), grid, block, 0, s, a);

@@ -198,15 +198,18 @@ __device__ __forceinline__ void mfma_rows(f32x4 &acc, const float *t, const f32x
 
 // ------------------------------------------------------------- enc_linear
 
-// Workgroup (x, y): rows 16x .. 16x + 15; wave w takes column block 8y + w.
-template <int KP>
-__global__ __launch_bounds__(kEncThreads) void enc_linear(EncLinArgs a) {
+// Workgroup y * tiles + x: rows 16x .. 16x + 15; wave w takes column block 8y + w.
+template <int KP, int GN>
+__global__ __launch_bounds__(kEncThreads) void enc_linear(Group<EncLinArgs, GN> grp) {
+  const int prob = group_problem(grp);
+  const EncLinArgs &a = grp.a[prob];
+  const int blk = (int)blockIdx.x - grp.first[prob], tiles = grp.x[prob];
   constexpr int S = KP + 4, KQ = KP / 16;
   __shared__ __attribute__((aligned(16))) float xs[kEncRows * S];
   __shared__ TileRows tr;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const long M = (long)a.rows * a.lanes, m0 = (long)blockIdx.x * kEncRows;
-  const int nb = (a.n + 15) / 16, j = blockIdx.y * 8 + w;
+  const long M = (long)a.rows * a.lanes, m0 = (long)(blk % tiles) * kEncRows;
+  const int nb = (a.n + 15) / 16, j = blk / tiles * 8 + w;
   f32x4 b[KQ];
   load_b<KQ>(b, a.wt, j, nb, lane);
   const LnRegs<KP> lr = ln_regs<KP>(a.ln, a.k);
@@ -237,17 +240,34 @@ __global__ __launch_bounds__(kEncThreads) void enc_linear(EncLinArgs a) {
 
 bool enc_linear_supported(int k, int n) { return k > 0 && k % 4 == 0 && k <= 128 && n > 0; }
 
-hipError_t launch_enc_linear(const EncLinArgs &a, hipStream_t s) {
-  const long M = (long)a.rows * a.lanes;
-  if (!enc_linear_supported(a.k, a.n) || a.x_lane_stride % 4 || M <= 0 || M >= (1L << 31))
-    return hipErrorInvalidValue;
-  const dim3 grid((unsigned)((M + kEncRows - 1) / kEncRows), (unsigned)(((a.n + 15) / 16 + 7) / 8));
-  switch (enc_kpad(a.k)) {
-    case 32: hipLaunchKernelGGL(enc_linear<32>, grid, dim3(kEncThreads), 0, s, a); break;
-    case 64: hipLaunchKernelGGL(enc_linear<64>, grid, dim3(kEncThreads), 0, s, a); break;
-    default: hipLaunchKernelGGL(enc_linear<128>, grid, dim3(kEncThreads), 0, s, a); break;
+hipError_t launch_enc_linear_group(const EncLinArgs *as, int n, hipStream_t s) {
+  if (n < 1 || n > kGroupMax) return hipErrorInvalidValue;
+  Group<EncLinArgs> g{};
+  long blocks = 0;
+  for (int p = 0; p < n; p++) {
+    const EncLinArgs &a = as[p];
+    const long M = (long)a.rows * a.lanes;
+    if (!enc_linear_supported(a.k, a.n) || a.x_lane_stride % 4 || M <= 0 || M >= (1L << 31) || a.k != as[0].k)
+      return hipErrorInvalidValue;
+    g.first[p] = (int)blocks, g.a[p] = a;
+    g.x[p] = (int)((M + kEncRows - 1) / kEncRows);
+    blocks += (long)g.x[p] * (((a.n + 15) / 16 + 7) / 8);
+    if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
   }
-  return hipGetLastError();
+  g.n = n, g.first[n] = (int)blocks;
+  const dim3 grid((unsigned)blocks);
+  auto go = [&](auto one, auto many) {
+    if (n == 1)
+      hipLaunchKernelGGL(one, grid, dim3(kEncThreads), 0, s, group_of<1>(g));
+    else
+      hipLaunchKernelGGL(many, grid, dim3(kEncThreads), 0, s, g);
+    return hipGetLastError();
+  };
+  switch (enc_kpad(as[0].k)) {
+    case 32: return go(enc_linear<32, 1>, enc_linear<32, kGroupMax>);
+    case 64: return go(enc_linear<64, 1>, enc_linear<64, kGroupMax>);
+    default: return go(enc_linear<128, 1>, enc_linear<128, kGroupMax>);
+  }
 }
 
 // --------------------------------------------------------- enc_attn_block
@@ -290,15 +310,18 @@ __host__ __device__ inline AttnLds attn_lds(int t, int heads, int tq, int kp, in
   return l;
 }
 
-template <int KP, int HP>
-__global__ __launch_bounds__(kEncThreads) void enc_attn_block(EncAttnArgs a, int tq) {
+template <int KP, int HP, int GN>
+__global__ __launch_bounds__(kEncThreads) void enc_attn_block(Group<EncAttnArgs, GN> grp) {
+  const int prob = group_problem(grp);
+  const EncAttnArgs &a = grp.a[prob];
+  const int tq = grp.x[prob];
   extern __shared__ __attribute__((aligned(16))) float sm[];
   constexpr int S = KP + 4, KQ = KP / 16;
   const int t = a.t, c = a.c, heads = a.heads, hd = c / heads, c4 = c / 4;
   const int runs = (t + tq - 1) / tq;
   // The runs of one line on one XCD (each reads the line's K and V: they
   // then meet in that XCD's L2).
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int tile = xcd_tile((int)blockIdx.x - grp.first[prob], grp.first[prob + 1] - grp.first[prob]);
   const int ln = tile / runs, q0 = (tile % runs) * tq, nq = min(tq, t - q0);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const AttnLds L = attn_lds(t, heads, tq, KP, HP);
@@ -603,8 +626,8 @@ __global__ __launch_bounds__(kEncThreads) void enc_attn_block(EncAttnArgs a, int
 
 // Query rows a workgroup: about one workgroup per CU (each loads its line's
 // K and V), at most kAttnTq.
-static int attn_tq(int t, int lanes) {
-  const long q = ((long)t * lanes + 255) / 256;
+static int attn_tq(long rows) {
+  const long q = (rows + 255) / 256;
   return (int)std::max(1L, std::min<long>(kAttnTq, q));
 }
 
@@ -620,27 +643,45 @@ bool enc_attn_supported(int c, int heads, int hidden) {
          hidden >= 0 && hidden <= 256;
 }
 
-hipError_t launch_enc_attn(const EncAttnArgs &a, hipStream_t s) {
-  const int hidden = a.w1 ? a.hidden : 0;
-  if (!enc_attn_supported(a.c, a.heads, hidden) || !enc_attn_fits(a.t, a.c, a.heads, hidden) ||
-      a.qkv_lane_stride % 4 || (hidden && a.y_lane_stride % 4))
-    return hipErrorInvalidValue;
-  const int kp = enc_kpad(a.c), hp = hidden ? enc_mlp_hpad(hidden) : 0, tq = attn_tq(a.t, a.lanes);
-  const size_t shm = (size_t)attn_lds(a.t, a.heads, tq, kp, hp).total * sizeof(float);
-  const unsigned blocks = (unsigned)((long)a.lanes * ((a.t + tq - 1) / tq));
-  auto go = [&](auto kernel) {
+hipError_t launch_enc_attn_group(const EncAttnArgs *as, int n, hipStream_t s) {
+  if (n < 1 || n > kGroupMax) return hipErrorInvalidValue;
+  const int hidden = as[0].w1 ? as[0].hidden : 0;
+  const int kp = enc_kpad(as[0].c), hp = hidden ? enc_mlp_hpad(hidden) : 0;
+  long rows = 0;
+  for (int p = 0; p < n; p++) rows += (long)as[p].t * as[p].lanes;
+  const int tq = attn_tq(rows);
+  Group<EncAttnArgs> g{};
+  long blocks = 0;
+  size_t shm = 0;
+  for (int p = 0; p < n; p++) {
+    const EncAttnArgs &a = as[p];
+    if (!enc_attn_supported(a.c, a.heads, hidden) || !enc_attn_fits(a.t, a.c, a.heads, hidden) ||
+        a.qkv_lane_stride % 4 || (hidden && a.y_lane_stride % 4) || a.c != as[0].c || (a.w1 ? a.hidden : 0) != hidden)
+      return hipErrorInvalidValue;
+    g.first[p] = (int)blocks, g.x[p] = tq, g.a[p] = a;
+    blocks += (long)a.lanes * ((a.t + tq - 1) / tq);
+    if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    shm = std::max(shm, (size_t)attn_lds(a.t, a.heads, tq, kp, hp).total * sizeof(float));
+  }
+  g.n = n, g.first[n] = (int)blocks;
+  auto go = [&](auto one, auto many) {
     // Allowed the whole LDS once, before any launch that needs over 64 KiB
     // (and so before a graph capture records one).
-    hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), int(kEncMaxLds));
+    const void *kernel = n == 1 ? reinterpret_cast<const void *>(one) : reinterpret_cast<const void *>(many);
+    hipError_t e = allow_lds(kernel, int(kEncMaxLds));
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kEncThreads), shm, s, a, tq);
+    const dim3 grid((unsigned)blocks);
+    if (n == 1)
+      hipLaunchKernelGGL(one, grid, dim3(kEncThreads), shm, s, group_of<1>(g));
+    else
+      hipLaunchKernelGGL(many, grid, dim3(kEncThreads), shm, s, g);
     return hipGetLastError();
   };
-#define PPOCR_ENC_HP(KP)                                      \
-  switch (hp) {                                              \
-    case 0: return go(enc_attn_block<KP, 0>);                \
-    case 128: return go(enc_attn_block<KP, 128>);            \
-    default: return go(enc_attn_block<KP, 256>);             \
+#define PPOCR_ENC_HP(KP)                                                                        \
+  switch (hp) {                                                                                \
+    case 0: return go(enc_attn_block<KP, 0, 1>, enc_attn_block<KP, 0, kGroupMax>);             \
+    case 128: return go(enc_attn_block<KP, 128, 1>, enc_attn_block<KP, 128, kGroupMax>);       \
+    default: return go(enc_attn_block<KP, 256, 1>, enc_attn_block<KP, 256, kGroupMax>);        \
   }
   switch (kp) {
     case 32: PPOCR_ENC_HP(32)
@@ -654,8 +695,10 @@ hipError_t launch_enc_attn(const EncAttnArgs &a, hipStream_t s) {
 
 // Workgroup x: rows 16x .. 16x + 15. Wave w takes fc1's column blocks w and
 // w + 8 and fc2's block w; all their weights are requested at the start.
-template <int KP, int HP>
-__global__ __launch_bounds__(kEncThreads) void enc_mlp(EncMlpArgs a) {
+template <int KP, int HP, int GN>
+__global__ __launch_bounds__(kEncThreads) void enc_mlp(Group<EncMlpArgs, GN> grp) {
+  const int prob = group_problem(grp);
+  const EncMlpArgs &a = grp.a[prob];
   constexpr int S = KP + 4, SH = HP + 4, KQ = KP / 16, HQ = HP / 16;
   __shared__ __attribute__((aligned(16))) float zs[kEncRows * S];
   __shared__ __attribute__((aligned(16))) float ns[kEncRows * S];
@@ -663,7 +706,7 @@ __global__ __launch_bounds__(kEncThreads) void enc_mlp(EncMlpArgs a) {
   __shared__ TileRows tr;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
-  const long M = (long)a.rows * a.lanes, m0 = (long)blockIdx.x * kEncRows;
+  const long M = (long)a.rows * a.lanes, m0 = (long)((int)blockIdx.x - grp.first[prob]) * kEncRows;
   const int c = a.c, hidden = a.hidden;
   const int nb1 = (hidden + 15) / 16, nb2 = (c + 15) / 16;
   f32x4 b0[KQ], b1[KQ], b2[HQ];
@@ -744,20 +787,34 @@ bool enc_mlp_supported(int c, int hidden) {
   return c > 0 && c % 4 == 0 && c <= 128 && hidden > 0 && hidden <= 256;
 }
 
-hipError_t launch_enc_mlp(const EncMlpArgs &a, hipStream_t s) {
-  const long M = (long)a.rows * a.lanes;
-  if (!enc_mlp_supported(a.c, a.hidden) || a.x_lane_stride % 4 || a.y_lane_stride % 4 || M <= 0 ||
-      M >= (1L << 31))
-    return hipErrorInvalidValue;
-  const dim3 grid((unsigned)((M + kEncRows - 1) / kEncRows));
-  const int kp = enc_kpad(a.c), hp = enc_mlp_hpad(a.hidden);
-  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kEncThreads), 0, s, a); };
-  if (kp == 32)
-    hp == 128 ? go(enc_mlp<32, 128>) : go(enc_mlp<32, 256>);
-  else if (kp == 64)
-    hp == 128 ? go(enc_mlp<64, 128>) : go(enc_mlp<64, 256>);
-  else
-    hp == 128 ? go(enc_mlp<128, 128>) : go(enc_mlp<128, 256>);
+hipError_t launch_enc_mlp_group(const EncMlpArgs *as, int n, hipStream_t s) {
+  if (n < 1 || n > kGroupMax) return hipErrorInvalidValue;
+  Group<EncMlpArgs> g{};
+  long blocks = 0;
+  for (int p = 0; p < n; p++) {
+    const EncMlpArgs &a = as[p];
+    const long M = (long)a.rows * a.lanes;
+    if (!enc_mlp_supported(a.c, a.hidden) || a.x_lane_stride % 4 || a.y_lane_stride % 4 || M <= 0 ||
+        M >= (1L << 31) || a.c != as[0].c || a.hidden != as[0].hidden)
+      return hipErrorInvalidValue;
+    g.first[p] = (int)blocks, g.a[p] = a;
+    blocks += (M + kEncRows - 1) / kEncRows;
+    if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+  }
+  g.n = n, g.first[n] = (int)blocks;
+  const dim3 grid((unsigned)blocks);
+  const int kp = enc_kpad(as[0].c), hp = enc_mlp_hpad(as[0].hidden);
+  auto go = [&](auto one, auto many) {
+    if (n == 1)
+      hipLaunchKernelGGL(one, grid, dim3(kEncThreads), 0, s, group_of<1>(g));
+    else
+      hipLaunchKernelGGL(many, grid, dim3(kEncThreads), 0, s, g);
+  };
+#define PPOCR_ENC_MLP(KP, HP) \
+  if (kp == KP && hp == HP) go(enc_mlp<KP, HP, 1>, enc_mlp<KP, HP, kGroupMax>);
+  PPOCR_ENC_MLP(32, 128) PPOCR_ENC_MLP(32, 256) PPOCR_ENC_MLP(64, 128) PPOCR_ENC_MLP(64, 256)
+  PPOCR_ENC_MLP(128, 128) PPOCR_ENC_MLP(128, 256)
+#undef PPOCR_ENC_MLP
   return hipGetLastError();
 }
 

@@ -553,7 +553,7 @@ __host__ __device__ inline int patch_col_stride(int taps, int row, int cb) {
 __device__ __attribute__((aligned(16))) float kPatchZeros[4];
 
 template <int WR, int BN, int CB, bool R8>
-__device__ __forceinline__ void conv_patch_body(const Group<ConvArgs> &grp) {
+__device__ __forceinline__ void conv_patch_body(const Group<ConvArgs, kGroupStep> &grp) {
   // Each XCD takes a contiguous run of tiles (xcd_tile): neighbouring tiles
   // share halo rows and columns, which then meet in one L2.
   const int bid = xcd_tile((int)blockIdx.x, (int)gridDim.x);
@@ -827,7 +827,7 @@ __device__ __forceinline__ void conv_patch_body(const Group<ConvArgs> &grp) {
 }
 
 template <int WR, int BN, int CB, bool R8>
-__global__ __launch_bounds__(256) void conv_patch(Group<ConvArgs> grp) {
+__global__ __launch_bounds__(256) void conv_patch(Group<ConvArgs, kGroupStep> grp) {
   conv_patch_body<WR, BN, CB, R8>(grp);
 }
 
@@ -835,7 +835,7 @@ __global__ __launch_bounds__(256) void conv_patch(Group<ConvArgs> grp) {
 // remainder: held to three waves per SIMD (the occupancy its LDS leaves room
 // for; 64 columns would spill).
 template <int BN, int CB, bool R8>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void conv_patch_w1(Group<ConvArgs> grp) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void conv_patch_w1(Group<ConvArgs, kGroupStep> grp) {
   conv_patch_body<1, BN, CB, R8>(grp);
 }
 
@@ -860,9 +860,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
 constexpr float kCtcUnit = 1.0f / 16777216.0f;  // 2^-24
 
 
-__global__ __launch_bounds__(256) void ctc_merge(const float4 *part, int rows, int ntiles, int run, float *y,
-                                                 long y_lane_stride, int rows_per_lane, CtcExact ex) {
-  int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+template <int GN>
+__global__ __launch_bounds__(256) void ctc_merge(Group<CtcArgs, GN> grp, int ntiles, int run, int has_tmax) {
+  const int prob = group_problem(grp);
+  const CtcArgs &ex = grp.a[prob];
+  const int rows_per_lane = ex.rows_per_lane, rows = rows_per_lane * ex.lanes;
+  const float4 *part = reinterpret_cast<const float4 *>(ex.part);
+  const float *tmax = has_tmax ? ex.part + (long)rows * ntiles * 4 : nullptr;
+  int row = ((int)blockIdx.x - grp.first[prob]) * 4 + (threadIdx.x >> 6);
   int lane = threadIdx.x & 63;
   if (row >= rows) return;
   CtcState st{-__builtin_inff(), 0.0f, __builtin_inff()};
@@ -945,10 +950,10 @@ __global__ __launch_bounds__(256) void ctc_merge(const float4 *part, int rows, i
     };
     // The 64-column tiles whose own maximum is close, found 64 tiles at a
     // time (a lane each), in column order.
-    const int units = ex.tmax ? ex.tmax_n : ntiles;
+    const int units = tmax ? (ex.vocab + 63) / 64 : ntiles;
     for (int u0 = 0; u0 < units; u0 += 64) {
       const int u = min(u0 + lane, units - 1);
-      const float um = ex.tmax ? ex.tmax[(long)u * rows + row] : part[(long)row * ntiles + u].x;
+      const float um = tmax ? tmax[(long)u * rows + row] : part[(long)row * ntiles + u].x;
       unsigned long long near = __ballot(u0 + lane < units && !(um < st.m - tie));
       while (near) {
         const int t = u0 + __builtin_ctzll(near);
@@ -966,7 +971,7 @@ __global__ __launch_bounds__(256) void ctc_merge(const float4 *part, int rows, i
     best = bb;
   }
   if (lane == 0) {
-    float *yp = y + (long)ln * y_lane_stride + 2L * tr;
+    float *yp = ex.y + (long)ln * ex.y_lane_stride + 2L * tr;
     yp[0] = best;
     yp[1] = 1.0f / st.s;
   }
@@ -1003,9 +1008,12 @@ constexpr int kCtcWaves = 4;              // waves a workgroup, 128 / (16 * kCtc
 constexpr int kCtcTarget = 512;           // workgroups a launch aims at
 constexpr int kCtcRunTiles = 6;           // 64-column tiles a partial record joins
 constexpr int kCtcFewRuns = 256;          // below so many workgroups of a run each, single tiles
-template <int KG>
+template <int KG, int GN>
 __global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(2))) void ctc_panel(
-    CtcDirectArgs a, int row_tiles, int per_run, int runs, int per_group) {
+    Group<CtcArgs, GN> grp, int per_run, int runs) {
+  const int prob = group_problem(grp);
+  const CtcArgs &a = grp.a[prob];
+  const int row_tiles = grp.x[prob], per_group = grp.y[prob];
   constexpr int W = kCtcWaves, MT = kCtcRows / (16 * W);
   constexpr int STAGE = 2 * KG * 3 * 64;          // 16-byte groups of a half tile's weights
   constexpr int TPI = (STAGE + 64 * W - 1) / (64 * W);  // direct loads a thread issues a half
@@ -1016,7 +1024,7 @@ __global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(
   const int li = lane & 15, lg = lane >> 4;
   const int M = a.rows_per_lane * a.lanes;
   const int vocab = a.vocab, ntn = (vocab + 63) / 64, nb = (vocab + 15) / 16;
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int tile = xcd_tile((int)blockIdx.x - grp.first[prob], grp.first[prob + 1] - grp.first[prob]);
   const int tm = tile % row_tiles, group = tile / row_tiles;
   const int t0 = group * per_group * per_run, t1 = min(ntn, t0 + per_group * per_run);
   const int m0 = tm * kCtcRows + wave * 16 * MT;
@@ -1026,7 +1034,7 @@ __global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(
   // the vocabulary read the last block (their columns are masked in the
   // epilogue).
   auto issue = [&](int h) {
-    const split_f4 *src = reinterpret_cast<const split_f4 *>(a.wt);
+    const split_f4 *src = reinterpret_cast<const split_f4 *>(a.split_wt);
 #pragma unroll
     for (int i = 0; i < TPI; i++) {
       const int e0 = (i * W + wave) * 64;
@@ -1102,7 +1110,8 @@ __global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(
         return;
       }
       recs[row * kCtcRunTiles + k] = rec;
-      if (a.tmax && m < M) a.tmax[(long)t * M + m] = rec.x;
+      // The tiles' own maxima, after the runs' records.
+      if (m < M) a.part[(long)M * runs * 4 + (long)t * M + m] = rec.x;
     });
     // A run's last tile: each row's records joined in column order, one
     // record out. (The next tile's stores wait behind its first barrier.)
@@ -1121,44 +1130,79 @@ __global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(
 bool ctc_direct_supported(int ci) { return ci > 0 && ci <= 128 && ci % 4 == 0; }
 int ctc_direct_kpad(int ci) { return ci <= 32 ? 32 : (ci <= 64 ? 64 : 128); }
 
-CtcRuns ctc_direct_runs(long rows, int vocab) {
-  const int row_tiles = (int)((rows + kCtcRows - 1) / kCtcRows), ntn = (vocab + 63) / 64;
+// The records' grouping of tiles is fixed, so that a row's joins, and so its
+// bits, do not depend on how many rows the launch has; how many records a
+// workgroup walks is what follows the launch's row tiles: about kCtcTarget
+// workgroups (two a CU). With fewer runs than CUs, each takes a tile or two
+// and writes single tiles' records.
+struct CtcRuns {
+  int run_tiles;  // 64-column tiles that are joined together, in the panel or in the merge
+  int per_run;    // tiles a partial record covers: run_tiles, or 1 (few rows)
+  int runs;       // partial records per row
+  int per_group;  // records a workgroup makes per row
+};
+static CtcRuns ctc_direct_runs(long row_tiles, int vocab) {
+  const int ntn = (vocab + 63) / 64;
   CtcRuns r;
-  // The records' grouping of tiles is fixed, so that a row's joins, and so
-  // its bits, do not depend on how many rows the launch has; how many
-  // records a workgroup walks is what follows the row count: about
-  // kCtcTarget workgroups (two a CU). With fewer runs than CUs, each takes a
-  // tile or two and writes single tiles' records.
   r.run_tiles = std::min(kCtcRunTiles, ntn);
   const int all = (ntn + r.run_tiles - 1) / r.run_tiles;
-  r.per_run = long(row_tiles) * all < kCtcFewRuns ? 1 : r.run_tiles;
+  r.per_run = row_tiles * all < kCtcFewRuns ? 1 : r.run_tiles;
   r.runs = r.per_run == 1 ? ntn : all;
-  r.per_group = std::max(1, int((long(row_tiles) * r.runs + kCtcTarget - 1) / kCtcTarget));
+  r.per_group = (int)std::max<long>(1, (row_tiles * r.runs + kCtcTarget - 1) / kCtcTarget);
   return r;
 }
+static long ctc_row_tiles(const CtcArgs &a) { return ((long)a.rows_per_lane * a.lanes + kCtcRows - 1) / kCtcRows; }
+static long ctc_row_tiles(const CtcArgs *as, int n) {
+  long t = 0;
+  for (int p = 0; p < n; p++) t += ctc_row_tiles(as[p]);
+  return t;
+}
 
-hipError_t launch_ctc_direct(const CtcDirectArgs &a, hipStream_t s) {
-  if (!ctc_direct_supported(a.ci) || a.x_lane_stride % 4 || a.vocab <= 0) return hipErrorInvalidValue;
-  const long M = (long)a.rows_per_lane * a.lanes;
-  if (M <= 0 || M >= (1L << 31)) return hipErrorInvalidValue;
-  const int row_tiles = (int)((M + kCtcRows - 1) / kCtcRows);
-  const CtcRuns r = ctc_direct_runs(M, a.vocab);
-  const unsigned blocks = (unsigned)(row_tiles * ((r.runs + r.per_group - 1) / r.per_group));
-  const int kg = ctc_direct_kpad(a.ci) / 32;
+size_t ctc_part_floats(long rows, int vocab) {
+  // A record per row and tile, or per run and each tile's maximum.
+  return size_t(rows) * size_t((vocab + 63) / 64) * 5;
+}
+
+hipError_t launch_ctc_direct_group(const CtcArgs *as, int n, hipStream_t s) {
+  if (n < 1 || n > kGroupMax) return hipErrorInvalidValue;
+  const CtcArgs &a0 = as[0];
+  for (int p = 0; p < n; p++) {
+    const CtcArgs &a = as[p];
+    const long M = (long)a.rows_per_lane * a.lanes;
+    if (!ctc_direct_supported(a.ci) || a.x_lane_stride % 4 || a.vocab <= 0 || M <= 0 || M >= (1L << 31) || !a.split_wt ||
+        a.ci != a0.ci || a.vocab != a0.vocab)
+      return hipErrorInvalidValue;
+  }
+  const CtcRuns r = ctc_direct_runs(ctc_row_tiles(as, n), a0.vocab);
+  Group<CtcArgs> g{};
+  long blocks = 0;
+  for (int p = 0; p < n; p++) {
+    g.first[p] = (int)blocks, g.a[p] = as[p];
+    g.x[p] = (int)ctc_row_tiles(as[p]), g.y[p] = r.per_group;
+    blocks += (long)g.x[p] * ((r.runs + r.per_group - 1) / r.per_group);
+    if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+  }
+  g.n = n, g.first[n] = (int)blocks;
+  const int kg = ctc_direct_kpad(a0.ci) / 32;
   // Two weight stages, then the run's per-tile records.
   const size_t shm = size_t(2) * 2 * kg * 3 * 64 * 16 + (r.per_run > 1 ? size_t(kCtcRows) * kCtcRunTiles * 16 : 0);
-  auto go = [&](auto kernel) {
+  auto go = [&](auto one, auto many) {
     if (shm > 64 * 1024) {
-      hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), int(shm));
+      const void *kernel = n == 1 ? reinterpret_cast<const void *>(one) : reinterpret_cast<const void *>(many);
+      hipError_t e = allow_lds(kernel, int(shm));
       if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kCtcWaves), shm, s, a, row_tiles, r.per_run, r.runs, r.per_group);
+    const dim3 grid((unsigned)blocks), block(64 * kCtcWaves);
+    if (n == 1)
+      hipLaunchKernelGGL(one, grid, block, shm, s, group_of<1>(g), r.per_run, r.runs);
+    else
+      hipLaunchKernelGGL(many, grid, block, shm, s, g, r.per_run, r.runs);
     return hipGetLastError();
   };
   switch (kg) {
-    case 1: return go(ctc_panel<1>);
-    case 2: return go(ctc_panel<2>);
-    default: return go(ctc_panel<4>);
+    case 1: return go(ctc_panel<1, 1>, ctc_panel<1, kGroupMax>);
+    case 2: return go(ctc_panel<2, 1>, ctc_panel<2, kGroupMax>);
+    default: return go(ctc_panel<4, 1>, ctc_panel<4, kGroupMax>);
   }
 }
 
@@ -1225,8 +1269,8 @@ struct RingShape {
 };
 
 
-template <int MT, int NT, int ST, int BK, bool GATE, bool WIN>
-__global__ __launch_bounds__(256) void conv_ring(Group<ConvArgs> grp) {
+template <int MT, int NT, int ST, int BK, bool GATE, bool WIN, int GN>
+__global__ __launch_bounds__(256) void conv_ring(Group<ConvArgs, GN> grp) {
   typedef RingShape<MT, NT, ST, BK> R;
   const int prob = group_problem(grp);
   const ConvArgs &a = grp.a[prob];
@@ -1534,12 +1578,17 @@ static hipError_t go_ring1(const ConvArgs *as, int n, hipStream_t s) {
   }
   grp.first[n] = (int)total;
   if (lds > kMaxLdsBytes) return hipErrorInvalidValue;
-  if (lds > 64 * 1024) {
-    hipError_t e = allow_lds(reinterpret_cast<const void *>(conv_ring<MT, NT, ST, BK, GATE, WIN>), (int)kMaxLdsBytes);
-    if (e != hipSuccess) return e;
-  }
-  hipLaunchKernelGGL((conv_ring<MT, NT, ST, BK, GATE, WIN>), dim3((unsigned)total), dim3(256), lds, s, grp);
-  return hipGetLastError();
+  auto go = [&](auto kernel, const auto &gr) {
+    if (lds > 64 * 1024) {
+      hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), (int)kMaxLdsBytes);
+      if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(256), lds, s, gr);
+    return hipGetLastError();
+  };
+  if (n == 1) return go(conv_ring<MT, NT, ST, BK, GATE, WIN, 1>, group_of<1>(grp));
+  if (n <= kGroupStep) return go(conv_ring<MT, NT, ST, BK, GATE, WIN, kGroupStep>, group_of<kGroupStep>(grp));
+  return go(conv_ring<MT, NT, ST, BK, GATE, WIN, kGroupMax>, grp);
 }
 
 template <int MT, int NT, int ST, int BK>
@@ -1701,7 +1750,7 @@ static hipError_t go_patch(const ConvArgs *as, int n, hipStream_t s) {
   if constexpr (WR == 1 && BN <= 32) kernel = reinterpret_cast<const void *>(conv_patch_w1<BN, CB, R8>);
   else kernel = reinterpret_cast<const void *>(conv_patch<WR, BN, CB, R8>);
   constexpr int TH = 4 * WR;
-  Group<ConvArgs> grp{};
+  Group<ConvArgs, kGroupStep> grp{};
   grp.n = n;
   long blocks = 0;
   size_t shm = 0;
@@ -1742,7 +1791,7 @@ hipError_t launch_conv_patch(const ConvArgs &a, int wr, int bk, int bn, hipStrea
 }
 
 hipError_t launch_conv_patch_group(const ConvArgs *as, int n, int wr, int bk, int bn, hipStream_t s) {
-  if (n < 1 || n > kGroupMax) return hipErrorInvalidValue;
+  if (n < 1 || n > kGroupStep) return hipErrorInvalidValue;
   // 17 to 24 columns on 32-column tiles: the 8-column remainder (R8); the
   // detector head's 3 x 3 (two row blocks a wave) went from 40 to 35 us, the
   // neck's group (one row block a wave, its patch within four float4s a
@@ -1798,15 +1847,36 @@ hipError_t launch_split_pack(const SplitPackArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_ctc_merge(const float *part, int rows, int ntiles, int run, float *y, long y_lane_stride,
-                            int rows_per_lane, const CtcExact &ex, hipStream_t s) {
-  if (rows <= 0) return hipSuccess;
-  if (run < 1) return hipErrorInvalidValue;
-  // The recompute reads packed rows as float4.
-  if (ex.wt && (ex.wt_k % 4 || (uintptr_t(ex.wt) & 15))) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(ctc_merge, dim3((rows + 3) / 4), dim3(256), 0, s,
-                     reinterpret_cast<const float4 *>(part), rows, ntiles, run, y, y_lane_stride,
-                     rows_per_lane, ex);
+hipError_t launch_ctc_merge_group(const CtcArgs *as, int n, hipStream_t s) {
+  if (n < 1 || n > kGroupMax) return hipErrorInvalidValue;
+  Group<CtcArgs> g{};
+  long blocks = 0;
+  for (int p = 0; p < n; p++) {
+    const CtcArgs &a = as[p];
+    // The recompute reads packed rows as float4.
+    if (a.wt && (a.wt_k % 4 || (uintptr_t(a.wt) & 15))) return hipErrorInvalidValue;
+    if (a.vocab != as[0].vocab || (a.split_wt != nullptr) != (as[0].split_wt != nullptr)) return hipErrorInvalidValue;
+    g.first[p] = (int)blocks, g.a[p] = a;
+    blocks += ((long)a.rows_per_lane * a.lanes + 3) / 4;
+    if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+  }
+  if (!blocks) return hipSuccess;
+  g.n = n, g.first[n] = (int)blocks;
+  // The panel's records (the same launch's layers together), or the implicit
+  // GEMM's one per 64-column tile.
+  int ntiles = (as[0].vocab + 63) / 64, run = 1, has_tmax = 0;
+  if (as[0].split_wt) {
+    const CtcRuns r = ctc_direct_runs(ctc_row_tiles(as, n), as[0].vocab);
+    ntiles = r.runs;
+    if (r.per_run > 1)
+      has_tmax = 1;
+    else
+      run = r.run_tiles;
+  }
+  if (n == 1)
+    hipLaunchKernelGGL(ctc_merge<1>, dim3((unsigned)blocks), dim3(256), 0, s, group_of<1>(g), ntiles, run, has_tmax);
+  else
+    hipLaunchKernelGGL(ctc_merge<kGroupMax>, dim3((unsigned)blocks), dim3(256), 0, s, g, ntiles, run, has_tmax);
   return hipGetLastError();
 }
 

@@ -84,17 +84,32 @@ struct ConvSrc {
 enum GemmMode : int { GEMM_STORE = 0, GEMM_SPREAD = 1, GEMM_CTC = 2 };
 
 // Up to kGroupMax independent problems of one kernel in one launch (so that
-// small layers which do not depend on each other fill the GPU together):
+// small layers which do not depend on each other, or one layer over lanes of
+// different sizes, fill the GPU together; sixteen take at most 6 KB of kernel
+// arguments, which cost no more than a few hundred bytes):
 // workgroup b runs block b - first[p] of problem p, first[p] <= b <
 // first[p + 1]; x and y carry two per-problem integers of the kernel.
-constexpr int kGroupMax = 4;
-template <typename A>
+constexpr int kGroupMax = 16;
+constexpr int kGroupStep = 4;  // launches of one batch of lanes that a group takes
+template <typename A, int N = kGroupMax>
 struct Group {
   int n;
-  int first[kGroupMax + 1];
-  int x[kGroupMax], y[kGroupMax];
-  A a[kGroupMax];
+  int first[N + 1];
+  int x[N], y[N];
+  A a[N];
 };
+// The same group with room for N. A kernel compiled for one problem reads its
+// arguments at fixed offsets, all at once; found by a search and read through
+// an index they cost a short launch 1 to 7 us (the recogniser's stem over one
+// line 8.3 -> 14.8 us, its first depthwise and 1x1 17.7 -> 19.8).
+template <int N, typename A>
+inline Group<A, N> group_of(const Group<A> &g) {
+  Group<A, N> r{};
+  r.n = g.n;
+  for (int p = 0; p < N && p < g.n; p++) r.first[p] = g.first[p], r.x[p] = g.x[p], r.y[p] = g.y[p], r.a[p] = g.a[p];
+  r.first[g.n < N ? g.n : N] = g.first[g.n < N ? g.n : N];
+  return r;
+}
 
 // Workgroup i of a launch runs on XCD i % 8 (the dispatcher deals them round
 // robin) and each XCD has its own L2. Renumber so that each XCD takes one
@@ -110,11 +125,11 @@ __device__ __forceinline__ int xcd_tile(int i, int groups) {
 }
 
 // The problem of a grouped launch that workgroup blockIdx.x belongs to.
-template <typename A>
-__device__ __forceinline__ int group_problem(const Group<A> &g) {
+template <typename A, int N>
+__device__ __forceinline__ int group_problem(const Group<A, N> &g) {
   int p = 0;
 #pragma unroll
-  for (int k = 1; k < kGroupMax; k++)
+  for (int k = 1; k < N; k++)
     if (k < g.n && (int)blockIdx.x >= g.first[k]) p = k;
   return p;
 }
@@ -185,60 +200,36 @@ bool patch_fits(int kh, int kw, int stride, int wr, int bk, int bn);
 bool patch_supported(const ConvArgs &a, int wr, int bk, int bn);
 size_t patch_lds_bytes(const ConvArgs &a, int wr, int bk, int bn);
 hipError_t launch_conv_patch(const ConvArgs &a, int wr, int bk, int bn, hipStream_t s);
-// n <= kGroupMax problems, each patch_supported for (wr, bk, bn), as one launch.
+// n <= kGroupStep problems, each patch_supported for (wr, bk, bn), as one launch.
 hipError_t launch_conv_patch_group(const ConvArgs *a, int n, int wr, int bk, int bn, hipStream_t s);
 
-// CTC choice from the GEMM's per-tile partials: y[2m] = best, y[2m+1] = 1/sum.
-// `ex` names the head's input rows and weights, for rows whose two largest
-// logits are too close for the GPU's summation order to decide (wt null:
-// no such check).
-struct CtcExact {
-  const float *x;      // the head's input: rows_per_lane rows of ci per lane
+// The CTC head over rows of ci inputs, rows_per_lane of them per lane:
+// launch_ctc_direct_group (an input at most 128 wide, a multiple of 4; or
+// launch_conv in GEMM_CTC mode) writes partial records to `part`,
+// launch_ctc_merge_group the choice: y[2m] = best, y[2m + 1] = 1 / sum. Rows
+// whose two largest logits are too close for the GPU's summation order to
+// decide are recomputed from `wt` in the CPU's order (null: no such check).
+struct CtcArgs {
+  const float *x;
   long x_lane_stride;
-  int ci;
-  const float *wt;     // packed weights: column n's ci inputs at wt + n * wt_k
+  int rows_per_lane, lanes, ci, vocab;
+  const float *split_wt;  // SplitPackArgs' order, kp = ctc_direct_kpad(ci); null: `part` is launch_conv's
+  const float *wt;        // packed weights: column n's ci inputs at wt + n * wt_k
   long wt_k;
-  const float *bias;   // per column
-  int vocab;
-  // Where a record covers more than one 64-column tile: per tile and row its
-  // maximum, tile t's row m at t * rows + m, and the tiles.
-  const float *tmax;
-  int tmax_n;
+  const float *bias;      // per column
+  float *part;            // ctc_part_floats(rows, vocab) floats, 16-byte aligned
   // Bounds of a column's terms for the near-tie test: the largest |bias| and
   // the largest sum of a column's |weights|.
   float bias_max, wsum_max;
-};
-// `part`: ntiles records a row; `run` consecutive ones are joined first, in
-// order (1: none).
-hipError_t launch_ctc_merge(const float *part, int rows, int ntiles, int run, float *y, long y_lane_stride,
-                            int rows_per_lane, const CtcExact &ex, hipStream_t s);
-
-// The CTC head's GEMM over an input at most 128 wide (a multiple of 4): the
-// rows of x (ci floats, rows_per_lane of them per lane) against the weights
-// in SplitPackArgs' order (kp = ctc_direct_kpad(ci), columns padded to
-// 16), bias per column; per row and run of columns (ctc_direct_runs) a float4
-// partial (max, sum of exp, first column of the
-// max, second value), row m's record k at part[m * runs + k], for
-// launch_ctc_merge.
-struct CtcDirectArgs {
-  const float *x;
-  long x_lane_stride;
-  int rows_per_lane, lanes, ci;
-  const float *wt, *bias;
-  int vocab;
-  float *part;
-  float *tmax;  // where a record covers more than one: per 64-column tile and row its maximum, tile t's row m at t * rows + m
+  float *y;
+  long y_lane_stride;
 };
 bool ctc_direct_supported(int ci);
 int ctc_direct_kpad(int ci);
-struct CtcRuns {
-  int run_tiles; // 64-column tiles that are joined together, in the panel or in the merge
-  int per_run;   // tiles a partial record covers: run_tiles, or 1 (few rows)
-  int runs;      // partial records per row
-  int per_group; // records a workgroup makes per row
-};
-CtcRuns ctc_direct_runs(long rows, int vocab);
-hipError_t launch_ctc_direct(const CtcDirectArgs &a, hipStream_t s);
+size_t ctc_part_floats(long rows, int vocab);
+// The same n layers in both calls (one vocabulary and width).
+hipError_t launch_ctc_direct_group(const CtcArgs *a, int n, hipStream_t s);
+hipError_t launch_ctc_merge_group(const CtcArgs *a, int n, hipStream_t s);
 
 // Packs a layer's weights (k inputs x n outputs) for kernels that multiply on
 // the bf16 matrix cores (split.hpp), in the order of a 16 x 16 x 32 step's
@@ -272,7 +263,12 @@ struct DwArgs {
   // mean that reads y (joined by launch_mean_group with x null).
   double *mean_part;
 };
-hipError_t launch_dwconv(const DwArgs &a, hipStream_t s);
+// Launches of several layers (`_group`, n <= kGroupMax): one layer of a plan
+// over lanes of different sizes, so every argument but sizes, strides and
+// pointers is the same. Layers whose `_group_key`s are equal and not negative
+// may share a launch; any one layer runs alone.
+hipError_t launch_dwconv_group(const DwArgs *a, int n, hipStream_t s);
+long dw_group_key(const DwArgs &a);
 bool dw_mean_supported(const DwArgs &a);
 int dw_mean_blocks(const DwArgs &a);
 
@@ -290,7 +286,7 @@ struct DwPwArgs {
   long y_lane_stride;
 };
 bool dwpw_supported(const DwArgs &d, int n, bool res);
-hipError_t launch_dwpw(const DwPwArgs &a, hipStream_t s);
+hipError_t launch_dwpw_group(const DwPwArgs *a, int n, hipStream_t s);
 
 // ---------------------------------------------------------------- elementwise
 
@@ -347,7 +343,7 @@ struct PoolArgs {
   const float *x; long x_lane_stride;
   float *y; long y_lane_stride;
 };
-hipError_t launch_pool(const PoolArgs &a, hipStream_t s);
+hipError_t launch_pool_group(const PoolArgs *a, int n, hipStream_t s);
 
 // ---------------------------------------------------------------- reductions
 
@@ -410,9 +406,17 @@ hipError_t launch_layernorm(const float *x, long x_lane_stride, const float *w, 
 // the line is long, when they take attention_scratch_floats() floats of
 // `scratch` (nonzero only then).
 size_t attention_scratch_floats(int t, int c, int heads, int lanes);
-hipError_t launch_attention(const float *x, long x_lane_stride, float scale, int t, int c,
-                            int heads, int lanes, float *y, long y_lane_stride, float *scratch,
-                            hipStream_t s);
+struct AttnRowsArgs {
+  const float *x;
+  long x_lane_stride;
+  float scale;
+  int t, c, heads, lanes;
+  float *y;
+  long y_lane_stride;
+  float *scratch;
+};
+long attention_group_key(const AttnRowsArgs &a);
+hipError_t launch_attention_group(const AttnRowsArgs *a, int n, hipStream_t s);
 
 // ------------------------------------------------------ transformer encoder
 
@@ -441,7 +445,7 @@ struct EncLinArgs {
   long y_lane_stride;
 };
 bool enc_linear_supported(int k, int n);
-hipError_t launch_enc_linear(const EncLinArgs &a, hipStream_t s);
+hipError_t launch_enc_linear_group(const EncLinArgs *a, int n, hipStream_t s);
 
 // Attention of the lanes' t steps (rows of q | k | v, 3c floats), then
 // z = act2(act(attention Wp + bias) + res) with the c x c projection Wp;
@@ -469,7 +473,7 @@ struct EncAttnArgs {
 // hidden: the MLP's width, 0 without it.
 bool enc_attn_supported(int c, int heads, int hidden);
 bool enc_attn_fits(int t, int c, int heads, int hidden);  // the line's K and V fit LDS
-hipError_t launch_enc_attn(const EncAttnArgs &a, hipStream_t s);
+hipError_t launch_enc_attn_group(const EncAttnArgs *a, int n, hipStream_t s);
 
 // z = act3(x + act2(act1(LN(x) W1 + b1) W2 + b2)) (the residual when
 // `residual`, else without x), then LN_out(z) in its place when ln_out is set.
@@ -488,7 +492,7 @@ struct EncMlpArgs {
   long y_lane_stride;
 };
 bool enc_mlp_supported(int c, int hidden);
-hipError_t launch_enc_mlp(const EncMlpArgs &a, hipStream_t s);
+hipError_t launch_enc_mlp_group(const EncMlpArgs *a, int n, hipStream_t s);
 
 hipError_t launch_row_argmax(const float *x, float *y, int rows, int cols, hipStream_t s);
 
@@ -521,7 +525,8 @@ bool direct_supported(int kh, int kw, int ic);
 // The window shapes the direct kernel also takes with four or more channels
 // (each output pixel's outputs from one thread).
 bool direct_pix_supported(int kh, int kw, int ic, int oc);
-hipError_t launch_conv_direct(const DirectArgs &a, hipStream_t s);
+hipError_t launch_conv_direct_group(const DirectArgs *a, int n, hipStream_t s);
+long direct_group_key(const DirectArgs &a);
 
 // The detector's stem block in one pass: s1 = 3x3 stride-2 convolution of
 // the RGB input (pad 1, 3 -> C1, the stem rule), then from s1 both a 2x2

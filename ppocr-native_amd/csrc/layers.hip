@@ -104,8 +104,11 @@ __global__ __launch_bounds__(256) void dwconv_kernel(DwArgs a) {
 // Threads of a block of the depthwise kernel that also sums its outputs.
 constexpr int kDwMeanThreads = 256;
 
-template <int K, int S, int DX, bool MEAN, int TB = 256>
-__global__ __launch_bounds__(MEAN ? TB : 256) void dwconv_fixed(DwArgs a) {
+template <int K, int S, int DX, bool MEAN, int TB, int GN>
+__global__ __launch_bounds__(MEAN ? TB : 256) void dwconv_fixed(Group<DwArgs, GN> grp) {
+  const int prob = group_problem(grp);
+  const DwArgs &a = grp.a[prob];
+  const int blk = (int)blockIdx.x - grp.first[prob], nblk = grp.first[prob + 1] - grp.first[prob];
   constexpr int SPAN = (DX - 1) * S + K;
   const int cv = a.c / 4;
   const int runs = (a.ow + DX - 1) / DX;
@@ -119,8 +122,8 @@ __global__ __launch_bounds__(MEAN ? TB : 256) void dwconv_fixed(DwArgs a) {
     const int R = TB / cv;
     const int r = threadIdx.x / cv;
     ch = (threadIdx.x - r * cv) * 4;
-    const int nbx = (int)gridDim.x;
-    const int lin = xcd_tile((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y));
+    const int nbx = grp.x[prob];
+    const int lin = xcd_tile(blk, nblk);
     bx = lin % nbx;
     const int rg = bx * R + r;
     ln = lin / nbx;
@@ -130,7 +133,7 @@ __global__ __launch_bounds__(MEAN ? TB : 256) void dwconv_fixed(DwArgs a) {
   } else {
     // Blocks numbered XCD by XCD (xcd_tile): neighbouring output rows, which
     // read the same input rows, meet in one L2.
-    const long g = (long)xcd_tile((int)blockIdx.x, (int)gridDim.x) * blockDim.x + threadIdx.x;
+    const long g = (long)xcd_tile(blk, nblk) * blockDim.x + threadIdx.x;
     const long total = (long)a.lanes * a.oh * runs * cv;
     if (g >= total) return;
     ch = (int)(g % cv) * 4;
@@ -215,17 +218,11 @@ __global__ __launch_bounds__(MEAN ? TB : 256) void dwconv_fixed(DwArgs a) {
       for (int r = 0; r < R; r++)
 #pragma unroll
         for (int k = 0; k < 4; k++) tot[k] += red[(r * cv + threadIdx.x) * 4 + k];
-      double *out = a.mean_part + ((long)ln * gridDim.x + bx) * a.c + threadIdx.x * 4;
+      double *out = a.mean_part + ((long)ln * grp.x[prob] + bx) * a.c + threadIdx.x * 4;
 #pragma unroll
       for (int k = 0; k < 4; k++) out[k] = tot[k];
     }
   }
-}
-
-template <typename F>
-static hipError_t launch_fixed(F kernel, dim3 grid, dim3 block, const DwArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL(kernel, grid, block, 0, s, a);
-  return hipGetLastError();
 }
 
 static constexpr int kDwRun = 4;  // outputs per thread along a row
@@ -235,9 +232,8 @@ static constexpr int kDwRun = 4;  // outputs per thread along a row
 // With the channel sums the block count is the count of partial rows the
 // mean joins, so those layers keep four (one output a thread in blocks four
 // times as wide, to keep that count, ran slower: fewer blocks than CUs).
-static int dw_run(const DwArgs &a) {
-  return (long)a.lanes * a.oh * a.ow * (a.c / 4) < (1L << 18) && !a.mean_part ? 1 : kDwRun;
-}
+static long dw_work(const DwArgs &a) { return (long)a.lanes * a.oh * a.ow * (a.c / 4); }
+static int dw_run(long work, bool sums) { return work < (1L << 18) && !sums ? 1 : kDwRun; }
 
 // The fixed-window variants: (kernel, stride) pairs with a template, the
 // height-only strides (the recogniser's (2, 1) stages) run as stride 1.
@@ -279,6 +275,14 @@ constexpr int kDwTileThreads = 256;
 struct DwTile {
   int cg, tr, tw, tiles_x, tiles_y;
 };
+struct DwTileArgs {
+  DwArgs a;
+  DwTile t;
+};
+struct DwPwTileArgs {
+  DwPwArgs a;
+  DwTile t;
+};
 
 __device__ __attribute__((aligned(16))) float kDwZeros[4];
 
@@ -286,15 +290,18 @@ __device__ __attribute__((aligned(16))) float kDwZeros[4];
 __host__ __device__ inline int dw_tile_rows(const DwArgs &a, int tr) { return (tr - 1) * a.sh + a.kh; }
 __host__ __device__ inline int dw_tile_cols(const DwArgs &a, int tw) { return (tw - 1) * a.sw + a.kw; }
 
-template <int K, int S, int CG, bool MEAN>
-__global__ __launch_bounds__(kDwTileThreads) void dwconv_tile(DwArgs a, DwTile tt) {
+template <int K, int S, int CG, bool MEAN, int GN>
+__global__ __launch_bounds__(kDwTileThreads) void dwconv_tile(Group<DwTileArgs, GN> grp) {
+  const int prob = group_problem(grp);
+  const DwArgs &a = grp.a[prob].a;
+  const DwTile &tt = grp.a[prob].t;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int groups = a.c / (4 * CG);
   const int per_lane = tt.tiles_y * tt.tiles_x;
   // Blocks numbered XCD by XCD: neighbouring tiles of one channel group,
   // which share halo rows, meet in one L2.
-  int b = xcd_tile((int)blockIdx.x, (int)gridDim.x);
+  int b = xcd_tile((int)blockIdx.x - grp.first[prob], grp.first[prob + 1] - grp.first[prob]);
   const int tx = b % tt.tiles_x;
   b /= tt.tiles_x;
   const int ty = b % tt.tiles_y;
@@ -390,12 +397,14 @@ __global__ __launch_bounds__(kDwTileThreads) void dwconv_tile(DwArgs a, DwTile t
 // sixteen lines and on the fused block's 3 x 3 with sums, dwconv_fixed's
 // four outputs a thread reusing their loaded rows win (recogniser 413 ->
 // 419 us, fused block 42.4 -> 47.9 us when tiled).
-static DwTile dw_tile_of(const DwArgs &a, bool sums) {
+// `lanes`, `total`: the lanes and output float4s of the launch, a's own or
+// those of every layer that shares it.
+static DwTile dw_tile_of(const DwArgs &a, bool sums, long lanes, long total) {
   DwTile t{};
   const bool kind = a.kh == a.kw && (a.kh == 3 || a.kh == 5 || a.kh == 7) && (a.sw == 1 || (a.sw == 2 && a.kh != 7));
   if (!kind || a.c % 16 != 0 || a.sh < 1 || a.sh > 2) return t;
-  const long work = (long)a.lanes * a.oh * a.ow * (a.c / 4) * a.sw;
-  const bool one_image_3x3 = a.kh == 3 && a.lanes == 1 && !sums;
+  const long work = total * a.sw;
+  const bool one_image_3x3 = a.kh == 3 && lanes == 1 && !sums;
   if (!(a.kh == 7 || (a.kh == 5 && work <= 180L * 1024) || one_image_3x3)) return t;
   const int cg = a.c % 32 == 0 ? 8 : 4;
   const int pix = kDwTileThreads / cg;
@@ -418,22 +427,34 @@ static size_t dw_tile_lds(const DwArgs &a, const DwTile &t) {
 }
 
 template <int CG, bool MEAN>
-static hipError_t go_dw_tile(const DwArgs &a, const DwTile &t, hipStream_t s) {
-  const long blocks = (long)a.lanes * (a.c / (4 * CG)) * t.tiles_y * t.tiles_x;
-  if (blocks < 1 || blocks > 0x7fffffffL) return hipErrorInvalidValue;
+static hipError_t go_dw_tile(const DwArgs *as, const DwTile *ts, int n, hipStream_t s) {
+  Group<DwTileArgs> g{};
+  long blocks = 0;
+  size_t lds = 0;
+  for (int p = 0; p < n; p++) {
+    g.first[p] = (int)blocks;
+    g.a[p] = DwTileArgs{as[p], ts[p]};
+    blocks += (long)as[p].lanes * (as[p].c / (4 * CG)) * ts[p].tiles_y * ts[p].tiles_x;
+    if (blocks < 1 || blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    lds = std::max(lds, dw_tile_lds(as[p], ts[p]));
+  }
+  g.n = n, g.first[n] = (int)blocks;
   const dim3 grid((unsigned)blocks), block(kDwTileThreads);
-  const size_t lds = dw_tile_lds(a, t);
-  const int kind = a.kh * 10 + a.sw;
+  const int kind = as[0].kh * 10 + as[0].sw;
 #define PPOCR_DW_TILE(KK, SS) \
-  if (kind == KK * 10 + SS) { hipLaunchKernelGGL((dwconv_tile<KK, SS, CG, MEAN>), grid, block, lds, s, a, t); return hipGetLastError(); }
+  if (kind == KK * 10 + SS) { \
+    if (n == 1) hipLaunchKernelGGL((dwconv_tile<KK, SS, CG, MEAN, 1>), grid, block, lds, s, group_of<1>(g)); \
+    else hipLaunchKernelGGL((dwconv_tile<KK, SS, CG, MEAN, kGroupMax>), grid, block, lds, s, g); \
+    return hipGetLastError(); \
+  }
   PPOCR_DW_TILE(3, 1) PPOCR_DW_TILE(3, 2) PPOCR_DW_TILE(5, 1) PPOCR_DW_TILE(5, 2) PPOCR_DW_TILE(7, 1)
 #undef PPOCR_DW_TILE
   return hipErrorInvalidValue;
 }
 
-static hipError_t launch_dw_tile(const DwArgs &a, const DwTile &t, hipStream_t s) {
-  if (a.mean_part) return t.cg == 8 ? go_dw_tile<8, true>(a, t, s) : go_dw_tile<4, true>(a, t, s);
-  return t.cg == 8 ? go_dw_tile<8, false>(a, t, s) : go_dw_tile<4, false>(a, t, s);
+static hipError_t launch_dw_tile(const DwArgs *as, const DwTile *ts, int n, hipStream_t s) {
+  if (as[0].mean_part) return ts[0].cg == 8 ? go_dw_tile<8, true>(as, ts, n, s) : go_dw_tile<4, true>(as, ts, n, s);
+  return ts[0].cg == 8 ? go_dw_tile<8, false>(as, ts, n, s) : go_dw_tile<4, false>(as, ts, n, s);
 }
 
 // ------------------------------------------- depthwise, then a 1x1, on tiles
@@ -504,9 +525,12 @@ __device__ __forceinline__ void dwpw_mfma(f32x4 (&acc)[RB][NBW], const float *A,
   }
 }
 
-template <int K, int S, int RB, int NBW>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void dwpw_tile(DwPwArgs a, DwTile tt) {
+template <int K, int S, int RB, int NBW, int GN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void dwpw_tile(Group<DwPwTileArgs, GN> grp) {
   constexpr int P = 16 * RB;
+  const int prob = group_problem(grp);
+  const DwPwArgs &a = grp.a[prob].a;
+  const DwTile &tt = grp.a[prob].t;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const DwArgs &d = a.d;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -514,7 +538,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
   const int C = d.c, C4 = C / 4, KQ = C / 16, N = a.n, N4 = N / 4, NB = (N + 15) / 16;
   const int AS = C + 4, ON = NB * 16 + 4;
   // Tiles numbered XCD by XCD: neighbours, which share halo rows, meet in one L2.
-  int b = xcd_tile((int)blockIdx.x, (int)gridDim.x);
+  int b = xcd_tile((int)blockIdx.x - grp.first[prob], grp.first[prob + 1] - grp.first[prob]);
   const int tx = b % tt.tiles_x;
   b /= tt.tiles_x;
   const int ty = b % tt.tiles_y, ln = b / tt.tiles_y;
@@ -686,53 +710,81 @@ static bool dwpw_shape_ok(const DwArgs &d, int n) {
 // 192 output channels (three column blocks a wave): the recogniser's
 // 128 -> 256 block fused on four took 20.4 us against 16.4 for its two
 // launches.
-static DwTile dwpw_tile_of(const DwArgs &d, int n, bool res, int &rb) {
-  DwTile t{};
-  rb = 0;
-  if (!dwpw_shape_ok(d, n)) return t;
+// Of several layers that share a launch, the tiles count together.
+static DwTile dwpw_tile(const DwArgs &d, int p) {
+  int tw = p == 16 ? 4 : 8, tr = p / tw;
+  if (d.ow < tw) tw = d.ow, tr = p / tw;
+  if (d.oh < tr) tr = d.oh, tw = std::min(d.ow, p / tr);
+  return DwTile{0, tr, tw, (d.ow + tw - 1) / tw, (d.oh + tr - 1) / tr};
+}
+
+// Pixels of the tiles of n layers (0: not taken).
+static int dwpw_pixels(const DwPwArgs *as, int n) {
+  int best = 0;
   for (int p : {64, 32, 16}) {
-    int tw = p == 16 ? 4 : 8, tr = p / tw;
-    if (d.ow < tw) tw = d.ow, tr = p / tw;
-    if (d.oh < tr) tr = d.oh, tw = std::min(d.ow, p / tr);
-    const long tiles = long(d.lanes) * ((d.oh + tr - 1) / tr) * ((d.ow + tw - 1) / tw);
-    if (size_t(dwpw_lds(d, n, tr, tw, p, res).total) * 4 > 64 * 1024) continue;
-    t = DwTile{0, tr, tw, (d.ow + tw - 1) / tw, (d.oh + tr - 1) / tr};
-    rb = p / 16;
+    long tiles = 0;
+    bool fits = true;
+    for (int i = 0; i < n; i++) {
+      const DwArgs &d = as[i].d;
+      if (!dwpw_shape_ok(d, as[i].n)) return 0;
+      const DwTile t = dwpw_tile(d, p);
+      tiles += long(d.lanes) * t.tiles_x * t.tiles_y;
+      fits = fits && size_t(dwpw_lds(d, as[i].n, t.tr, t.tw, p, as[i].res != nullptr).total) * 4 <= 64 * 1024;
+    }
+    if (!fits) continue;
+    best = p;
     if (tiles >= 256) break;
   }
-  return t;
+  return best;
 }
 
 bool dwpw_supported(const DwArgs &d, int n, bool res) {
-  int rb;
-  dwpw_tile_of(d, n, res, rb);
-  return rb > 0;
+  static const float some = 0.0f;
+  DwPwArgs a{};
+  a.d = d, a.n = n, a.res = res ? &some : nullptr;
+  return dwpw_pixels(&a, 1) > 0;
 }
 
 template <int K, int S, int RB>
-static hipError_t go_dwpw(const DwPwArgs &a, const DwTile &t, size_t lds, dim3 grid, hipStream_t s) {
-  const int nbw = ((a.n + 15) / 16 + 3) / 4;
+static hipError_t go_dwpw(const Group<DwPwTileArgs> &g, size_t lds, dim3 grid, hipStream_t s) {
+  const int nbw = ((g.a[0].a.n + 15) / 16 + 3) / 4;
+  auto go = [&](auto one, auto many) {
+    if (g.n == 1)
+      hipLaunchKernelGGL(one, grid, dim3(256), lds, s, group_of<1>(g));
+    else
+      hipLaunchKernelGGL(many, grid, dim3(256), lds, s, g);
+    return hipGetLastError();
+  };
   switch (nbw) {
-    case 1: hipLaunchKernelGGL((dwpw_tile<K, S, RB, 1>), grid, dim3(256), lds, s, a, t); break;
-    case 2: hipLaunchKernelGGL((dwpw_tile<K, S, RB, 2>), grid, dim3(256), lds, s, a, t); break;
-    case 3: hipLaunchKernelGGL((dwpw_tile<K, S, RB, 3>), grid, dim3(256), lds, s, a, t); break;
-    default: return hipErrorInvalidValue;
+    case 1: return go(dwpw_tile<K, S, RB, 1, 1>, dwpw_tile<K, S, RB, 1, kGroupMax>);
+    case 2: return go(dwpw_tile<K, S, RB, 2, 1>, dwpw_tile<K, S, RB, 2, kGroupMax>);
+    case 3: return go(dwpw_tile<K, S, RB, 3, 1>, dwpw_tile<K, S, RB, 3, kGroupMax>);
   }
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
-hipError_t launch_dwpw(const DwPwArgs &a, hipStream_t s) {
-  const DwArgs &d = a.d;
-  int rb;
-  const DwTile t = dwpw_tile_of(d, a.n, a.res != nullptr, rb);
-  if (!rb || !a.pw || !a.y) return hipErrorInvalidValue;
-  const long blocks = long(d.lanes) * t.tiles_y * t.tiles_x;
-  if (blocks < 1 || blocks > 0x7fffffffL) return hipErrorInvalidValue;
-  const size_t lds = size_t(dwpw_lds(d, a.n, t.tr, t.tw, 16 * rb, a.res != nullptr).total) * 4;
+hipError_t launch_dwpw_group(const DwPwArgs *as, int n, hipStream_t s) {
+  if (n < 1 || n > kGroupMax) return hipErrorInvalidValue;
+  const int p = dwpw_pixels(as, n);
+  if (!p) return hipErrorInvalidValue;
+  Group<DwPwTileArgs> g{};
+  long blocks = 0;
+  size_t lds = 0;
+  for (int i = 0; i < n; i++) {
+    const DwArgs &d = as[i].d;
+    if (!as[i].pw || !as[i].y || d.kh != as[0].d.kh || d.sw != as[0].d.sw || as[i].n != as[0].n) return hipErrorInvalidValue;
+    const DwTile t = dwpw_tile(d, p);
+    g.first[i] = (int)blocks;
+    g.a[i] = DwPwTileArgs{as[i], t};
+    blocks += long(d.lanes) * t.tiles_y * t.tiles_x;
+    if (blocks < 1 || blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    lds = std::max(lds, size_t(dwpw_lds(d, as[i].n, t.tr, t.tw, p, as[i].res != nullptr).total) * 4);
+  }
+  g.n = n, g.first[n] = (int)blocks;
   const dim3 grid((unsigned)blocks);
-  const int kind = d.kh * 100 + d.sw * 10 + rb;
+  const int kind = as[0].d.kh * 100 + as[0].d.sw * 10 + p / 16;
 #define PPOCR_DWPW(KK, SS, RR) \
-  if (kind == KK * 100 + SS * 10 + RR) return go_dwpw<KK, SS, RR>(a, t, lds, grid, s);
+  if (kind == KK * 100 + SS * 10 + RR) return go_dwpw<KK, SS, RR>(g, lds, grid, s);
   PPOCR_DWPW(3, 1, 4) PPOCR_DWPW(3, 1, 2) PPOCR_DWPW(3, 1, 1)
   PPOCR_DWPW(3, 2, 4) PPOCR_DWPW(3, 2, 2) PPOCR_DWPW(3, 2, 1)
   PPOCR_DWPW(5, 1, 4) PPOCR_DWPW(5, 1, 2) PPOCR_DWPW(5, 1, 1)
@@ -744,7 +796,7 @@ hipError_t launch_dwpw(const DwPwArgs &a, hipStream_t s) {
 bool dw_mean_supported(const DwArgs &a) { return a.c % 4 == 0 && a.c <= 1024 && dw_fixed_kind(a) != 0; }
 
 int dw_mean_blocks(const DwArgs &a) {
-  const DwTile t = dw_tile_of(a, true);
+  const DwTile t = dw_tile_of(a, true, a.lanes, dw_work(a));
   if (t.cg) return t.tiles_y * t.tiles_x;  // one partial row per spatial tile
   const int cv = a.c / 4, R = kDwMeanThreads / cv;
   const int runs = (a.ow + kDwRun - 1) / kDwRun;  // the run with the sums (dw_run)
@@ -752,42 +804,81 @@ int dw_mean_blocks(const DwArgs &a) {
 }
 
 template <bool MEAN, int DX, int TB>
-static hipError_t launch_dw_fixed(int kind, dim3 grid, const DwArgs &a, hipStream_t s) {
-  const dim3 block(MEAN ? TB : 256);
-  switch (kind) {
-    case 31: return launch_fixed(dwconv_fixed<3, 1, DX, MEAN, TB>, grid, block, a, s);
-    case 32: return launch_fixed(dwconv_fixed<3, 2, DX, MEAN, TB>, grid, block, a, s);
-    case 51: return launch_fixed(dwconv_fixed<5, 1, DX, MEAN, TB>, grid, block, a, s);
-    case 52: return launch_fixed(dwconv_fixed<5, 2, DX, MEAN, TB>, grid, block, a, s);
-    case 71: return launch_fixed(dwconv_fixed<7, 1, DX, MEAN, TB>, grid, block, a, s);
-  }
+static hipError_t launch_dw_fixed(int kind, const Group<DwArgs> &g, hipStream_t s) {
+  const dim3 grid((unsigned)g.first[g.n]), block(MEAN ? TB : 256);
+  auto go = [&](auto one, auto many) {
+    if (g.n == 1)
+      hipLaunchKernelGGL(one, grid, block, 0, s, group_of<1>(g));
+    else
+      hipLaunchKernelGGL(many, grid, block, 0, s, g);
+    return hipGetLastError();
+  };
+#define PPOCR_DW_FIXED(KIND, K, S) \
+  if (kind == KIND) return go(dwconv_fixed<K, S, DX, MEAN, TB, 1>, dwconv_fixed<K, S, DX, MEAN, TB, kGroupMax>);
+  PPOCR_DW_FIXED(31, 3, 1) PPOCR_DW_FIXED(32, 3, 2) PPOCR_DW_FIXED(51, 5, 1) PPOCR_DW_FIXED(52, 5, 2)
+  PPOCR_DW_FIXED(71, 7, 1)
+#undef PPOCR_DW_FIXED
   return hipErrorInvalidValue;
 }
 
-template <bool MEAN>
-static hipError_t launch_dw_fixed(int kind, dim3 grid, const DwArgs &a, hipStream_t s) {
-  if (MEAN) return launch_dw_fixed<true, kDwRun, kDwMeanThreads>(kind, grid, a, s);
-  return dw_run(a) == 1 ? launch_dw_fixed<false, 1, 256>(kind, grid, a, s)
-                        : launch_dw_fixed<false, kDwRun, 256>(kind, grid, a, s);
+static bool dw_vec(const DwArgs &a) {
+  auto aligned = [](const void *p) { return p == nullptr || (uintptr_t(p) & 15) == 0; };
+  return a.c % 4 == 0 && aligned(a.x) && aligned(a.y) && aligned(a.w) && aligned(a.bias) &&
+         a.x_lane_stride % 4 == 0 && a.y_lane_stride % 4 == 0;
 }
 
-hipError_t launch_dwconv(const DwArgs &a, hipStream_t s) {
-  const int DX = dw_run(a);
-  auto aligned = [](const void *p) { return p == nullptr || (uintptr_t(p) & 15) == 0; };
-  bool vec = a.c % 4 == 0 && aligned(a.x) && aligned(a.y) && aligned(a.w) && aligned(a.bias) &&
-             a.x_lane_stride % 4 == 0 && a.y_lane_stride % 4 == 0;
-  const DwTile t = dw_tile_of(a, a.mean_part != nullptr);
-  if (vec && t.cg) return launch_dw_tile(a, t, s);
-  const int kind = dw_fixed_kind(a);
-  if (a.mean_part) {
-    // With the channel sums: only the fixed variants, one grid row per lane.
-    if (!vec || !dw_mean_supported(a) || a.lanes > 65535) return hipErrorInvalidValue;
-    return launch_dw_fixed<true>(kind, dim3(dw_mean_blocks(a), a.lanes), a, s);
+long dw_group_key(const DwArgs &a) {
+  if (!dw_vec(a) || !dw_fixed_kind(a)) return -1;
+  // With the sums a layer's blocks are its partial rows: its own tiling.
+  return a.mean_part ? dw_tile_of(a, true, a.lanes, dw_work(a)).cg : 0;
+}
+
+hipError_t launch_dwconv_group(const DwArgs *as, int n, hipStream_t s) {
+  if (n < 1 || n > kGroupMax) return hipErrorInvalidValue;
+  const bool sums = as[0].mean_part != nullptr;
+  const int kind = dw_fixed_kind(as[0]);
+  long lanes = 0, work = 0;
+  bool vec = true;
+  for (int p = 0; p < n; p++) {
+    const DwArgs &a = as[p];
+    lanes += a.lanes, work += dw_work(a);
+    vec = vec && dw_vec(a);
+    if (n > 1 && (a.kh != as[0].kh || a.kw != as[0].kw || a.sh != as[0].sh || a.sw != as[0].sw || a.c != as[0].c ||
+                  (a.mean_part != nullptr) != sums || dw_group_key(a) != dw_group_key(as[0]) || dw_group_key(a) < 0))
+      return hipErrorInvalidValue;
   }
-  long runs = (a.ow + DX - 1) / DX;
-  long total = (long)a.lanes * a.oh * runs * (vec ? a.c / 4 : a.c);
-  dim3 grid(blocks_for(total, 256));
-  if (vec && kind) return launch_dw_fixed<false>(kind, grid, a, s);
+  DwTile ts[kGroupMax];
+  for (int p = 0; p < n; p++)
+    ts[p] = sums ? dw_tile_of(as[p], true, as[p].lanes, dw_work(as[p])) : dw_tile_of(as[p], false, lanes, work);
+  // A tile per layer: all or none of one launch's layers run tiled.
+  bool tiled = vec;
+  for (int p = 0; p < n; p++) tiled = tiled && ts[p].cg && ts[p].cg == ts[0].cg;
+  if (tiled) return launch_dw_tile(as, ts, n, s);
+  const int DX = dw_run(work, sums);
+  if (vec && kind) {
+    Group<DwArgs> g{};
+    long blocks = 0;
+    for (int p = 0; p < n; p++) {
+      const DwArgs &a = as[p];
+      g.first[p] = (int)blocks;
+      g.a[p] = a;
+      if (sums) {
+        if (!dw_mean_supported(a) || ts[p].cg) return hipErrorInvalidValue;
+        g.x[p] = dw_mean_blocks(a);
+        blocks += (long)g.x[p] * a.lanes;
+      } else {
+        blocks += blocks_for((long)a.lanes * a.oh * ((a.ow + DX - 1) / DX) * (a.c / 4), 256);
+      }
+      if (blocks < 1 || blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    }
+    g.n = n, g.first[n] = (int)blocks;
+    if (sums) return launch_dw_fixed<true, kDwRun, kDwMeanThreads>(kind, g, s);
+    return DX == 1 ? launch_dw_fixed<false, 1, 256>(kind, g, s) : launch_dw_fixed<false, kDwRun, 256>(kind, g, s);
+  }
+  if (n > 1 || sums) return hipErrorInvalidValue;
+  const DwArgs &a = as[0];
+  const long runs = (a.ow + DX - 1) / DX;
+  const dim3 grid(blocks_for((long)a.lanes * a.oh * runs * (vec ? a.c / 4 : a.c), 256));
   if (vec && DX == 1)
     hipLaunchKernelGGL((dwconv_kernel<4, 1>), grid, dim3(256), 0, s, a);
   else if (vec)
@@ -820,8 +911,8 @@ __device__ __forceinline__ void vstore(float *p, const float (&v)[V]) {
   }
 }
 
-template <int V>
-__global__ __launch_bounds__(256) void eltwise_kernel(Group<EltArgs> grp) {
+template <int V, int GN>
+__global__ __launch_bounds__(256) void eltwise_kernel(Group<EltArgs, GN> grp) {
   const int prob = group_problem(grp);
   const EltArgs &a = grp.a[prob];
   const long blk = (long)blockIdx.x - grp.first[prob], nblk = grp.first[prob + 1] - grp.first[prob];
@@ -991,8 +1082,13 @@ hipError_t launch_eltwise_group(const EltArgs *as, int n, hipStream_t s) {
     grp.a[p] = as[p];
   }
   grp.first[n] = (int)blocks;
-  if (vec) hipLaunchKernelGGL(eltwise_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, s, grp);
-  else hipLaunchKernelGGL(eltwise_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, s, grp);
+  auto go = [&](auto kernel, const auto &g) { hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, g); };
+  if (n == 1)
+    vec ? go(eltwise_kernel<4, 1>, group_of<1>(grp)) : go(eltwise_kernel<1, 1>, group_of<1>(grp));
+  else if (n <= kGroupStep)
+    vec ? go(eltwise_kernel<4, kGroupStep>, group_of<kGroupStep>(grp)) : go(eltwise_kernel<1, kGroupStep>, group_of<kGroupStep>(grp));
+  else
+    vec ? go(eltwise_kernel<4, kGroupMax>, grp) : go(eltwise_kernel<1, kGroupMax>, grp);
   return hipGetLastError();
 }
 
@@ -1004,13 +1100,15 @@ hipError_t launch_eltwise(const EltArgs &a, hipStream_t s) { return launch_eltwi
 // tap, each later tap kept only when greater (src/engine/conv.rs:404-440).
 // Average: whole windows, taps summed from zero in row-major order, then
 // divided (src/engine/layers.rs:443-463).
-template <int V>
-__global__ __launch_bounds__(256) void pool_kernel(PoolArgs a) {
+template <int V, int GN>
+__global__ __launch_bounds__(256) void pool_kernel(Group<PoolArgs, GN> grp) {
+  const int prob = group_problem(grp);
+  const PoolArgs &a = grp.a[prob];
   const int cv = a.c / V;
   long per = (long)a.oh * a.ow * cv;
   // Blocks numbered XCD by XCD (xcd_tile): neighbouring output rows, which
   // read the same input rows, meet in one L2.
-  long g = (long)xcd_tile((int)blockIdx.x, (int)gridDim.x) * blockDim.x + threadIdx.x;
+  long g = (long)xcd_tile((int)blockIdx.x - grp.first[prob], grp.first[prob + 1] - grp.first[prob]) * blockDim.x + threadIdx.x;
   if (g >= (long)a.lanes * per) return;
   int ln = (int)(g / per);
   long off = g - (long)ln * per;
@@ -1048,14 +1146,30 @@ __global__ __launch_bounds__(256) void pool_kernel(PoolArgs a) {
   vstore<V>(a.y + (long)ln * a.y_lane_stride + pix * a.c + ch, accv);
 }
 
-hipError_t launch_pool(const PoolArgs &a, hipStream_t s) {
-  const bool v4 = a.c % 4 == 0 && a.x_lane_stride % 4 == 0 && a.y_lane_stride % 4 == 0 &&
-                  (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
-  long n = (long)a.lanes * a.oh * a.ow * (v4 ? a.c / 4 : a.c);
-  if (v4)
-    hipLaunchKernelGGL(pool_kernel<4>, dim3(blocks_for(n, 256)), dim3(256), 0, s, a);
+hipError_t launch_pool_group(const PoolArgs *as, int n, hipStream_t s) {
+  if (n < 1 || n > kGroupMax) return hipErrorInvalidValue;
+  bool v4 = true;
+  for (int p = 0; p < n; p++) {
+    const PoolArgs &a = as[p];
+    v4 = v4 && a.c % 4 == 0 && a.x_lane_stride % 4 == 0 && a.y_lane_stride % 4 == 0 &&
+         (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
+  }
+  Group<PoolArgs> g{};
+  long blocks = 0;
+  for (int p = 0; p < n; p++) {
+    const PoolArgs &a = as[p];
+    g.first[p] = (int)blocks;
+    g.a[p] = a;
+    blocks += blocks_for((long)a.lanes * a.oh * a.ow * (v4 ? a.c / 4 : a.c), 256);
+    if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+  }
+  g.n = n, g.first[n] = (int)blocks;
+  const dim3 grid((unsigned)blocks);
+  auto go = [&](auto kernel, const auto &gr) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, gr); };
+  if (n == 1)
+    v4 ? go(pool_kernel<4, 1>, group_of<1>(g)) : go(pool_kernel<1, 1>, group_of<1>(g));
   else
-    hipLaunchKernelGGL(pool_kernel<1>, dim3(blocks_for(n, 256)), dim3(256), 0, s, a);
+    v4 ? go(pool_kernel<4, kGroupMax>, g) : go(pool_kernel<1, kGroupMax>, g);
   return hipGetLastError();
 }
 
@@ -1242,8 +1356,8 @@ __device__ __forceinline__ T get_shared(const T *p) {
 
 // SE: some job of the group has a squeeze-and-excite (the layers' register
 // queues are compiled in only then).
-template <int V, bool SE>
-__global__ __launch_bounds__(256) void mean_se(Group<MeanJob> grp) {
+template <int V, bool SE, int GN>
+__global__ __launch_bounds__(256) void mean_se(Group<MeanJob, GN> grp) {
   extern __shared__ __attribute__((aligned(16))) float dyn[];
   __shared__ double red[256 * V];
   __shared__ int flag;
@@ -1447,15 +1561,21 @@ hipError_t launch_mean_group(const MeanJob *jobs, int n, hipStream_t s) {
   g.n = n;
   g.first[n] = (int)blocks;
   const dim3 grid((unsigned)blocks);
-  if (vec && any_se)
-    hipLaunchKernelGGL((mean_se<4, true>), grid, dim3(256), shm, s, g);
-  else if (vec)
-    hipLaunchKernelGGL((mean_se<4, false>), grid, dim3(256), shm, s, g);
-  else if (any_se)
-    hipLaunchKernelGGL((mean_se<1, true>), grid, dim3(256), shm, s, g);
-  else
-    hipLaunchKernelGGL((mean_se<1, false>), grid, dim3(256), shm, s, g);
-  return hipGetLastError();
+  auto go = [&](auto kernel, const auto &gr) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), shm, s, gr);
+    return hipGetLastError();
+  };
+#define PPOCR_MEAN(V, SE)                                                            \
+  {                                                                                  \
+    if (n == 1) return go(mean_se<V, SE, 1>, group_of<1>(g));                        \
+    if (n <= kGroupStep) return go(mean_se<V, SE, kGroupStep>, group_of<kGroupStep>(g)); \
+    return go(mean_se<V, SE, kGroupMax>, g);                                         \
+  }
+  if (vec && any_se) PPOCR_MEAN(4, true)
+  if (vec) PPOCR_MEAN(4, false)
+  if (any_se) PPOCR_MEAN(1, true)
+  PPOCR_MEAN(1, false)
+#undef PPOCR_MEAN
 }
 
 // ------------------------------------------------------------ layer norm
@@ -1720,13 +1840,19 @@ __global__ __launch_bounds__(NT) void attention_kernel(const float *x, long x_la
 // reads, an output thread's four dimensions of V per key as one. Every
 // value keeps the order above (the products and sums of a score over
 // d < hd only, each output's keys in order).
-template <int HDV>
-__global__ __launch_bounds__(256) void attention_rows(const float *x, long x_lane_stride, float scale, int t,
-                                                      int c, int heads, int runs, float *y, long y_lane_stride) {
+template <int HDV, int GN>
+__global__ __launch_bounds__(256) void attention_rows(Group<AttnRowsArgs, GN> grp) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
+  const int prob = group_problem(grp);
+  const AttnRowsArgs &a = grp.a[prob];
+  const float *x = a.x;
+  float *y = a.y;
+  const long x_lane_stride = a.x_lane_stride, y_lane_stride = a.y_lane_stride;
+  const float scale = a.scale;
+  const int t = a.t, c = a.c, heads = a.heads, runs = grp.x[prob];
   const int hd = c / heads;
   const int tq = (t + runs - 1) / runs;
-  const int blk = blockIdx.x;
+  const int blk = (int)blockIdx.x - grp.first[prob];
   const int run = blk % runs, lh = blk / runs;
   const int ln = lh / heads, h = lh % heads;
   const int q0 = run * tq, nq = min(tq, t - q0);
@@ -1865,17 +1991,73 @@ size_t attention_scratch_floats(int t, int c, int heads, int lanes) {
   return (size_t)lanes * heads * t * (t + 1);
 }
 
-hipError_t launch_attention(const float *x, long x_lane_stride, float scale, int t, int c,
-                            int heads, int lanes, float *y, long y_lane_stride, float *scratch,
-                            hipStream_t s) {
-  if (heads <= 0 || c % heads) return hipErrorInvalidValue;
-  int hd = c / heads;
-  if (hd > 64) return hipErrorInvalidValue;
-  bool lds = attention_in_lds(t, hd);
-  if (!lds && !scratch) return hipErrorInvalidValue;
-  size_t shm = attention_lds_floats(t, hd, lds) * sizeof(float);
+// Runs of query rows a (lane, head): enough for two blocks per CU of `all`
+// (lane, head) pairs, and, in a launch of several layers, so many that a
+// run's LDS fits (0: none does).
+static int attention_runs(int t, int hdv, long all, bool grow) {
+  int runs = (int)std::max<long>(1, std::min<long>(t, (512 + all - 1) / all));
+  while (grow && runs < t && attention_rows_floats(t, hdv, runs) * sizeof(float) > 64 * 1024) runs++;
+  return attention_rows_floats(t, hdv, runs) * sizeof(float) <= 64 * 1024 ? runs : 0;
+}
+
+static int attention_hdv(const AttnRowsArgs &a) {
+  const int hd = a.c / a.heads;
+  return hd <= 16 ? 16 : (hd <= 32 ? 32 : 64);
+}
+
+long attention_group_key(const AttnRowsArgs &a) {
+  if (a.heads <= 0 || a.c % a.heads || a.c / a.heads > 64) return -1;
+  // (Alone in its launch a line takes the kernel that its runs fit.)
+  return attention_runs(a.t, attention_hdv(a), (long)a.lanes * a.heads, true) ? attention_hdv(a) : -1;
+}
+
+hipError_t launch_attention_group(const AttnRowsArgs *as, int n, hipStream_t s) {
+  if (n < 1 || n > kGroupMax) return hipErrorInvalidValue;
+  long all = 0;
+  for (int p = 0; p < n; p++) {
+    const AttnRowsArgs &a = as[p];
+    if (a.heads <= 0 || a.c % a.heads || a.c / a.heads > 64 || attention_hdv(a) != attention_hdv(as[0]))
+      return hipErrorInvalidValue;
+    all += (long)a.lanes * a.heads;
+  }
+  const int hdv = attention_hdv(as[0]);
+  // Lines whose K, V and a run's scores fit LDS.
+  Group<AttnRowsArgs> g{};
+  long blocks = 0;
+  size_t rshm = 0;
+  bool rows = true;
+  for (int p = 0; p < n; p++) {
+    const AttnRowsArgs &a = as[p];
+    const int runs = attention_runs(a.t, hdv, all, n > 1);
+    rows = rows && runs > 0;
+    if (!rows) break;
+    g.first[p] = (int)blocks, g.x[p] = runs, g.a[p] = a;
+    blocks += (long)a.lanes * a.heads * runs;
+    if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    rshm = std::max(rshm, attention_rows_floats(a.t, hdv, runs) * sizeof(float));
+  }
+  if (rows) {
+    g.n = n, g.first[n] = (int)blocks;
+    const dim3 grid((unsigned)blocks);
+    auto go = [&](auto one, auto many) {
+      if (n == 1)
+        hipLaunchKernelGGL(one, grid, dim3(256), rshm, s, group_of<1>(g));
+      else
+        hipLaunchKernelGGL(many, grid, dim3(256), rshm, s, g);
+      return hipGetLastError();
+    };
+    if (hdv == 16) return go(attention_rows<16, 1>, attention_rows<16, kGroupMax>);
+    if (hdv == 32) return go(attention_rows<32, 1>, attention_rows<32, kGroupMax>);
+    return go(attention_rows<64, 1>, attention_rows<64, kGroupMax>);
+  }
+  if (n > 1) return hipErrorInvalidValue;
+  const AttnRowsArgs &a = as[0];
+  const int t = a.t, hd = a.c / a.heads;
+  const bool lds = attention_in_lds(t, hd);
+  if (!lds && !a.scratch) return hipErrorInvalidValue;
+  const size_t shm = attention_lds_floats(t, hd, lds) * sizeof(float);
   if (shm > kMaxLds) return hipErrorInvalidValue;
-  float *g = lds ? nullptr : scratch;
+  float *sc = lds ? nullptr : a.scratch;
   auto go = [&](auto kernel, int nt) {
     // Allowed before any use beyond 64 KiB (and so before a graph capture
     // records such a launch).
@@ -1883,28 +2065,10 @@ hipError_t launch_attention(const float *x, long x_lane_stride, float scale, int
       hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), int(kMaxLds));
       if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(kernel, dim3(lanes * heads), dim3(nt), shm, s, x, x_lane_stride, scale, t,
-                       c, heads, y, y_lane_stride, g);
+    hipLaunchKernelGGL(kernel, dim3(a.lanes * a.heads), dim3(nt), shm, s, a.x, a.x_lane_stride, a.scale, t,
+                       a.c, a.heads, a.y, a.y_lane_stride, sc);
     return hipGetLastError();
   };
-  // Lines whose K, V and a run's scores fit LDS: runs of query rows, enough
-  // blocks for two per CU.
-  const int hdv = hd <= 16 ? 16 : (hd <= 32 ? 32 : 64);
-  const int runs = std::max(1, std::min(t, (512 + lanes * heads - 1) / (lanes * heads)));
-  const size_t rshm = attention_rows_floats(t, hdv, runs) * sizeof(float);
-  if (rshm <= 64 * 1024) {
-    const long blocks = (long)lanes * heads * runs;
-    if (hdv == 16)
-      hipLaunchKernelGGL(attention_rows<16>, dim3((unsigned)blocks), dim3(256), rshm, s, x, x_lane_stride, scale, t,
-                         c, heads, runs, y, y_lane_stride);
-    else if (hdv == 32)
-      hipLaunchKernelGGL(attention_rows<32>, dim3((unsigned)blocks), dim3(256), rshm, s, x, x_lane_stride, scale, t,
-                         c, heads, runs, y, y_lane_stride);
-    else
-      hipLaunchKernelGGL(attention_rows<64>, dim3((unsigned)blocks), dim3(256), rshm, s, x, x_lane_stride, scale, t,
-                         c, heads, runs, y, y_lane_stride);
-    return hipGetLastError();
-  }
   if (hd <= 16) return go(attention_kernel<16, 1024>, 1024);
   if (hd <= 32) return go(attention_kernel<32, 512>, 512);
   return go(attention_kernel<64, 256>, 256);
