@@ -140,8 +140,8 @@ const uint64_t *ppocr_gpu_lane_db_mask(const ppocr_gpu_model *model, size_t lane
                                        size_t *rows);
 
 /* Runs record their launches in a HIP graph from the second run after the
- * lanes were set, and replay it (default, `enable` 1); with 0 every run
- * launches each kernel itself. Returns 0, or 1 for a NULL model. */
+ * lanes were set, and replay it (default, `enable` 1), unless they are so few
+ * that launching them is faster; with 0 every run launches each kernel itself. Returns 0, or 1 for a NULL model. */
 int ppocr_gpu_set_graphs(ppocr_gpu_model *model, int enable);
 
 /* Kernel launches one run makes, and launch `i`'s kernel name (valid for the

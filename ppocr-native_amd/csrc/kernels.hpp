@@ -572,6 +572,18 @@ hipError_t launch_copy_lds(const float *x, float *y, long n, hipStream_t s);
 hipError_t launch_db_bits(const float *map, long lane_stride, int w, int h, int lanes, float thresh,
                           unsigned long long *bits, hipStream_t s);
 
+// Lanes of n floats, each `*_stride` floats after the last, from src to dst,
+// either of which may be pinned host memory; any number of them, up to
+// kGroupMax a launch.
+struct CopyArgs {
+  const float *src;
+  long src_stride;
+  float *dst;
+  long dst_stride;
+  int n, lanes;
+};
+hipError_t launch_copy(const CopyArgs *a, int n, hipStream_t s);
+
 // ------------------------------------------------------------- image stages
 
 // Device-memory image stages (HWC, 8-bit BGR in). See image.hip.

@@ -229,6 +229,12 @@ struct Model {
   // The launches of one run over every batch, captured as a HIP graph on the
   // second run after the lanes were arranged (the first runs them eagerly,
   // which also sets any kernel attribute outside the capture).
+  // A replay costs about 15 us before its first kernel starts, and then
+  // spaces its kernels closer than the host can launch them: from about ten
+  // launches on it is no slower, and it leaves the host free (a call of two
+  // launches: CTC head 106 us replayed, 94 launched; encoder 73 and 67; 26
+  // launches of the 224 x 320 detector 260 and 267).
+  static constexpr size_t kGraphLaunches = 9;
   bool use_graphs = true;
   int eager_runs = 0;
   // The output whose DB threshold each run also writes as row bitmasks
@@ -265,6 +271,9 @@ struct Model {
   bool run(bool copy_in, bool copy_out, std::string &err, bool sync = true);
   bool set_db_mask(long output, float thresh, std::string &err);
   bool copy_out_all(std::string &err);
+  // The most bytes a kernel copies to and from the host (the rest by DMA).
+  static constexpr size_t kKernelCopyIn = size_t(1) << 20, kKernelCopyOut = size_t(64) << 20;
+  bool host_copy(const std::vector<CopyArgs> &cs, hipMemcpyKind kind, const char *what, std::string &err);
   std::vector<size_t> step_reads(const Step &s) const;
   int enc_hidden(const Step &s) const { return s.kind == S_ENC_BLOCK ? int(plan.ops[s.m_fc1].oc) : 0; }
   size_t step_writes(const Step &s) const;
@@ -2190,7 +2199,7 @@ void Model::drop_graph() {
 // after the lanes were arranged, from the captured graph afterwards. A
 // capture that fails leaves the model running eagerly.
 bool Model::enqueue(std::string &err) {
-  if (use_graphs && !graph_exec && eager_runs >= 1) {
+  if (use_graphs && !graph_exec && eager_runs >= 1 && run_list().size() >= kGraphLaunches) {
     bool ok = hipStreamBeginCapture(stream, hipStreamCaptureModeRelaxed) == hipSuccess;
     std::string ignored;
     ok = ok && launch_all(ignored);
@@ -2229,14 +2238,13 @@ bool Model::run(bool copy_in, bool copy_out, std::string &err, bool sync) {
   HIPTRY(hipSetDevice(device), "selecting the GPU");
   if (lane_at.empty()) return err = "no lanes are set", false;
   if (copy_in) {
+    std::vector<CopyArgs> in;
     for (size_t g = 0; g < active_batches; g++) {
       Batch &b = *batches[g];
-      const Plan &p = b.plan;
-      HIPTRY(hipMemcpy2DAsync(b.dev(p.in_slot), b.stride(p.in_slot) * sizeof(float), b.host_in,
-                              b.in_len * sizeof(float), b.in_len * sizeof(float), b.lanes.size(),
-                              hipMemcpyHostToDevice, stream),
-             "copying the input");
+      const size_t slot = b.plan.in_slot;
+      in.push_back({b.host_in, long(b.in_len), b.dev(slot), b.stride(slot), int(b.in_len), int(b.lanes.size())});
     }
+    if (!host_copy(in, hipMemcpyHostToDevice, "copying the input", err)) return false;
   }
   if (!enqueue(err)) return false;
   // The DB threshold's bitmasks of the map, after the forward (outside the
@@ -2257,20 +2265,34 @@ bool Model::run(bool copy_in, bool copy_out, std::string &err, bool sync) {
 // Every batch's outputs (and DB bitmasks) to the pinned host buffers, queued
 // on the model's stream.
 bool Model::copy_out_all(std::string &err) {
+  std::vector<CopyArgs> out;
   for (size_t g = 0; g < active_batches; g++) {
     Batch &b = *batches[g];
     const Plan &p = b.plan;
+    const int L = int(b.lanes.size());
     for (size_t k = 0; k < p.out_slot.size(); k++)
-      HIPTRY(hipMemcpy2DAsync(b.host_out[k], p.out_n[k] * sizeof(float), b.dev(p.out_slot[k]),
-                              b.stride(p.out_slot[k]) * sizeof(float), p.out_n[k] * sizeof(float),
-                              b.lanes.size(), hipMemcpyDeviceToHost, stream),
-             "copying the results");
-    if (db_output >= 0)
-      HIPTRY(hipMemcpyAsync(b.host_bits, b.arena + b.bits_off,
-                            b.lanes.size() * b.bits_h * b.bits_wpr * sizeof(unsigned long long),
-                            hipMemcpyDeviceToHost, stream),
-             "copying the DB mask");
+      out.push_back({b.dev(p.out_slot[k]), b.stride(p.out_slot[k]), b.host_out[k], long(p.out_n[k]), int(p.out_n[k]), L});
+    if (db_output >= 0) {
+      const long n = long(2 * b.bits_h * b.bits_wpr);
+      out.push_back({b.arena + b.bits_off, n, reinterpret_cast<float *>(b.host_bits), n, int(n), L});
+    }
   }
+  return host_copy(out, hipMemcpyDeviceToHost, "copying the results", err);
+}
+
+// Copies between the lanes and their pinned host memory, on the model's
+// stream: by launch_copy, all in one launch.
+bool Model::host_copy(const std::vector<CopyArgs> &cs, hipMemcpyKind kind, const char *what, std::string &err) {
+  size_t bytes = 0;
+  for (const CopyArgs &c : cs) bytes += size_t(c.n) * size_t(c.lanes) * sizeof(float);
+  if (bytes <= (kind == hipMemcpyHostToDevice ? kKernelCopyIn : kKernelCopyOut)) {
+    HIPTRY(launch_copy(cs.data(), int(cs.size()), stream), what);
+    return true;
+  }
+  for (const CopyArgs &c : cs)
+    HIPTRY(hipMemcpy2DAsync(c.dst, size_t(c.dst_stride) * sizeof(float), c.src, size_t(c.src_stride) * sizeof(float),
+                            size_t(c.n) * sizeof(float), size_t(c.lanes), kind, stream),
+           what);
   return true;
 }
 
