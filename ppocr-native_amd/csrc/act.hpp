@@ -80,4 +80,17 @@ __device__ __forceinline__ float act(float v, int a) {
   }
 }
 
+// An activation of four values, dispatched once for the four (the common
+// codes fold to their own few instructions).
+typedef float act_f4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ act_f4 act4(act_f4 v, int a) {
+  switch (a) {
+    case ACT_NONE: return v;
+    case ACT_RELU: return act_f4{act(v.x, ACT_RELU), act(v.y, ACT_RELU), act(v.z, ACT_RELU), act(v.w, ACT_RELU)};
+    case ACT_HARDSWISH:
+      return act_f4{act(v.x, ACT_HARDSWISH), act(v.y, ACT_HARDSWISH), act(v.z, ACT_HARDSWISH), act(v.w, ACT_HARDSWISH)};
+    default: return act_f4{act(v.x, a), act(v.y, a), act(v.z, a), act(v.w, a)};
+  }
+}
+
 }  // namespace ppocr

@@ -839,6 +839,234 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
   conv_patch_body<1, BN, CB, R8>(grp);
 }
 
+// ------------------------------------------------------ halo tiles, split
+
+// conv_patch's 3 x 3 windows for 17 to 32 outputs with the products on the
+// bf16 matrix cores (split.hpp). A tile is 16 output pixels by NW * WR rows of
+// a lane; for each block of 32 input channels (one MFMA step deep) the
+// workgroup stages the patch, split into its three parts (four threads a
+// pixel, eight channels each), and every tap's weights in LDS, the next
+// block's in flight to registers meanwhile. Every operand read is 1 KB of
+// consecutive LDS. A wave takes the window column by column, that column's
+// weights in registers, and reads each input row once for all its output
+// rows. Reduction order: channel block, window column, input row.
+//
+// What bounds it: the matrix cores, two waves a SIMD that wait together at
+// the block's barriers (LDS holds one workgroup a CU), and on small maps the
+// first loads and the three blocks in turn. Measured against f32 MFMA
+// (conv_patch): 96 -> 24 over four upsampled sources at 496 x 384 98.9 -> 58.6
+// us, the neck's four maps 129.6 -> 79.3; at 240 x 184 28.3 -> 20.8 and 34.3
+// -> 22.0; at 56 x 80 16.3 -> 11.6 and 16.4 -> 13.1, 48 -> 32 at stride 2 23.1
+// -> 11.1.
+constexpr int kSplitTaps = 9;
+// Tiles of 16 rows (eight waves of two) when that leaves most CUs one, of 8
+// (eight waves of one) when half, else of 4 (four waves of one).
+constexpr long kSplitTiles16 = 160, kSplitTiles8 = 128;
+constexpr int kSplitWeights = kSplitTaps * 2 * 192;  // 16-byte groups of a channel block's weights
+
+template <int NW, int WR, int S>
+struct SplitTile {
+  static constexpr int T = 64 * NW, TH = NW * WR;             // threads, output rows
+  static constexpr int PR = (TH - 1) * S + 3, PC = 15 * S + 3;  // the patch
+  static constexpr int NPX = PR * PC;
+  static constexpr int UNITS = (NPX * 4 + T - 1) / T;         // (pixel, 8 channels) a thread stages
+  static constexpr int WUNITS = (kSplitWeights + T - 1) / T;
+  static constexpr size_t LDS = size_t(NPX) * 192 + size_t(kSplitWeights) * 16;
+};
+
+template <int NW, int WR, int S, int GN>
+__global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> grp) {
+  typedef SplitTile<NW, WR, S> K;
+  constexpr int T = K::T, PC = K::PC, NPX = K::NPX, TW = 16;
+  const int bid = xcd_tile((int)blockIdx.x, (int)gridDim.x);
+  int prob = 0;
+#pragma unroll
+  for (int k = 1; k < GN; k++)
+    if (k < grp.n && bid >= grp.first[k]) prob = k;
+  const ConvArgs &a = grp.a[prob];
+  const int tiles_x = grp.x[prob], tiles_y = grp.y[prob];
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  split_u4 *P = reinterpret_cast<split_u4 *>(lds);       // part p's pixel q: P[(p * NPX + q) * 4 + g], channels 8g..
+  split_u4 *B = P + NPX * 12;                            // tap t, block j, part p, lane l: B[((t * 2 + j) * 3 + p) * 64 + l]
+  int t = bid - grp.first[prob];
+  const int tx0 = (t % tiles_x) * TW;
+  t /= tiles_x;
+  const int ty0 = (t % tiles_y) * K::TH, ln = t / tiles_y;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, lg = lane >> 4;
+  const int iy0 = ty0 * S - a.pt, ix0 = tx0 * S - a.pl;
+  const int cpt = (a.ctot + 31) / 32;
+  // A stride-2 patch keeps each row's even columns before its odd ones: the
+  // pixels a tap reads lie side by side.
+  auto place = [](int col) { return S == 1 ? col : (col & 1) * ((PC + 1) / 2) + (col >> 1); };
+
+  split_f4 rp[K::UNITS][2];
+  split_u4 rw[K::WUNITS];
+  const int g = tid & 3, p0 = tid >> 2;
+  auto fetch = [&](int cc) {
+    const int c = cc * 32 + g * 8;
+    const bool live = c < a.ctot;
+    const ConvSrc src = pick_src(a, live ? c : 0);
+    const int sh = src.shift, sw_ = a.iw >> sh;
+    const float *base = src.p + (long)ln * src.lane_stride + (c - src.coff);
+#pragma unroll
+    for (int k = 0; k < K::UNITS; k++) {
+      const int q = p0 + k * (T / 4), py = q / PC, px = q - py * PC;
+      const int iy = iy0 + py, ix = ix0 + px;
+      const bool in = live && q < NPX && iy >= 0 && iy < a.ih && ix >= 0 && ix < a.iw;
+      const float *p = base + ((long)(iy >> sh) * sw_ + (ix >> sh)) * src.c;
+      rp[k][0] = *reinterpret_cast<const split_f4 *>(in ? p : kPatchZeros);
+      rp[k][1] = *reinterpret_cast<const split_f4 *>(in ? p + 4 : kPatchZeros);
+    }
+    const split_u4 *wsrc = reinterpret_cast<const split_u4 *>(a.split_wt);
+#pragma unroll
+    for (int k = 0; k < K::WUNITS; k++) {
+      const int e = min(tid + k * T, kSplitWeights - 1), tj = e / 192;
+      rw[k] = wsrc[((long)tj * cpt + cc) * 192 + (e - tj * 192)];
+    }
+  };
+  auto store = [&]() {
+#pragma unroll
+    for (int k = 0; k < K::UNITS; k++) {
+      const int q = p0 + k * (T / 4), py = q / PC, px = q - py * PC;
+      if (q < NPX) {
+        split_u4 v[3];
+        split8(rp[k][0], rp[k][1], v[0], v[1], v[2]);
+#pragma unroll
+        for (int p = 0; p < 3; p++) P[(p * NPX + py * PC + place(px)) * 4 + g] = v[p];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < K::WUNITS; k++)
+      if (tid + k * T < kSplitWeights) B[tid + k * T] = rw[k];
+  };
+  const float *bsrc = a.bias ? a.bias : kPatchZeros;
+  float bcol[2];
+#pragma unroll
+  for (int j = 0; j < 2; j++) bcol[j] = bsrc[a.bias ? min(j * 16 + li, a.n - 1) : 0];
+
+  f32x4 hi[WR][2], lo[WR][2];
+#pragma unroll
+  for (int i = 0; i < WR; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) hi[i][j] = lo[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+
+  fetch(0);
+  for (int cc = 0; cc < cpt; cc++) {
+    if (cc) __syncthreads();  // every wave is done with the previous block
+    store();
+    __syncthreads();
+    if (cc + 1 < cpt) fetch(cc + 1);
+    // The next block's loads stay ahead of this block's multiply-adds.
+    asm volatile("" ::: "memory");
+    // Window column by window column: its taps' weights in registers, then
+    // every input row of the wave's output rows once.
+#pragma unroll
+    for (int kx = 0; kx < 3; kx++) {
+      bf16x8 bv[3][2][3];
+#pragma unroll
+      for (int ky = 0; ky < 3; ky++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+          for (int p = 0; p < 3; p++)
+            bv[ky][j][p] = __builtin_bit_cast(bf16x8, B[(((ky * 3 + kx) * 2 + j) * 3 + p) * 64 + lane]);
+#pragma unroll
+      for (int r = 0; r < (WR - 1) * S + 3; r++) {
+        const int pix = (wave * WR * S + r) * PC + place(kx) + li;
+        bf16x8 av[3];
+#pragma unroll
+        for (int p = 0; p < 3; p++) av[p] = __builtin_bit_cast(bf16x8, P[(p * NPX + pix) * 4 + lg]);
+#pragma unroll
+        for (int s = 0; s < 6; s++)
+#pragma unroll
+          for (int i = 0; i < WR; i++) {
+            const int ky = r - i * S;
+            if (ky < 0 || ky > 2) continue;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+              f32x4 &d = s == 5 ? hi[i][j] : lo[i][j];
+              d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[pa[s]], bv[ky][j][pb[s]], d, 0, 0, 0);
+            }
+          }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < WR; i++) {
+    const int oy = ty0 + wave * WR + i;
+    if (oy >= a.oh) continue;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const int n = j * 16 + li, ox = tx0 + lg * 4;
+      if (n >= a.n) continue;
+      const long at = ((long)oy * a.ow + ox) * a.n + n;
+      f32x4 v = hi[i][j] + lo[i][j];
+      if (a.bias) v = v + bcol[j];
+      v = act4(v, a.act);
+      if (a.res) {
+        const float *res = a.res + (long)ln * a.res_lane_stride + at;
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = v[r] + (ox + r < a.ow ? res[(long)r * a.n] : 0.0f);
+        v = act4(v, a.act2);
+      }
+      float *y = a.y + (long)ln * a.y_lane_stride + at;
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if (ox + r < a.ow) y[(long)r * a.n] = v[r];
+    }
+  }
+}
+
+bool patch_split_shape(int kh, int kw, int sh, int sw, int n) {
+  return kh == 3 && kw == 3 && sh == sw && (sh == 1 || sh == 2) && n > 16 && n <= 32;
+}
+
+size_t patch_split_floats(int ctot) { return size_t(kSplitTaps) * split_pack_floats((ctot + 31) / 32 * 32, 32); }
+
+template <int NW, int WR, int S>
+static hipError_t go_patch_split(const ConvArgs *as, int n, hipStream_t s) {
+  typedef SplitTile<NW, WR, S> K;
+  Group<ConvArgs> g{};
+  long blocks = 0;
+  for (int p = 0; p < n; p++) {
+    const ConvArgs &a = as[p];
+    g.first[p] = (int)blocks, g.a[p] = a;
+    g.x[p] = (a.ow + 15) / 16, g.y[p] = (a.oh + K::TH - 1) / K::TH;
+    blocks += (long)a.lanes * g.x[p] * g.y[p];
+    if (blocks < 1 || blocks > 0x7fffffffL) return hipErrorInvalidValue;
+  }
+  g.n = n, g.first[n] = (int)blocks;
+  auto go = [&](auto kernel, const auto &gr) {
+    hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), (int)K::LDS);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(K::T), K::LDS, s, gr);
+    return hipGetLastError();
+  };
+  if (n == 1) return go(conv_patch_split<NW, WR, S, 1>, group_of<1>(g));
+  return go(conv_patch_split<NW, WR, S, kGroupStep>, group_of<kGroupStep>(g));
+}
+
+hipError_t launch_conv_patch_split_group(const ConvArgs *as, int n, hipStream_t s) {
+  if (n < 1 || n > kGroupStep) return hipErrorInvalidValue;
+  long tiles16 = 0, tiles8 = 0;
+  for (int p = 0; p < n; p++) {
+    const ConvArgs &a = as[p];
+    if (!patch_split_shape(a.kh, a.kw, a.sh, a.sw, a.n) || a.sh != as[0].sh || a.mode != GEMM_STORE || a.gate || a.pw_w ||
+        !a.split_wt || a.nsrc < 1 || a.nsrc > 4)
+      return hipErrorInvalidValue;
+    for (int k = 0; k < a.nsrc; k++)
+      if (a.src[k].c % 8 || a.src[k].coff % 8 || a.src[k].lane_stride % 4) return hipErrorInvalidValue;
+    tiles16 += (long)a.lanes * ((a.ow + 15) / 16) * ((a.oh + 15) / 16);
+    tiles8 += (long)a.lanes * ((a.ow + 15) / 16) * ((a.oh + 7) / 8);
+  }
+  if (as[0].sh == 2) return go_patch_split<4, 1, 2>(as, n, s);
+  if (tiles16 >= kSplitTiles16) return go_patch_split<8, 2, 1>(as, n, s);
+  if (tiles8 >= kSplitTiles8) return go_patch_split<8, 1, 1>(as, n, s);
+  return go_patch_split<4, 1, 1>(as, n, s);
+}
+
 // One wave per row: join the row's tile partials, then y = (best, 1 / sum).
 // The tiles also carry their second value: when the row's two largest
 // values lie within `tie` of each other, the GPU's summation order could

@@ -165,6 +165,9 @@ struct ConvArgs {
   // columns a pixel. Null pw_w: none.
   const float *pw_w, *pw_b;
   int pw_n, pw_act;
+  // launch_conv_patch_split_group: the weights' bf16 parts, tap by tap in
+  // SplitPackArgs' order (kp = ctot padded to 32, columns to 32).
+  const float *split_wt;
 };
 
 struct GemmTile {
@@ -202,6 +205,13 @@ size_t patch_lds_bytes(const ConvArgs &a, int wr, int bk, int bn);
 hipError_t launch_conv_patch(const ConvArgs &a, int wr, int bk, int bn, hipStream_t s);
 // n <= kGroupStep problems, each patch_supported for (wr, bk, bn), as one launch.
 hipError_t launch_conv_patch_group(const ConvArgs *a, int n, int wr, int bk, int bn, hipStream_t s);
+
+// The 3 x 3 window on halo tiles with its products on the bf16 matrix cores
+// (split.hpp): stride 1 or 2, 17 to 32 outputs, sources of channels a
+// multiple of 8, no gate. n <= kGroupStep problems of one stride.
+bool patch_split_shape(int kh, int kw, int sh, int sw, int n);
+size_t patch_split_floats(int ctot);  // of the weights' parts
+hipError_t launch_conv_patch_split_group(const ConvArgs *a, int n, hipStream_t s);
 
 // The CTC head over rows of ci inputs, rows_per_lane of them per lane:
 // launch_ctc_direct_group (an input at most 128 wide, a multiple of 4; or

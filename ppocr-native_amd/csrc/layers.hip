@@ -492,18 +492,6 @@ __host__ __device__ inline DwPwLds dwpw_lds(const DwArgs &d, int n, int tr, int 
   return l;
 }
 
-// An activation of four values, dispatched once for the four (the common
-// codes fold to their own few instructions).
-__device__ __forceinline__ f32x4 act4(f32x4 v, int a) {
-  switch (a) {
-    case ACT_NONE: return v;
-    case ACT_RELU: return f32x4{act(v.x, ACT_RELU), act(v.y, ACT_RELU), act(v.z, ACT_RELU), act(v.w, ACT_RELU)};
-    case ACT_HARDSWISH:
-      return f32x4{act(v.x, ACT_HARDSWISH), act(v.y, ACT_HARDSWISH), act(v.z, ACT_HARDSWISH), act(v.w, ACT_HARDSWISH)};
-    default: return f32x4{act(v.x, a), act(v.y, a), act(v.z, a), act(v.w, a)};
-  }
-}
-
 // The 1x1's products over KQ groups of 16 channels: wave-uniform, every
 // column block of the wave (blocks past the last are computed and dropped),
 // no branch inside the chain.

@@ -102,6 +102,7 @@ struct Step {
   std::vector<int> chain, chain_gate;
   bool dw_sums = false;    // S_DW: also sum its output per channel for the next step's mean
   bool patch = false;      // S_GEMM: a windowed convolution on halo tiles (conv_patch)
+  bool patch_split = false;  // ... whose products run on the bf16 matrix cores
   bool ring = false;       // S_GEMM: a windowed convolution on the LDS ring (conv_ring)
   int mean_of_dw = -1;     // S_MEAN: the depthwise operation whose sums it joins
   int elt = 0;             // EltMode
@@ -953,6 +954,17 @@ bool Model::pack(std::string &err) {
           if (waste < pw_best - 1e-12) pb = cand, pw_best = waste;
         }
         if (pb) s.patch = true, bk = pb;
+        bool eights = s.gate < 0;
+        for (auto &x : srcs) eights = eights && x.c % 8 == 0;
+        if (pb && eights && patch_split_shape(int(op.kh), int(op.kw), int(op.sh), int(op.sw), N)) {
+          // The taps' bf16 parts, one packing after the other.
+          s.patch_split = true;
+          const int kp = (ctot + 31) / 32 * 32;
+          for (int tap = 0; tap < taps; tap++) {
+            const size_t at = split_job({dweights + op.w0 + size_t(tap) * ctot * N, ctot, N, kp, N, 0, N, nullptr});
+            if (!tap) s.split_w = at;
+          }
+        }
       }
       // A windowed convolution that neither halo tiles nor the register-staged
       // implicit GEMM take well (a window wider than 3 or unequal strides)
@@ -1357,6 +1369,13 @@ void Model::build_launches(Batch &b) {
           const int wr = patch_rows(tiles4, tiles8, patch_fits(a.kh, a.kw, a.sh, 2, t.bk, t.bn),
                                     patch_lds_bytes(a, 1, t.bk, t.bn), patch_lds_bytes(a, 2, t.bk, t.bn));
           const int bk = t.bk, bn = t.bn;
+          if (s.patch_split) {
+            a.split_wt = dsplit + s.split_w;
+            b.launches.push_back({"conv_patch", s.op, [a](hipStream_t st) { return launch_conv_patch_split_group(&a, 1, st); }});
+            Launch &l = b.launches.back();
+            l.gk = GK_PATCH, l.gkey = -a.sh, l.conv = a, l.bk = bk, l.bn = bn;
+            break;
+          }
           b.launches.push_back({"conv_patch", s.op, [a, wr, bk, bn](hipStream_t st) {
                                   return launch_conv_patch(a, wr, bk, bn, st);
                                 }});
@@ -1870,6 +1889,10 @@ void Model::group(Batch &b) const {
           fits2 = fits2 && patch_fits(x.conv.kh, x.conv.kw, x.conv.sh, 2, x.bk, x.bn);
           lds4 = std::max(lds4, patch_lds_bytes(x.conv, 1, x.bk, x.bn));
           lds8 = std::max(lds8, patch_lds_bytes(x.conv, 2, x.bk, x.bn));
+        }
+        if (as[0].split_wt) {
+          gl.fn = [as](hipStream_t st) { return launch_conv_patch_split_group(as.data(), int(as.size()), st); };
+          break;
         }
         const int wr = patch_rows(tiles4, tiles8, fits2, lds4, lds8), bk = gl.bk, bn = gl.bn;
         gl.fn = [as, wr, bk, bn](hipStream_t st) {

@@ -60,3 +60,60 @@ def test_ctc_panel_odd_values(oracle):
     want = oracle.OracleModel(plan).run(y)[0].reshape(-1, 2)
     assert b[11, 0] == want[11, 0]
     np.testing.assert_allclose(b[11, 1], want[11, 1], rtol=1e-5)
+
+
+def conv_plan(rng, h, w, cs, n, s, act, res):
+    """A 3 x 3 window over one map of cs[0] channels and, upsampled by two,
+    one of cs[1]; with an Add of its output and a 1 x 1 layer's when `res`."""
+    b = PlanBuilder(h, w, 8)
+    x = b.conv(b.input, rng.normal(0, 0.4, (1, 1, 8, cs[0])).astype(np.float32), None)
+    ctot, up = sum(cs), None
+    if len(cs) > 1:
+        half = b.conv(b.input, rng.normal(0, 0.2, (2, 2, 8, cs[1])).astype(np.float32), None, k=(2, 2), s=(2, 2))
+        up = b.upsample(half, 2)
+    wt = rng.normal(0, 1 / np.sqrt(9 * ctot), (3, 3, ctot, n)).astype(np.float32)
+    y = b.conv(x, wt, rng.normal(0, 0.3, n).astype(np.float32), k=(3, 3), s=(s, s), pad=(1, 1, 1, 1), x2=up, fused=act)
+    if res:
+        r = b.conv(b.input, rng.normal(0, 0.4, (1, 1, 8, n)).astype(np.float32), None, s=(s, s))
+        y = b.add(y, r, fused="relu")
+    return b.to_bytes([y])
+
+
+# Tiles of 4, 8 and 16 rows (few tiles, more, enough for 160 of 16 rows over
+# the lanes), edges that cut them, channels within and past a block of 32, 17
+# to 32 outputs, both strides, two sources, a folded Add.
+@pytest.mark.parametrize("h,w,cs,n,s,act,res", [
+    (1, 1, (8,), 17, 1, "none", False), (5, 17, (40,), 24, 1, "hardswish", True), (33, 31, (96,), 32, 1, "relu", False),
+    (66, 130, (32, 24), 24, 1, "relu", True), (150, 220, (24, 72), 20, 1, "none", False),
+    (7, 9, (48,), 32, 2, "hardswish", False), (64, 66, (16, 16), 25, 2, "relu", True)])
+def test_conv_patch_split(oracle, h, w, cs, n, s, act, res):
+    rng = np.random.default_rng(h + w)
+    plan = conv_plan(rng, h, w, cs, n, s, act, res)
+    xs = [rng.uniform(-1, 1, (h, w, 8)).astype(np.float32) for _ in range(3)]
+    m = oracle.OracleModel(plan)
+    for x, got in zip(xs, gpu(plan, (h, w, 8), xs)):
+        want = m.run(x)[0].reshape(-1).astype(np.float64)
+        # The layer tests' tolerance for sums in another order.
+        assert (np.abs(got - want) <= 1e-5 * np.abs(want) + 1e-5).all()
+
+
+def test_conv_patch_split_odd_values(oracle):
+    """An infinity or NaN reaches the outputs its window covers as it does in
+    f32, and no others."""
+    rng = np.random.default_rng(8)
+    b = PlanBuilder(20, 24, 16)
+    wt = rng.normal(0, 0.1, (3, 3, 16, 24)).astype(np.float32)
+    plan = b.to_bytes([b.conv(b.input, wt, None, k=(3, 3), pad=(1, 1, 1, 1))])
+    x = rng.uniform(-1, 1, (20, 24, 16)).astype(np.float32)
+    y = x.copy()
+    y[3, 4, 5], y[10, 20, 2], y[17, 1, 15], y[14, 10, 0] = np.inf, -np.inf, np.nan, 3.4e38
+    a, c = (v.reshape(20, 24, 24) for v in gpu(plan, (20, 24, 16), [x, y]))
+    want = oracle.OracleModel(plan).run(y)[0].reshape(20, 24, 24)
+    far = np.ones((20, 24), bool)
+    for py, px in ((3, 4), (10, 20), (17, 1), (14, 10)):
+        far[max(py - 1, 0):py + 2, max(px - 1, 0):px + 2] = False
+    assert np.array_equal(a[far].view(np.uint32), c[far].view(np.uint32))
+    assert np.array_equal(np.isnan(c), np.isnan(want)) and np.array_equal(np.isinf(c), np.isinf(want))
+    assert np.array_equal(c[np.isinf(c)], want[np.isinf(want)])
+    fin = np.isfinite(want)
+    np.testing.assert_allclose(c[fin], want[fin], rtol=1e-5, atol=1e-5)
