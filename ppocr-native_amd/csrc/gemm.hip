@@ -125,16 +125,43 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v + dpp16<0x140>(v);
 }
 
-// A CTC tile's per-row statistics from its logits (acc + bias, columns past
-// the vocabulary -inf): per row the maximum, the sum of exp(v - max) by
+// A row's statistics over a tile from its logits v (lane li's columns n0 +
+// 16j + li; -inf past the vocabulary): the maximum, the sum of exp(v - max) by
 // hardware exp2, the first column holding the maximum and the second value,
-// each the same in the 16 lanes of the row's DPP row, handed to `use` with
-// the row's block and index in it.
+// each the same in the 16 lanes of the row's DPP row.
+template <int NT>
+__device__ __forceinline__ float4 ctc_row(const float (&v)[NT], int n0, int lane) {
+  constexpr float L = 1.44269504088896341f;  // log2(e)
+  float lm = -__builtin_inff(), lb = __builtin_inff(), ls = -__builtin_inff();
+#pragma unroll
+  for (int j = 0; j < NT; j++) {
+    const int n = n0 + j * 16 + (lane & 15);
+    if (v[j] > lm)
+      ls = lm, lm = v[j], lb = (float)n;
+    else if (v[j] > ls)
+      ls = v[j];
+  }
+  const float gm = row16_max(lm);
+  // The tile's second value (the maximum again when two columns hold
+  // it), for the near-tie check of ctc_merge.
+  float g2 = row16_max(lm == gm ? ls : lm);
+  const unsigned long long held = __ballot(lm == gm);
+  if (__popcll((held >> (lane & 48)) & 0xffffull) >= 2) g2 = gm;
+  const float c = gm * L;
+  float sum = 0.0f;
+#pragma unroll
+  for (int j = 0; j < NT; j++) sum += __builtin_amdgcn_exp2f(fmaf(v[j], L, -c));
+  sum = row16_sum(sum);
+  const float b = row16_min(lm == gm ? lb : __builtin_inff());
+  return make_float4(gm, sum, b, g2);
+}
+
+// A CTC tile's per-row statistics (ctc_row) from its products, with the bias
+// added, handed to `use` with the row's block and index in it.
 template <int MT, int NT, typename Use>
 __device__ __forceinline__ void ctc_tile_rows(const f32x4 (&acc)[MT][NT], int n0, const float *bias, int vocab,
                                               int lane, Use use) {
   const int li = lane & 15;
-  constexpr float L = 1.44269504088896341f;  // log2(e)
   float bn[NT];  // this lane's columns' bias, once for the tile's rows
 #pragma unroll
   for (int j = 0; j < NT; j++) {
@@ -146,29 +173,10 @@ __device__ __forceinline__ void ctc_tile_rows(const f32x4 (&acc)[MT][NT], int n0
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       float v[NT];
-      float lm = -__builtin_inff(), lb = __builtin_inff(), ls = -__builtin_inff();
 #pragma unroll
-      for (int j = 0; j < NT; j++) {
-        const int n = n0 + j * 16 + li;
-        v[j] = n < vocab ? acc[i][j][r] + bn[j] : -__builtin_inff();
-        if (v[j] > lm)
-          ls = lm, lm = v[j], lb = (float)n;
-        else if (v[j] > ls)
-          ls = v[j];
-      }
-      const float gm = row16_max(lm);
-      // The tile's second value (the maximum again when two columns hold
-      // it), for the near-tie check of ctc_merge.
-      float g2 = row16_max(lm == gm ? ls : lm);
-      const unsigned long long held = __ballot(lm == gm);
-      if (__popcll((held >> (lane & 48)) & 0xffffull) >= 2) g2 = gm;
-      const float c = gm * L;
-      float sum = 0.0f;
-#pragma unroll
-      for (int j = 0; j < NT; j++) sum += __builtin_amdgcn_exp2f(fmaf(v[j], L, -c));
-      sum = row16_sum(sum);
-      const float b = row16_min(lm == gm ? lb : __builtin_inff());
-      use(i, r, make_float4(gm, sum, b, g2));
+      for (int j = 0; j < NT; j++)
+        v[j] = n0 + j * 16 + li < vocab ? acc[i][j][r] + bn[j] : -__builtin_inff();
+      use(i, r, ctc_row<NT>(v, n0, lane));
     }
   }
 }
@@ -874,6 +882,23 @@ struct SplitTile {
   static constexpr size_t LDS = size_t(NPX) * 192 + size_t(kSplitWeights) * 16;
 };
 
+// Output (oy, ox) of column n of lane ln by f32 multiply-adds, the taps in
+// row-major order and each one's channels in order; `wt` in the plan's order.
+template <int K, int S>
+__device__ __forceinline__ float conv_f32(const ConvArgs &a, int ln, int oy, int ox, int n) {
+  float sum = 0.0f;
+  for (int tap = 0; tap < K * K; tap++) {
+    const int iy = oy * S - a.pt + tap / K, ix = ox * S - a.pl + tap % K;
+    if (iy < 0 || iy >= a.ih || ix < 0 || ix >= a.iw) continue;
+    for (int c = 0; c < a.ctot; c++) {
+      const ConvSrc src = pick_src(a, c);
+      const float x = src.p[(long)ln * src.lane_stride + ((long)(iy >> src.shift) * (a.iw >> src.shift) + (ix >> src.shift)) * src.c + c - src.coff];
+      sum = fmaf(x, a.wt[((long)tap * a.ctot + c) * a.n + n], sum);
+    }
+  }
+  return sum;
+}
+
 template <int NW, int WR, int S, int GN>
 __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> grp) {
   typedef SplitTile<NW, WR, S> K;
@@ -993,6 +1018,26 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
       }
     }
   }
+  // Outputs that came out as an infinity or NaN again by f32 multiply-adds.
+  uint32_t odd = 0;
+#pragma unroll
+  for (int i = 0; i < WR; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      hi[i][j] = hi[i][j] + lo[i][j];
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if (!(fabsf(hi[i][j][r]) < __builtin_inff()) && ty0 + wave * WR + i < a.oh && tx0 + lg * 4 + r < a.ow && j * 16 + li < a.n)
+          odd |= 1u << ((i * 2 + j) * 4 + r);
+    }
+  while (__builtin_expect(odd != 0, 0)) {
+    const int b = __builtin_ctz(odd);
+    odd &= odd - 1;
+    const float v = conv_f32<3, S>(a, ln, ty0 + wave * WR + (b >> 3), tx0 + lg * 4 + (b & 3), (b >> 2 & 1) * 16 + li);
+#pragma unroll
+    for (int k = 0; k < WR * 8; k++)
+      if (k == b) hi[k >> 3][k >> 2 & 1][k & 3] = v;
+  }
 #pragma unroll
   for (int i = 0; i < WR; i++) {
     const int oy = ty0 + wave * WR + i;
@@ -1002,7 +1047,7 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
       const int n = j * 16 + li, ox = tx0 + lg * 4;
       if (n >= a.n) continue;
       const long at = ((long)oy * a.ow + ox) * a.n + n;
-      f32x4 v = hi[i][j] + lo[i][j];
+      f32x4 v = hi[i][j];
       if (a.bias) v = v + bcol[j];
       v = act4(v, a.act);
       if (a.res) {
@@ -1329,8 +1374,7 @@ __global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(
         for (int j = 0; j < 2; j++) acc[i][2 * h + j] = hi[i][j] + lo[i][j];
     }
     const int k = t % kCtcRunTiles;
-    ctc_tile_rows<MT, 4>(acc, t * 64, a.bias, vocab, lane, [&](int i, int r, float4 rec) {
-      const int row = wave * 16 * MT + i * 16 + lg * 4 + r;
+    auto store = [&](int row, float4 rec) {
       const int m = tm * kCtcRows + row;
       if (li != 0) return;
       if (per_run == 1) {
@@ -1340,7 +1384,29 @@ __global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(
       recs[row * kCtcRunTiles + k] = rec;
       // The tiles' own maxima, after the runs' records.
       if (m < M) a.part[(long)M * runs * 4 + (long)t * M + m] = rec.x;
+    };
+    // Rows that hold an infinity or NaN (in 16 lanes alike).
+    uint32_t odd = 0;
+    ctc_tile_rows<MT, 4>(acc, t * 64, a.bias, vocab, lane, [&](int i, int r, float4 rec) {
+      store(wave * 16 * MT + i * 16 + lg * 4 + r, rec);
+      if (!(fabsf(rec.x) < __builtin_inff()) || rec.y != rec.y) odd |= 1u << (i * 4 + r);
     });
+    // Those again by f32 multiply-adds (split.hpp).
+    while (__builtin_expect(odd != 0, 0)) {
+      const int b = __builtin_ctz(odd), row = wave * 16 * MT + (b >> 2) * 16 + lg * 4 + (b & 3);
+      odd &= odd - 1;
+      const int m = min(tm * kCtcRows + row, M - 1), ln = m / a.rows_per_lane;
+      const float *xr = a.x + ln * a.x_lane_stride + (long)(m - ln * a.rows_per_lane) * a.ci;
+      float v[4];
+      for (int j = 0; j < 4; j++) {
+        const int n = t * 64 + j * 16 + li, nc = min(n, vocab - 1);
+        const float *wr = a.wt + (long)nc * a.wt_k;
+        float sum = 0.0f;
+        for (int c = 0; c < a.ci; c++) sum = fmaf(xr[c], wr[c], sum);
+        v[j] = n < vocab ? sum + a.bias[nc] : -__builtin_inff();
+      }
+      store(row, ctc_row<4>(v, t * 64, lane));
+    }
     // A run's last tile: each row's records joined in column order, one
     // record out. (The next tile's stores wait behind its first barrier.)
     if (per_run > 1 && (k == kCtcRunTiles - 1 || t + 1 == t1)) {
@@ -1397,7 +1463,7 @@ hipError_t launch_ctc_direct_group(const CtcArgs *as, int n, hipStream_t s) {
   for (int p = 0; p < n; p++) {
     const CtcArgs &a = as[p];
     const long M = (long)a.rows_per_lane * a.lanes;
-    if (!ctc_direct_supported(a.ci) || a.x_lane_stride % 4 || a.vocab <= 0 || M <= 0 || M >= (1L << 31) || !a.split_wt ||
+    if (!ctc_direct_supported(a.ci) || a.x_lane_stride % 4 || a.vocab <= 0 || M <= 0 || M >= (1L << 31) || !a.split_wt || !a.wt ||
         a.ci != a0.ci || a.vocab != a0.vocab)
       return hipErrorInvalidValue;
   }

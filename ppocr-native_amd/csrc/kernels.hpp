@@ -166,7 +166,8 @@ struct ConvArgs {
   const float *pw_w, *pw_b;
   int pw_n, pw_act;
   // launch_conv_patch_split_group: the weights' bf16 parts, tap by tap in
-  // SplitPackArgs' order (kp = ctot padded to 32, columns to 32).
+  // SplitPackArgs' order (kp = ctot padded to 32, columns to 32); `wt` is then
+  // the plan's own, tap by tap and channel by channel rows of n.
   const float *split_wt;
 };
 
@@ -224,7 +225,7 @@ struct CtcArgs {
   long x_lane_stride;
   int rows_per_lane, lanes, ci, vocab;
   const float *split_wt;  // SplitPackArgs' order, kp = ctc_direct_kpad(ci); null: `part` is launch_conv's
-  const float *wt;        // packed weights: column n's ci inputs at wt + n * wt_k
+  const float *wt;        // packed weights: column n's ci inputs at wt + n * wt_k (with split_wt never null)
   long wt_k;
   const float *bias;      // per column
   float *part;            // ctc_part_floats(rows, vocab) floats, 16-byte aligned

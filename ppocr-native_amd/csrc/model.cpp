@@ -1371,6 +1371,7 @@ void Model::build_launches(Batch &b) {
           const int bk = t.bk, bn = t.bn;
           if (s.patch_split) {
             a.split_wt = dsplit + s.split_w;
+            a.wt = W + op.w0, a.wt_k = 0;
             b.launches.push_back({"conv_patch", s.op, [a](hipStream_t st) { return launch_conv_patch_split_group(&a, 1, st); }});
             Launch &l = b.launches.back();
             l.gk = GK_PATCH, l.gkey = -a.sh, l.conv = a, l.bk = bk, l.bn = bn;

@@ -12,10 +12,9 @@
 // are at most 2^-7 of the whole, so summing them in an accumulator of their
 // own keeps the count of full-size roundings at one per product, as in f32.
 //
-// Values that have no such triple: an infinity or NaN goes whole into the
-// third part with the first two zero, so that its one product with a first
-// part has the sign and the class of the f32 product (0 * inf is NaN in
-// both); a finite value past bf16's largest takes its first part truncated.
+// Infinities, NaN, values that round past bf16's largest, and sums within
+// 2^-7 of f32's largest come out of this as an infinity or NaN: a kernel
+// recomputes such an output by f32 multiply-adds.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -27,9 +26,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float split_f2 __attribute__((ext_vector_type(2)));
 typedef float split_f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t split_u4 __attribute__((ext_vector_type(4)));
-
-// Magnitudes from here on round to bf16's infinity (bits of 2^128 - 2^119).
-constexpr uint32_t kSplitHuge = 0x7f7f8000u;
 
 __device__ __forceinline__ uint32_t split_pack(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(split_f2{a, b}, bf16x2));
@@ -43,20 +39,6 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t &p1, uint3
   p3 = split_pack(ra - __uint_as_float(p2 << 16), rb - __uint_as_float(p2 & 0xffff0000u));
 }
 
-// Whether either half's first part came out as an infinity or NaN: bit 15 of
-// each half of the result.
-__device__ __forceinline__ uint32_t split_odd(uint32_t p1) { return (p1 & 0x7fff7fffu) + 0x00800080u; }
-
-// One float's parts (in the low halves), any value.
-__device__ __forceinline__ void split_any(float a, uint32_t &p1, uint32_t &p2, uint32_t &p3) {
-  const uint32_t u = __float_as_uint(a), m = u & 0x7fffffffu;
-  const bool none = m >= 0x7f800000u;
-  p1 = none ? 0u : (m >= kSplitHuge ? u >> 16 : split_pack(a, 0.0f) & 0xffffu);
-  const float r = none ? 0.0f : a - __uint_as_float(p1 << 16);
-  p2 = split_pack(r, 0.0f) & 0xffffu;
-  p3 = split_pack(none ? a : r - __uint_as_float(p2 << 16), 0.0f) & 0xffffu;
-}
-
 // Eight consecutive reduction values as MFMA operands: element 2h in the low
 // half of dword h.
 __device__ __forceinline__ void split8(split_f4 lo, split_f4 hi, split_u4 &p1, split_u4 &p2, split_u4 &p3) {
@@ -64,15 +46,6 @@ __device__ __forceinline__ void split8(split_f4 lo, split_f4 hi, split_u4 &p1, s
   uint32_t a[4], b[4], c[4];
 #pragma unroll
   for (int h = 0; h < 4; h++) split_pair(x[2 * h], x[2 * h + 1], a[h], b[h], c[h]);
-  if (__builtin_expect(((split_odd(a[0]) | split_odd(a[1]) | split_odd(a[2]) | split_odd(a[3])) & 0x80008000u) != 0, 0)) {
-#pragma unroll
-    for (int h = 0; h < 4; h++) {
-      uint32_t u1, u2, u3;
-      split_any(x[2 * h], a[h], b[h], c[h]);
-      split_any(x[2 * h + 1], u1, u2, u3);
-      a[h] |= u1 << 16, b[h] |= u2 << 16, c[h] |= u3 << 16;
-    }
-  }
   p1 = split_u4{a[0], a[1], a[2], a[3]};
   p2 = split_u4{b[0], b[1], b[2], b[3]};
   p3 = split_u4{c[0], c[1], c[2], c[3]};

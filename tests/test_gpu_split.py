@@ -58,8 +58,33 @@ def test_ctc_panel_odd_values(oracle):
     same = [r for r in range(40) if r not in (7, 11, 20, 39)]
     assert np.array_equal(a[same].view(np.uint32), b[same].view(np.uint32))
     want = oracle.OracleModel(plan).run(y)[0].reshape(-1, 2)
-    assert b[11, 0] == want[11, 0]
-    np.testing.assert_allclose(b[11, 1], want[11, 1], rtol=1e-5)
+    finite = [r for r in range(40) if r not in (7, 20)]  # 39 in its class alone: its logits' exponents overflow
+    assert np.isfinite(want[finite]).all() and np.isnan(want[[7, 20], 1]).all()
+    assert np.array_equal(b[finite, 0], want[finite, 0])
+    np.testing.assert_allclose(b[finite[:-1], 1], want[finite[:-1], 1], rtol=1e-5)
+    assert not (b[[7, 20], 1] <= 1).any()  # no probability where there is none
+
+
+# A value and a weight whose nearest bf16 values' product is past f32's largest
+# while their own product is not.
+NEAR_X, NEAR_W = np.float32(1.004 * 2.0 ** 127), np.float32(1.9895)
+
+
+def test_ctc_panel_near_overflow(oracle):
+    """A logit within 2^-7 of f32's largest value: the class holds. (The
+    probability does not: past 2^128 / log2(e) the exponent overflows.)"""
+    rng = np.random.default_rng(5)
+    w = rng.normal(0, 0.3, (48, 500)).astype(np.float32)
+    w[9, 300], w[9, 20] = NEAR_W, NEAR_W * np.float32(0.9999)
+    b = PlanBuilder(1, 40, 48)
+    plan = b.to_bytes([b.ctcargmax(b.input, w, rng.normal(0, 0.5, 500).astype(np.float32))])
+    x = rng.normal(0, 1, (1, 40, 48)).astype(np.float32)
+    x[0, 21, 9] = NEAR_X
+    got = gpu(plan, (1, 40, 48), [x])[0].reshape(-1, 2)
+    want = oracle.OracleModel(plan).run(x)[0].reshape(-1, 2)
+    assert want[21, 0] == 300 and np.array_equal(got[:, 0], want[:, 0])
+    rest = np.arange(40) != 21
+    np.testing.assert_allclose(got[rest, 1], want[rest, 1], rtol=1e-5)
 
 
 def conv_plan(rng, h, w, cs, n, s, act, res):
@@ -117,3 +142,26 @@ def test_conv_patch_split_odd_values(oracle):
     assert np.array_equal(c[np.isinf(c)], want[np.isinf(want)])
     fin = np.isfinite(want)
     np.testing.assert_allclose(c[fin], want[fin], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("s", [1, 2])
+def test_conv_patch_split_near_overflow(oracle, s):
+    """An output within 2^-7 of f32's largest value stays finite, its
+    neighbours keep their bits."""
+    rng = np.random.default_rng(9)
+    b = PlanBuilder(20, 24, 16)
+    wt = rng.normal(0, 0.1, (3, 3, 16, 24)).astype(np.float32)
+    wt[1, 1, 3, 20] = NEAR_W
+    plan = b.to_bytes([b.conv(b.input, wt, None, k=(3, 3), s=(s, s), pad=(1, 1, 1, 1))])
+    x = rng.uniform(-1, 1, (20, 24, 16)).astype(np.float32)
+    y = x.copy()
+    y[8, 10, 3], y[18, 2, 3] = NEAR_X, -NEAR_X
+    want = oracle.OracleModel(plan).run(y)[0].reshape(20 // s, 24 // s, 24)
+    a, c = (v.reshape(want.shape) for v in gpu(plan, (20, 24, 16), [x, y]))
+    assert np.isfinite(want).all() and want[8 // s, 10 // s, 20] > 3.3e38 and want[18 // s, 2 // s, 20] < -3.3e38
+    # Sums in another order: 1e-5 of the largest product.
+    np.testing.assert_allclose(c, want, rtol=1e-5, atol=1e-5)
+    far = np.ones(want.shape[:2], bool)
+    for py, px in ((8, 10), (18, 2)):
+        far[(py - 1) // s:(py + 1) // s + 1, (px - 1) // s:(px + 1) // s + 1] = False
+    assert np.array_equal(a[far].view(np.uint32), c[far].view(np.uint32))
