@@ -970,12 +970,7 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
 #pragma unroll
   for (int j = 0; j < 2; j++) bcol[j] = bsrc[a.bias ? min(j * 16 + li, a.n - 1) : 0];
 
-  f32x4 hi[WR][2], lo[WR][2];
-#pragma unroll
-  for (int i = 0; i < WR; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++) hi[i][j] = lo[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+  SplitAcc acc[WR][2] = {};
 
   fetch(0);
   for (int cc = 0; cc < cpt; cc++) {
@@ -1011,8 +1006,8 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
             if (ky < 0 || ky > 2) continue;
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-              f32x4 &d = s == 5 ? hi[i][j] : lo[i][j];
-              d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[pa[s]], bv[ky][j][pb[s]], d, 0, 0, 0);
+              f32x4 &d = acc[i][j].s[kSplitScale[s]];
+              d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[kSplitA[s]], bv[ky][j][kSplitB[s]], d, 0, 0, 0);
             }
           }
       }
@@ -1020,14 +1015,15 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
   }
   // Outputs that came out as an infinity or NaN again by f32 multiply-adds.
   uint32_t odd = 0;
+  f32x4 sum[WR][2];
 #pragma unroll
   for (int i = 0; i < WR; i++)
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-      hi[i][j] = hi[i][j] + lo[i][j];
+      sum[i][j] = split_sum(acc[i][j]);
 #pragma unroll
       for (int r = 0; r < 4; r++)
-        if (!(fabsf(hi[i][j][r]) < __builtin_inff()) && ty0 + wave * WR + i < a.oh && tx0 + lg * 4 + r < a.ow && j * 16 + li < a.n)
+        if (!(fabsf(sum[i][j][r]) < __builtin_inff()) && ty0 + wave * WR + i < a.oh && tx0 + lg * 4 + r < a.ow && j * 16 + li < a.n)
           odd |= 1u << ((i * 2 + j) * 4 + r);
     }
   while (__builtin_expect(odd != 0, 0)) {
@@ -1036,7 +1032,7 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
     const float v = conv_f32<3, S>(a, ln, ty0 + wave * WR + (b >> 3), tx0 + lg * 4 + (b & 3), (b >> 2 & 1) * 16 + li);
 #pragma unroll
     for (int k = 0; k < WR * 8; k++)
-      if (k == b) hi[k >> 3][k >> 2 & 1][k & 3] = v;
+      if (k == b) sum[k >> 3][k >> 2 & 1][k & 3] = v;
   }
 #pragma unroll
   for (int i = 0; i < WR; i++) {
@@ -1047,7 +1043,7 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
       const int n = j * 16 + li, ox = tx0 + lg * 4;
       if (n >= a.n) continue;
       const long at = ((long)oy * a.ow + ox) * a.n + n;
-      f32x4 v = hi[i][j];
+      f32x4 v = sum[i][j];
       if (a.bias) v = v + bcol[j];
       v = act4(v, a.act);
       if (a.res) {
@@ -1123,10 +1119,12 @@ hipError_t launch_conv_patch_split_group(const ConvArgs *as, int n, hipStream_t 
 // `tie` bounds how far the two orders can put two columns' logits apart (u =
 // 2^-24, T = |bias| + sum |w_i x_i| <= bias_max + wsum_max * max |x_i|): the
 // CPU's bias + sum of ci products has n = ci + 1 roundings, each at most u T.
-// The panel's six products of split parts leave out at most 2 u T; its hi
-// accumulator rounds at most ci times, its lo one at most 5 ci times at sums
-// below 2^-6.9 T (0.042 ci u T), and joining them and the bias rounds twice:
-// (1.042 ci + 4) u T. So two columns' differences lie within (4.1 ci + 10)
+// The panel's six products of split parts leave out at most 2.01 u T; its
+// accumulator of the first parts' products rounds at most ci times at sums up
+// to 1.008 T, those of the smaller ones 2 ci times below 2^-6.9 T and 3 ci
+// below 2^-14 T (0.018 ci u T), and joining them and the bias rounds at most
+// 2.02 u T: from ci = 4 on at most (1.04 ci + 4) u T. So two columns'
+// differences lie within (4.1 ci + 10)
 // u T of each other. The test takes 8 n u T, which from ci = 4 on also covers
 // accumulations that round toward zero, so columns further below the maximum
 // on the GPU are below it in the CPU's order too.
@@ -1353,11 +1351,7 @@ __global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(
       ring_wait<0>();
       ring_barrier();
       if (h == 0 || t + 1 < t1) issue(2 * t + h + 1);
-      f32x4 hi[MT][2], lo[MT][2];
-#pragma unroll
-      for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) hi[i][j] = lo[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      SplitAcc part[MT][2] = {};
       const bf16x8 *bl = reinterpret_cast<const bf16x8 *>(bs) + h * STAGE + lane;
 #pragma unroll
       for (int q = 0; q < KG; q++) {
@@ -1366,24 +1360,16 @@ __global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(
         for (int j = 0; j < 2; j++)
 #pragma unroll
           for (int p = 0; p < 3; p++) bv[j][p] = bl[((j * KG + q) * 3 + p) * 64];
-        split_mma(av[q], bv, hi, lo);
+        split_mma(av[q], bv, part);
       }
 #pragma unroll
       for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][2 * h + j] = hi[i][j] + lo[i][j];
+        for (int j = 0; j < 2; j++) acc[i][2 * h + j] = split_sum(part[i][j]);
     }
-    const int k = t % kCtcRunTiles;
+    const int k = per_run == 1 ? 0 : t % kCtcRunTiles;
     auto store = [&](int row, float4 rec) {
-      const int m = tm * kCtcRows + row;
-      if (li != 0) return;
-      if (per_run == 1) {
-        if (m < M) reinterpret_cast<float4 *>(a.part)[(long)m * ntn + t] = rec;
-        return;
-      }
-      recs[row * kCtcRunTiles + k] = rec;
-      // The tiles' own maxima, after the runs' records.
-      if (m < M) a.part[(long)M * runs * 4 + (long)t * M + m] = rec.x;
+      if (li == 0) recs[row * kCtcRunTiles + k] = rec;
     };
     // Rows that hold an infinity or NaN (in 16 lanes alike).
     uint32_t odd = 0;
@@ -1407,15 +1393,25 @@ __global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(
       }
       store(row, ctc_row<4>(v, t * 64, lane));
     }
-    // A run's last tile: each row's records joined in column order, one
-    // record out. (The next tile's stores wait behind its first barrier.)
-    if (per_run > 1 && (k == kCtcRunTiles - 1 || t + 1 == t1)) {
+    // A record's last tile: each row's tiles joined in column order, one
+    // record out, and after all rows' records each tile's own maximum. (The
+    // next tile's stores wait behind its first barrier.)
+    if (per_run == 1 || k == kCtcRunTiles - 1 || t + 1 == t1) {
       __syncthreads();
       const int m = tm * kCtcRows + tid;
       if (tid < kCtcRows && m < M) {
-        float4 run_rec = recs[tid * kCtcRunTiles];
-        for (int q = 1; q <= k; q++) run_rec = ctc_join_partial(run_rec, recs[tid * kCtcRunTiles + q]);
-        reinterpret_cast<float4 *>(a.part)[(long)m * runs + t / kCtcRunTiles] = run_rec;
+        const float4 *tiles = recs + tid * kCtcRunTiles;
+        float4 rec = tiles[0];
+        if (per_run > 1) {
+          float *tmax = a.part + (long)M * runs * 4 + (long)(t - k) * M + m;
+          tmax[0] = rec.x;
+          for (int q = 1; q <= k; q++) {
+            const float4 next = tiles[q];
+            tmax[(long)q * M] = next.x;
+            rec = ctc_join_partial(rec, next);
+          }
+        }
+        reinterpret_cast<float4 *>(a.part)[(long)m * runs + t / per_run] = rec;
       }
     }
   }
@@ -1479,7 +1475,7 @@ hipError_t launch_ctc_direct_group(const CtcArgs *as, int n, hipStream_t s) {
   g.n = n, g.first[n] = (int)blocks;
   const int kg = ctc_direct_kpad(a0.ci) / 32;
   // Two weight stages, then the run's per-tile records.
-  const size_t shm = size_t(2) * 2 * kg * 3 * 64 * 16 + (r.per_run > 1 ? size_t(kCtcRows) * kCtcRunTiles * 16 : 0);
+  const size_t shm = size_t(2) * 2 * kg * 3 * 64 * 16 + size_t(kCtcRows) * kCtcRunTiles * 16;
   auto go = [&](auto one, auto many) {
     if (shm > 64 * 1024) {
       const void *kernel = n == 1 ? reinterpret_cast<const void *>(one) : reinterpret_cast<const void *>(many);

@@ -76,22 +76,24 @@ def test_merge_bound_covers_column_bounds():
 
 
 def parts(v):
-    """The three bf16 parts of a float32, whose sum it is."""
+    """The three bf16 parts of a float32 at scales 1, 2^-8 and 2^-16, whose
+    sum it is."""
     out = []
+    v = np.float32(v)
     for _ in range(3):
-        u = int(np.float32(v).view(np.uint32))
+        u = int(v.view(np.uint32))
         u = (u + 0x7FFF + ((u >> 16) & 1)) & 0xFFFF0000
         out.append(np.uint32(u).view(np.float32))
-        v = np.float32(v) - out[-1]
+        v = (v - out[-1]) * np.float32(256)
     assert v == 0
     return [float(p) for p in out]
 
 
 @pytest.mark.parametrize("ci", [4, 32, 120])
 def test_split_order_within_bound(ci):
-    """The panel kernel's order: six products of bf16 parts, the five small
-    ones in an accumulator of their own, every addition rounded (to nearest or
-    toward zero): within (1.042 ci + 4) u T, twice that toward zero."""
+    """The panel kernel's order: six products of bf16 parts, an accumulator
+    for each of their three scales, every addition rounded (to nearest or
+    toward zero): within (1.04 ci + 4) u T, twice the first toward zero."""
     rng = np.random.default_rng(ci)
     for trial in range(20):
         x = rng.normal(0, 3, ci).astype(np.float32)
@@ -107,11 +109,20 @@ def test_split_order_within_bound(ci):
                 if toward_zero and abs(float(s)) > abs(v + t):
                     s = np.nextafter(s, np.float32(0))
                 return float(s)
-            hi = lo = 0.0
+            acc = [0.0, 0.0, 0.0]
             for a, b in zip(w, x):
                 p, q = parts(a), parts(b)
-                for i, j in ((2, 0), (0, 2), (1, 1), (1, 0), (0, 1)):
-                    lo = add(lo, p[i] * q[j])
-                hi = add(hi, p[0] * q[0])
-            got = float(np.float32(np.float32(hi + lo) + bias))
-            assert abs(got - exact) <= (1.042 * ci * (1 + toward_zero) + 4) * U * T
+                for i, j in ((2, 0), (0, 2), (1, 1), (1, 0), (0, 1), (0, 0)):
+                    acc[i + j] = add(acc[i + j], p[i] * q[j])
+            low = float(np.float32(acc[1] + acc[2] / 256))
+            got = float(np.float32(np.float32(acc[0] + low / 256) + bias))
+            assert abs(got - exact) <= (1.04 * ci * (1 + toward_zero) + 4) * U * T
+
+
+@pytest.mark.parametrize("e", [-149, -140, -134, -126, -120, -110, -60, 0, 120])
+def test_split_parts_exact(e):
+    """The parts are the value, down to f32's smallest."""
+    rng = np.random.default_rng(e + 200)
+    for v in np.float32(rng.uniform(1, 2, 200) * 2.0 ** e) * rng.choice([-1, 1], 200).astype(np.float32):
+        p = parts(v)
+        assert p[0] + p[1] / 256 + p[2] / 65536 == float(v)

@@ -65,6 +65,40 @@ def test_ctc_panel_odd_values(oracle):
     assert not (b[[7, 20], 1] <= 1).any()  # no probability where there is none
 
 
+# Inputs, and then weights, so small that their last bits lie below bf16's
+# smallest step: normal ones, the last normal ones, subnormal inputs.
+TINY = [(2.0 ** -118, 2.0 ** 117), (2.0 ** -127, 2.0 ** 125), (2.0 ** -136, 2.0 ** 125), (2.0 ** 100, 2.0 ** -122)]
+
+
+@pytest.mark.parametrize("sx,sw", TINY)
+def test_ctc_panel_tiny_values(oracle, sx, sw):
+    rng = np.random.default_rng(6)
+    w = (rng.normal(0, 0.3, (48, 500)) * sw).astype(np.float32)
+    b = PlanBuilder(1, 40, 48)
+    plan = b.to_bytes([b.ctcargmax(b.input, w, rng.normal(0, 0.1 * sx * sw, 500).astype(np.float32))])
+    x = (rng.normal(0, 1, (1, 40, 48)) * sx).astype(np.float32)
+    got = gpu(plan, (1, 40, 48), [x])[0].reshape(-1, 2)
+    want = oracle.OracleModel(plan).run(x)[0].reshape(-1, 2)
+    assert np.array_equal(got[:, 0], want[:, 0])
+    np.testing.assert_allclose(got[:, 1], want[:, 1], rtol=1e-5)
+
+
+@pytest.mark.parametrize("sx,sw", TINY)
+@pytest.mark.parametrize("s", [1, 2])
+def test_conv_patch_split_tiny_values(oracle, s, sx, sw):
+    rng = np.random.default_rng(7)
+    b = PlanBuilder(20, 24, 40)
+    wt = (rng.normal(0, 0.1, (3, 3, 40, 24)) * sw).astype(np.float32)
+    plan = b.to_bytes([b.conv(b.input, wt, None, k=(3, 3), s=(s, s), pad=(1, 1, 1, 1))])
+    x = (rng.uniform(-1, 1, (20, 24, 40)) * sx).astype(np.float32)
+    want = oracle.OracleModel(plan).run(x)[0].reshape(-1).astype(np.float64)
+    got = gpu(plan, (20, 24, 40), [x])[0]
+    # The layer tests' tolerance, in the outputs' scale, and half its own step
+    # (2^-149) of each subnormal input, twice.
+    step = 2.0 ** -149 * np.abs(wt.astype(np.float64)).sum(axis=(0, 1, 2)).max()
+    assert (np.abs(got - want) <= 1e-5 * np.abs(want) + 1e-5 * sx * sw + step).all()
+
+
 # A value and a weight whose nearest bf16 values' product is past f32's largest
 # while their own product is not.
 NEAR_X, NEAR_W = np.float32(1.004 * 2.0 ** 127), np.float32(1.9895)
