@@ -33,7 +33,7 @@ if int(os.environ.get("GPU_MAX_HW_QUEUES", "4")) < 8:
     os.environ["GPU_MAX_HW_QUEUES"] = "8"
 PEAK_HBM_GBS = 8000.0
 PEAK_FP32_MFMA_TFLOPS = 157.3
-GEMM_LAUNCHES = {"pointwise_gemm", "conv_gemm", "conv_patch", "convt_gemm", "ctc_gemm"}
+GEMM_LAUNCHES = {"pointwise_gemm", "conv_gemm", "conv_patch", "conv_patch_split", "convt_gemm", "ctc_gemm"}
 # Launches whose products run as FP32 fused multiply-adds on the vector ALUs
 # (in the CPU engine's order), scored against the unpacked FP32 vector rate:
 # 256 CUs x 4 SIMDs x 16 lanes x 2 flops x 2.4 GHz (packed FP32 is not used).
@@ -43,8 +43,8 @@ VALU_LAUNCHES = {"stem_block"}
 # scaled by a plain copy kernel's counters (x2.0 / x1.0), for the launches
 # the bench reports a roofline of: (kernel, plan operations) -> (read, write)
 # KiB and the profile summary the numbers come from.
-MEASURED_TRAFFIC = {("conv_patch", (65, 71, 77, 83)): (31904, 7172, "profiles/hbm_counters_detector_recognizer.md"),
-                    ("conv_patch", (94,)): (9420, 5400, "profiles/hbm_counters_detector_recognizer.md")}
+MEASURED_TRAFFIC = {("conv_patch_split", (65, 71, 77, 83)): (31904, 7172, "profiles/hbm_counters_detector_recognizer.md"),
+                    ("conv_patch_split", (94,)): (9420, 5400, "profiles/hbm_counters_detector_recognizer.md")}
 
 
 def package():

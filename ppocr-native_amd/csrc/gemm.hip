@@ -864,18 +864,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
 // first loads and the three blocks in turn. Measured against f32 MFMA
 // (conv_patch): 96 -> 24 over four upsampled sources at 496 x 384 98.9 -> 58.6
 // us, the neck's four maps 129.6 -> 79.3; at 240 x 184 28.3 -> 20.8 and 34.3
-// -> 22.0; at 56 x 80 16.3 -> 11.6 and 16.4 -> 13.1, 48 -> 32 at stride 2 23.1
-// -> 11.1.
+// -> 22.0; at 56 x 80 16.3 -> 11.6 and 16.4 -> 13.1.
 constexpr int kSplitTaps = 9;
 // Tiles of 16 rows (eight waves of two) when that leaves most CUs one, of 8
 // (eight waves of one) when half, else of 4 (four waves of one).
 constexpr long kSplitTiles16 = 160, kSplitTiles8 = 128;
 constexpr int kSplitWeights = kSplitTaps * 2 * 192;  // 16-byte groups of a channel block's weights
 
-template <int NW, int WR, int S>
+template <int NW, int WR>
 struct SplitTile {
   static constexpr int T = 64 * NW, TH = NW * WR;             // threads, output rows
-  static constexpr int PR = (TH - 1) * S + 3, PC = 15 * S + 3;  // the patch
+  static constexpr int PR = TH + 2, PC = 18;                  // the patch
   static constexpr int NPX = PR * PC;
   static constexpr int UNITS = (NPX * 4 + T - 1) / T;         // (pixel, 8 channels) a thread stages
   static constexpr int WUNITS = (kSplitWeights + T - 1) / T;
@@ -884,24 +883,24 @@ struct SplitTile {
 
 // Output (oy, ox) of column n of lane ln by f32 multiply-adds, the taps in
 // row-major order and each one's channels in order; `wt` in the plan's order.
-template <int K, int S>
 __device__ __forceinline__ float conv_f32(const ConvArgs &a, int ln, int oy, int ox, int n) {
   float sum = 0.0f;
-  for (int tap = 0; tap < K * K; tap++) {
-    const int iy = oy * S - a.pt + tap / K, ix = ox * S - a.pl + tap % K;
+  for (int tap = 0; tap < kSplitTaps; tap++) {
+    const int iy = oy - a.pt + tap / 3, ix = ox - a.pl + tap % 3;
     if (iy < 0 || iy >= a.ih || ix < 0 || ix >= a.iw) continue;
     for (int c = 0; c < a.ctot; c++) {
       const ConvSrc src = pick_src(a, c);
-      const float x = src.p[(long)ln * src.lane_stride + ((long)(iy >> src.shift) * (a.iw >> src.shift) + (ix >> src.shift)) * src.c + c - src.coff];
+      const long pix = (long)(iy >> src.shift) * (a.iw >> src.shift) + (ix >> src.shift);
+      const float x = src.p[(long)ln * src.lane_stride + pix * src.c + c - src.coff];
       sum = fmaf(x, a.wt[((long)tap * a.ctot + c) * a.n + n], sum);
     }
   }
   return sum;
 }
 
-template <int NW, int WR, int S, int GN>
+template <int NW, int WR, int GN>
 __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> grp) {
-  typedef SplitTile<NW, WR, S> K;
+  typedef SplitTile<NW, WR> K;
   constexpr int T = K::T, PC = K::PC, NPX = K::NPX, TW = 16;
   const int bid = xcd_tile((int)blockIdx.x, (int)gridDim.x);
   int prob = 0;
@@ -919,12 +918,8 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
   const int ty0 = (t % tiles_y) * K::TH, ln = t / tiles_y;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lg = lane >> 4;
-  const int iy0 = ty0 * S - a.pt, ix0 = tx0 * S - a.pl;
+  const int iy0 = ty0 - a.pt, ix0 = tx0 - a.pl;
   const int cpt = (a.ctot + 31) / 32;
-  // A stride-2 patch keeps each row's even columns before its odd ones: the
-  // pixels a tap reads lie side by side.
-  auto place = [](int col) { return S == 1 ? col : (col & 1) * ((PC + 1) / 2) + (col >> 1); };
-
   split_f4 rp[K::UNITS][2];
   split_u4 rw[K::WUNITS];
   const int g = tid & 3, p0 = tid >> 2;
@@ -953,12 +948,12 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
   auto store = [&]() {
 #pragma unroll
     for (int k = 0; k < K::UNITS; k++) {
-      const int q = p0 + k * (T / 4), py = q / PC, px = q - py * PC;
+      const int q = p0 + k * (T / 4);
       if (q < NPX) {
         split_u4 v[3];
         split8(rp[k][0], rp[k][1], v[0], v[1], v[2]);
 #pragma unroll
-        for (int p = 0; p < 3; p++) P[(p * NPX + py * PC + place(px)) * 4 + g] = v[p];
+        for (int p = 0; p < 3; p++) P[(p * NPX + q) * 4 + g] = v[p];
       }
     }
 #pragma unroll
@@ -993,8 +988,8 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
           for (int p = 0; p < 3; p++)
             bv[ky][j][p] = __builtin_bit_cast(bf16x8, B[(((ky * 3 + kx) * 2 + j) * 3 + p) * 64 + lane]);
 #pragma unroll
-      for (int r = 0; r < (WR - 1) * S + 3; r++) {
-        const int pix = (wave * WR * S + r) * PC + place(kx) + li;
+      for (int r = 0; r < WR + 2; r++) {
+        const int pix = (wave * WR + r) * PC + kx + li;
         bf16x8 av[3];
 #pragma unroll
         for (int p = 0; p < 3; p++) av[p] = __builtin_bit_cast(bf16x8, P[(p * NPX + pix) * 4 + lg]);
@@ -1002,7 +997,7 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
         for (int s = 0; s < 6; s++)
 #pragma unroll
           for (int i = 0; i < WR; i++) {
-            const int ky = r - i * S;
+            const int ky = r - i;
             if (ky < 0 || ky > 2) continue;
 #pragma unroll
             for (int j = 0; j < 2; j++) {
@@ -1029,7 +1024,7 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
   while (__builtin_expect(odd != 0, 0)) {
     const int b = __builtin_ctz(odd);
     odd &= odd - 1;
-    const float v = conv_f32<3, S>(a, ln, ty0 + wave * WR + (b >> 3), tx0 + lg * 4 + (b & 3), (b >> 2 & 1) * 16 + li);
+    const float v = conv_f32(a, ln, ty0 + wave * WR + (b >> 3), tx0 + lg * 4 + (b & 3), (b >> 2 & 1) * 16 + li);
 #pragma unroll
     for (int k = 0; k < WR * 8; k++)
       if (k == b) sum[k >> 3][k >> 2 & 1][k & 3] = v;
@@ -1060,15 +1055,23 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
   }
 }
 
-bool patch_split_shape(int kh, int kw, int sh, int sw, int n) {
-  return kh == 3 && kw == 3 && sh == sw && (sh == 1 || sh == 2) && n > 16 && n <= 32;
+// Stride 1 alone: a stride-2 patch is four times its outputs, one workgroup of
+// it and the weights fills a CU's LDS, and its staging costs what the products
+// save. It won on one small image (48 -> 32 at 56 x 80: 13.3 -> 10.8 us) and
+// lost where there are more tiles than CUs (two such images even, sixteen 37.9
+// -> 50.5 us; 8 channels 19.5 -> 30.2), and the choice cannot follow the number
+// of lanes, whose bits must not depend on each other. From 16 channels on, so
+// that padding them to 32 at most doubles the products: 8 -> 17 at 240 x 184
+// took 8.8 us in f32 and 9.5 split, 16 -> 17 9.3 and 9.2.
+bool patch_split_shape(int kh, int kw, int sh, int sw, int ctot, int n) {
+  return kh == 3 && kw == 3 && sh == 1 && sw == 1 && ctot >= 16 && n > 16 && n <= 32;
 }
 
 size_t patch_split_floats(int ctot) { return size_t(kSplitTaps) * split_pack_floats((ctot + 31) / 32 * 32, 32); }
 
-template <int NW, int WR, int S>
+template <int NW, int WR>
 static hipError_t go_patch_split(const ConvArgs *as, int n, hipStream_t s) {
-  typedef SplitTile<NW, WR, S> K;
+  typedef SplitTile<NW, WR> K;
   Group<ConvArgs> g{};
   long blocks = 0;
   for (int p = 0; p < n; p++) {
@@ -1085,8 +1088,8 @@ static hipError_t go_patch_split(const ConvArgs *as, int n, hipStream_t s) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(K::T), K::LDS, s, gr);
     return hipGetLastError();
   };
-  if (n == 1) return go(conv_patch_split<NW, WR, S, 1>, group_of<1>(g));
-  return go(conv_patch_split<NW, WR, S, kGroupStep>, group_of<kGroupStep>(g));
+  if (n == 1) return go(conv_patch_split<NW, WR, 1>, group_of<1>(g));
+  return go(conv_patch_split<NW, WR, kGroupStep>, group_of<kGroupStep>(g));
 }
 
 hipError_t launch_conv_patch_split_group(const ConvArgs *as, int n, hipStream_t s) {
@@ -1094,7 +1097,7 @@ hipError_t launch_conv_patch_split_group(const ConvArgs *as, int n, hipStream_t 
   long tiles16 = 0, tiles8 = 0;
   for (int p = 0; p < n; p++) {
     const ConvArgs &a = as[p];
-    if (!patch_split_shape(a.kh, a.kw, a.sh, a.sw, a.n) || a.sh != as[0].sh || a.mode != GEMM_STORE || a.gate || a.pw_w ||
+    if (!patch_split_shape(a.kh, a.kw, a.sh, a.sw, a.ctot, a.n) || a.mode != GEMM_STORE || a.gate || a.pw_w ||
         !a.split_wt || a.nsrc < 1 || a.nsrc > 4)
       return hipErrorInvalidValue;
     for (int k = 0; k < a.nsrc; k++)
@@ -1102,10 +1105,9 @@ hipError_t launch_conv_patch_split_group(const ConvArgs *as, int n, hipStream_t 
     tiles16 += (long)a.lanes * ((a.ow + 15) / 16) * ((a.oh + 15) / 16);
     tiles8 += (long)a.lanes * ((a.ow + 15) / 16) * ((a.oh + 7) / 8);
   }
-  if (as[0].sh == 2) return go_patch_split<4, 1, 2>(as, n, s);
-  if (tiles16 >= kSplitTiles16) return go_patch_split<8, 2, 1>(as, n, s);
-  if (tiles8 >= kSplitTiles8) return go_patch_split<8, 1, 1>(as, n, s);
-  return go_patch_split<4, 1, 1>(as, n, s);
+  if (tiles16 >= kSplitTiles16) return go_patch_split<8, 2>(as, n, s);
+  if (tiles8 >= kSplitTiles8) return go_patch_split<8, 1>(as, n, s);
+  return go_patch_split<4, 1>(as, n, s);
 }
 
 // One wave per row: join the row's tile partials, then y = (best, 1 / sum).

@@ -956,7 +956,7 @@ bool Model::pack(std::string &err) {
         if (pb) s.patch = true, bk = pb;
         bool eights = s.gate < 0;
         for (auto &x : srcs) eights = eights && x.c % 8 == 0;
-        if (pb && eights && patch_split_shape(int(op.kh), int(op.kw), int(op.sh), int(op.sw), N)) {
+        if (pb && eights && patch_split_shape(int(op.kh), int(op.kw), int(op.sh), int(op.sw), ctot, N)) {
           // The taps' bf16 parts, one packing after the other.
           s.patch_split = true;
           const int kp = (ctot + 31) / 32 * 32;
@@ -1372,9 +1372,9 @@ void Model::build_launches(Batch &b) {
           if (s.patch_split) {
             a.split_wt = dsplit + s.split_w;
             a.wt = W + op.w0, a.wt_k = 0;
-            b.launches.push_back({"conv_patch", s.op, [a](hipStream_t st) { return launch_conv_patch_split_group(&a, 1, st); }});
+            b.launches.push_back({"conv_patch_split", s.op, [a](hipStream_t st) { return launch_conv_patch_split_group(&a, 1, st); }});
             Launch &l = b.launches.back();
-            l.gk = GK_PATCH, l.gkey = -a.sh, l.conv = a, l.bk = bk, l.bn = bn;
+            l.gk = GK_PATCH, l.gkey = -1, l.conv = a, l.bk = bk, l.bn = bn;
             break;
           }
           b.launches.push_back({"conv_patch", s.op, [a, wr, bk, bn](hipStream_t st) {

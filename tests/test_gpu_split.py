@@ -140,9 +140,9 @@ def conv_plan(rng, h, w, cs, n, s, act, res):
 
 # Tiles of 4, 8 and 16 rows (few tiles, more, enough for 160 of 16 rows over
 # the lanes), edges that cut them, channels within and past a block of 32, 17
-# to 32 outputs, both strides, two sources, a folded Add.
+# to 32 outputs, two sources, a folded Add; 8 channels and stride 2 run in f32.
 @pytest.mark.parametrize("h,w,cs,n,s,act,res", [
-    (1, 1, (8,), 17, 1, "none", False), (5, 17, (40,), 24, 1, "hardswish", True), (33, 31, (96,), 32, 1, "relu", False),
+    (1, 1, (8,), 17, 1, "none", False), (1, 1, (16,), 17, 1, "none", False), (5, 17, (40,), 24, 1, "hardswish", True), (33, 31, (96,), 32, 1, "relu", False),
     (66, 130, (32, 24), 24, 1, "relu", True), (150, 220, (24, 72), 20, 1, "none", False),
     (7, 9, (48,), 32, 2, "hardswish", False), (64, 66, (16, 16), 25, 2, "relu", True)])
 def test_conv_patch_split(oracle, h, w, cs, n, s, act, res):
@@ -199,3 +199,16 @@ def test_conv_patch_split_near_overflow(oracle, s):
     for py, px in ((8, 10), (18, 2)):
         far[(py - 1) // s:(py + 1) // s + 1, (px - 1) // s:(px + 1) // s + 1] = False
     assert np.array_equal(a[far].view(np.uint32), c[far].view(np.uint32))
+
+
+@pytest.mark.parametrize("c,n,s,split", [(8, 24, 1, False), (16, 16, 1, False), (16, 17, 1, True), (24, 32, 1, True),
+                                         (24, 33, 1, False), (48, 32, 2, False), (96, 24, 1, True)])
+def test_conv_patch_split_rule(c, n, s, split):
+    """Which layers run split: not stride 2, which is slower on more tiles than
+    CUs, nor channels that padding to 32 more than doubles."""
+    b = PlanBuilder(20, 24, c)
+    wt = np.zeros((3, 3, c, n), np.float32)
+    g = GpuModel.load(b.to_bytes([b.conv(b.input, wt, None, k=(3, 3), s=(s, s), pad=(1, 1, 1, 1))]))
+    names = [name for name, _ in g.launches()]
+    g.close()
+    assert names == ["conv_patch_split" if split else "conv_patch"]
