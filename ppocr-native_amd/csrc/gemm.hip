@@ -866,9 +866,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
 // us, the neck's four maps 129.6 -> 79.3; at 240 x 184 28.3 -> 20.8 and 34.3
 // -> 22.0; at 56 x 80 16.3 -> 11.6 and 16.4 -> 13.1.
 constexpr int kSplitTaps = 9;
-// Tiles of 16 rows (eight waves of two) when that leaves most CUs one, of 8
-// (eight waves of one) when half, else of 4 (four waves of one).
-constexpr long kSplitTiles16 = 160, kSplitTiles8 = 128;
+// Tiles of 16 rows (eight waves of two), 8 (eight waves of one) or 4 (four
+// waves of one): those whose rounds of workgroups over the 256 CUs take least.
+// A round of 16-row tiles is 20 units long, of 8-row ones 13 (a CU holds one
+// of either); a CU holds two 4-row ones, 14 units together and 10 alone. On
+// 305 maps of 2 to 460 rows, 16 to 96 channels and 1 to 8 images that is
+// within 0.5% of the fastest of the three, and at least 5% faster than f32.
+// (Chosen by the number of 16-row tiles alone, maps of a few rows took tiles
+// mostly past their edge: 128 -> 20 over eight of 4 x 352 23.4 us, now 14.5;
+// 32 -> 17 over 143 x 254 12.3, now 9.5.)
+constexpr long kSplitRound16 = 20, kSplitRound8 = 13, kSplitRound4 = 10, kSplitRound4x2 = 14;
 constexpr int kSplitWeights = kSplitTaps * 2 * 192;  // 16-byte groups of a channel block's weights
 
 template <int NW, int WR>
@@ -1094,7 +1101,7 @@ static hipError_t go_patch_split(const ConvArgs *as, int n, hipStream_t s) {
 
 hipError_t launch_conv_patch_split_group(const ConvArgs *as, int n, hipStream_t s) {
   if (n < 1 || n > kGroupStep) return hipErrorInvalidValue;
-  long tiles16 = 0, tiles8 = 0;
+  long tiles16 = 0, tiles8 = 0, tiles4 = 0;
   for (int p = 0; p < n; p++) {
     const ConvArgs &a = as[p];
     if (!patch_split_shape(a.kh, a.kw, a.sh, a.sw, a.ctot, a.n) || a.mode != GEMM_STORE || a.gate || a.pw_w ||
@@ -1102,11 +1109,14 @@ hipError_t launch_conv_patch_split_group(const ConvArgs *as, int n, hipStream_t 
       return hipErrorInvalidValue;
     for (int k = 0; k < a.nsrc; k++)
       if (a.src[k].c % 8 || a.src[k].coff % 8 || a.src[k].lane_stride % 4) return hipErrorInvalidValue;
-    tiles16 += (long)a.lanes * ((a.ow + 15) / 16) * ((a.oh + 15) / 16);
-    tiles8 += (long)a.lanes * ((a.ow + 15) / 16) * ((a.oh + 7) / 8);
+    const long across = (long)a.lanes * ((a.ow + 15) / 16);
+    tiles16 += across * ((a.oh + 15) / 16), tiles8 += across * ((a.oh + 7) / 8), tiles4 += across * ((a.oh + 3) / 4);
   }
-  if (tiles16 >= kSplitTiles16) return go_patch_split<8, 2>(as, n, s);
-  if (tiles8 >= kSplitTiles8) return go_patch_split<8, 1>(as, n, s);
+  auto rounds = [](long tiles) { return (tiles + 255) / 256; };
+  const long t16 = rounds(tiles16) * kSplitRound16, t8 = rounds(tiles8) * kSplitRound8;
+  const long t4 = rounds(tiles4) / 2 * kSplitRound4x2 + rounds(tiles4) % 2 * kSplitRound4;
+  if (t16 <= t8 && t16 <= t4) return go_patch_split<8, 2>(as, n, s);
+  if (t8 <= t4) return go_patch_split<8, 1>(as, n, s);
   return go_patch_split<4, 1>(as, n, s);
 }
 

@@ -212,3 +212,21 @@ def test_conv_patch_split_rule(c, n, s, split):
     names = [name for name, _ in g.launches()]
     g.close()
     assert names == ["conv_patch_split" if split else "conv_patch"]
+
+
+@pytest.mark.parametrize("h,w,lanes", [(1, 352, 8), (4, 352, 8), (8, 300, 5), (9, 150, 16), (51, 130, 8), (143, 254, 1)])
+def test_conv_patch_split_tiles(oracle, h, w, lanes):
+    """Maps of few rows and of rows either side of a tile's, with as many tiles
+    as take one round of the CUs and more: a lane's bits are those of the lane
+    alone, whichever tiles each takes."""
+    rng = np.random.default_rng(h)
+    b = PlanBuilder(h, w, 32)
+    wt = rng.normal(0, 0.06, (3, 3, 32, 24)).astype(np.float32)
+    plan = b.to_bytes([b.conv(b.input, wt, None, k=(3, 3), pad=(1, 1, 1, 1), fused="relu")])
+    xs = [rng.uniform(-1, 1, (h, w, 32)).astype(np.float32) for _ in range(lanes)]
+    got = gpu(plan, (h, w, 32), xs)
+    m = oracle.OracleModel(plan)
+    for i in (0, lanes - 1):
+        assert np.array_equal(gpu(plan, (h, w, 32), [xs[i]])[0].view(np.uint32), got[i].view(np.uint32))
+        want = m.run(xs[i])[0].reshape(-1).astype(np.float64)
+        assert (np.abs(got[i] - want) <= 1e-5 * np.abs(want) + 1e-5).all()
