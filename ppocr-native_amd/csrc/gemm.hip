@@ -1155,6 +1155,7 @@ __global__ __launch_bounds__(256) void ctc_merge(Group<CtcArgs, GN> grp, int nti
   if (row >= rows) return;
   CtcState st{-__builtin_inff(), 0.0f, __builtin_inff()};
   float m2 = -__builtin_inff();
+  bool odd = false;  // a tile holds an infinity or NaN, which leaves its sum NaN
   for (int t = lane; t * run < ntiles; t += 64) {
     // A run's records, joined in column order as a workgroup that walks the
     // whole run joins them.
@@ -1165,6 +1166,7 @@ __global__ __launch_bounds__(256) void ctc_merge(Group<CtcArgs, GN> grp, int nti
     top2(st.m, m2, p.x, p.w, n1, n2);
     m2 = n2;
     st = ctc_join(st, CtcState{p.x, p.y, p.z});
+    odd = odd || p.y != p.y;
   }
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
@@ -1186,6 +1188,32 @@ __global__ __launch_bounds__(256) void ctc_merge(Group<CtcArgs, GN> grp, int nti
   for (int i = lane; i < ex.ci; i += 64) xm = fmaxf(xm, fabsf(x[i]));
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) xm = fmaxf(xm, __shfl_xor(xm, d, 64));
+  if (ex.split_wt && __ballot(odd) != 0) {
+    // The split products may hold one where f32 has none (split.hpp): the
+    // row's logits again by f32 multiply-adds in the CPU's order.
+    constexpr float L = 1.44269504088896341f;  // log2(e)
+    auto logit = [&](int n) {
+      float v = ex.bias[n];
+      for (int i = 0; i < ex.ci; i++) v = fmaf(ex.wt[(long)n * ex.wt_k + i], x[i], v);
+      return v;
+    };
+    float m = -__builtin_inff(), b = __builtin_inff(), sum = 0.0f;
+    for (int n = lane; n < ex.vocab; n += 64) {
+      const float v = logit(n);
+      if (v > m) m = v, b = (float)n;
+    }
+    for (int d = 1; d < 64; d <<= 1) {
+      const float om = __shfl_xor(m, d, 64), ob = __shfl_xor(b, d, 64);
+      if (om > m || (om == m && ob < b)) m = om, b = ob;
+    }
+    for (int n = lane; n < ex.vocab; n += 64) sum += __builtin_amdgcn_exp2f(fmaf(logit(n), L, -m * L));
+    for (int d = 1; d < 64; d <<= 1) sum += __shfl_xor(sum, d, 64);
+    if (lane == 0) {
+      float *yp = ex.y + (long)ln * ex.y_lane_stride + 2L * tr;
+      yp[0] = b, yp[1] = 1.0f / sum;
+    }
+    return;
+  }
   const float terms = ex.bias_max + ex.wsum_max * xm;
   const float tie = fmaxf(8.0f * float(ex.ci + 1) * kCtcUnit * terms * 1.0001f, 1e-30f);
   if (ex.wt && st.m - m2 <= tie) {
@@ -1363,48 +1391,26 @@ __global__ __launch_bounds__(64 * kCtcWaves) __attribute__((amdgpu_waves_per_eu(
       ring_wait<0>();
       ring_barrier();
       if (h == 0 || t + 1 < t1) issue(2 * t + h + 1);
-      SplitAcc part[MT][2] = {};
       const bf16x8 *bl = reinterpret_cast<const bf16x8 *>(bs) + h * STAGE + lane;
+      // A block of 16 columns after the other: three accumulators a row block.
 #pragma unroll
-      for (int q = 0; q < KG; q++) {
-        bf16x8 bv[2][3];
+      for (int j = 0; j < 2; j++) {
+        SplitAcc part[MT][1] = {};
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int q = 0; q < KG; q++) {
+          bf16x8 bv[1][3];
 #pragma unroll
-          for (int p = 0; p < 3; p++) bv[j][p] = bl[((j * KG + q) * 3 + p) * 64];
-        split_mma(av[q], bv, part);
+          for (int p = 0; p < 3; p++) bv[0][p] = bl[((j * KG + q) * 3 + p) * 64];
+          split_mma(av[q], bv, part);
+        }
+#pragma unroll
+        for (int i = 0; i < MT; i++) acc[i][2 * h + j] = split_sum(part[i][0]);
       }
-#pragma unroll
-      for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][2 * h + j] = split_sum(part[i][j]);
     }
     const int k = per_run == 1 ? 0 : t % kCtcRunTiles;
-    auto store = [&](int row, float4 rec) {
-      if (li == 0) recs[row * kCtcRunTiles + k] = rec;
-    };
-    // Rows that hold an infinity or NaN (in 16 lanes alike).
-    uint32_t odd = 0;
     ctc_tile_rows<MT, 4>(acc, t * 64, a.bias, vocab, lane, [&](int i, int r, float4 rec) {
-      store(wave * 16 * MT + i * 16 + lg * 4 + r, rec);
-      if (!(fabsf(rec.x) < __builtin_inff()) || rec.y != rec.y) odd |= 1u << (i * 4 + r);
+      if (li == 0) recs[(wave * 16 * MT + i * 16 + lg * 4 + r) * kCtcRunTiles + k] = rec;
     });
-    // Those again by f32 multiply-adds (split.hpp).
-    while (__builtin_expect(odd != 0, 0)) {
-      const int b = __builtin_ctz(odd), row = wave * 16 * MT + (b >> 2) * 16 + lg * 4 + (b & 3);
-      odd &= odd - 1;
-      const int m = min(tm * kCtcRows + row, M - 1), ln = m / a.rows_per_lane;
-      const float *xr = a.x + ln * a.x_lane_stride + (long)(m - ln * a.rows_per_lane) * a.ci;
-      float v[4];
-      for (int j = 0; j < 4; j++) {
-        const int n = t * 64 + j * 16 + li, nc = min(n, vocab - 1);
-        const float *wr = a.wt + (long)nc * a.wt_k;
-        float sum = 0.0f;
-        for (int c = 0; c < a.ci; c++) sum = fmaf(xr[c], wr[c], sum);
-        v[j] = n < vocab ? sum + a.bias[nc] : -__builtin_inff();
-      }
-      store(row, ctc_row<4>(v, t * 64, lane));
-    }
     // A record's last tile: each row's tiles joined in column order, one
     // record out, and after all rows' records each tile's own maximum. (The
     // next tile's stores wait behind its first barrier.)

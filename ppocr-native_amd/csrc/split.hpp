@@ -23,8 +23,9 @@
 // other factor at most.)
 //
 // Infinities, NaN, values that round past bf16's largest, and sums within
-// 2^-7 of f32's largest come out of this as an infinity or NaN: a kernel
-// recomputes such an output by f32 multiply-adds.
+// 2^-7 of f32's largest come out of this as an infinity or NaN: such an output
+// is recomputed by f32 multiply-adds (conv_f32; the CTC head's rows, whose sum
+// of exponentials it leaves NaN, by ctc_merge).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
