@@ -854,8 +854,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
 // a lane; for each block of 32 input channels (one MFMA step deep) the
 // workgroup stages the patch, split into its three parts (four threads a
 // pixel, eight channels each), and every tap's weights in LDS, the next
-// block's in flight to registers meanwhile. Every operand read is 1 KB of
-// consecutive LDS. A wave takes the window column by column, that column's
+// block's in flight to registers meanwhile. At stride 2, whose patch is four
+// times the outputs, LDS holds the weights of one window column at a time (75
+// KB in all, two workgroups a CU; with every tap's, one, it was slower than f32
+// on more tiles than CUs: 48 -> 32 over sixteen maps of 127 x 127 152.7 us,
+// now 91.7, f32 104). Every operand read is 1 KB of consecutive LDS. A wave takes the window column by column, that column's
 // weights in registers, and reads each input row once for all its output
 // rows. Reduction order: channel block, window column, input row.
 //
@@ -864,9 +867,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
 // first loads and the three blocks in turn. Measured against f32 MFMA
 // (conv_patch): 96 -> 24 over four upsampled sources at 496 x 384 98.9 -> 58.6
 // us, the neck's four maps 129.6 -> 79.3; at 240 x 184 28.3 -> 20.8 and 34.3
-// -> 22.0; at 56 x 80 16.3 -> 11.6 and 16.4 -> 13.1.
+// -> 22.0; at 56 x 80 16.3 -> 11.6 and 16.4 -> 13.1. Stride 2, 48 -> 32 to 56 x 80 13.4 -> 10.9, to
+// sixteen of them 37.5 -> 35.3.
 constexpr int kSplitTaps = 9;
-// Tiles of 16 rows (eight waves of two), 8 (eight waves of one) or 4 (four
+// At stride 1 tiles of 16 rows (eight waves of two), 8 (eight waves of one) or 4 (four
 // waves of one): those whose rounds of workgroups over the 256 CUs take least.
 // A round of 16-row tiles is 20 units long, of 8-row ones 13 (a CU holds one
 // of either); a CU holds two 4-row ones, 14 units together and 10 alone. On
@@ -878,22 +882,25 @@ constexpr int kSplitTaps = 9;
 constexpr long kSplitRound16 = 20, kSplitRound8 = 13, kSplitRound4 = 10, kSplitRound4x2 = 14;
 constexpr int kSplitWeights = kSplitTaps * 2 * 192;  // 16-byte groups of a channel block's weights
 
-template <int NW, int WR>
+template <int NW, int WR, int S>
 struct SplitTile {
   static constexpr int T = 64 * NW, TH = NW * WR;             // threads, output rows
-  static constexpr int PR = TH + 2, PC = 18;                  // the patch
+  static constexpr int PR = (TH - 1) * S + 3, PC = 15 * S + 3;  // the patch
+  static constexpr int WK = S == 1 ? 3 : 1;                   // window columns whose weights LDS holds
+  static constexpr int WG = kSplitWeights / 3 * WK;
   static constexpr int NPX = PR * PC;
   static constexpr int UNITS = (NPX * 4 + T - 1) / T;         // (pixel, 8 channels) a thread stages
-  static constexpr int WUNITS = (kSplitWeights + T - 1) / T;
-  static constexpr size_t LDS = size_t(NPX) * 192 + size_t(kSplitWeights) * 16;
+  static constexpr int WUNITS = (WG + T - 1) / T;
+  static constexpr size_t LDS = size_t(NPX) * 192 + size_t(WG) * 16;
 };
 
 // Output (oy, ox) of column n of lane ln by f32 multiply-adds, the taps in
 // row-major order and each one's channels in order; `wt` in the plan's order.
+template <int S>
 __device__ __forceinline__ float conv_f32(const ConvArgs &a, int ln, int oy, int ox, int n) {
   float sum = 0.0f;
   for (int tap = 0; tap < kSplitTaps; tap++) {
-    const int iy = oy - a.pt + tap / 3, ix = ox - a.pl + tap % 3;
+    const int iy = oy * S - a.pt + tap / 3, ix = ox * S - a.pl + tap % 3;
     if (iy < 0 || iy >= a.ih || ix < 0 || ix >= a.iw) continue;
     for (int c = 0; c < a.ctot; c++) {
       const ConvSrc src = pick_src(a, c);
@@ -905,9 +912,9 @@ __device__ __forceinline__ float conv_f32(const ConvArgs &a, int ln, int oy, int
   return sum;
 }
 
-template <int NW, int WR, int GN>
+template <int NW, int WR, int S, int GN>
 __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> grp) {
-  typedef SplitTile<NW, WR> K;
+  typedef SplitTile<NW, WR, S> K;
   constexpr int T = K::T, PC = K::PC, NPX = K::NPX, TW = 16;
   const int bid = xcd_tile((int)blockIdx.x, (int)gridDim.x);
   int prob = 0;
@@ -925,8 +932,11 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
   const int ty0 = (t % tiles_y) * K::TH, ln = t / tiles_y;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lg = lane >> 4;
-  const int iy0 = ty0 - a.pt, ix0 = tx0 - a.pl;
+  const int iy0 = ty0 * S - a.pt, ix0 = tx0 * S - a.pl;
   const int cpt = (a.ctot + 31) / 32;
+  // A stride-2 patch keeps each row's even columns before its odd ones: the
+  // pixels a tap reads lie side by side.
+  auto place = [](int col) { return S == 1 ? col : (col & 1) * ((PC + 1) / 2) + (col >> 1); };
   split_f4 rp[K::UNITS][2];
   split_u4 rw[K::WUNITS];
   const int g = tid & 3, p0 = tid >> 2;
@@ -945,27 +955,33 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
       rp[k][0] = *reinterpret_cast<const split_f4 *>(in ? p : kPatchZeros);
       rp[k][1] = *reinterpret_cast<const split_f4 *>(in ? p + 4 : kPatchZeros);
     }
-    const split_u4 *wsrc = reinterpret_cast<const split_u4 *>(a.split_wt);
+  };
+  const split_u4 *wsrc = reinterpret_cast<const split_u4 *>(a.split_wt);
+  // LDS weight group e: (tap row, window column, block) in turn.
+  auto fetch_w = [&](int cc, int kx) {
 #pragma unroll
     for (int k = 0; k < K::WUNITS; k++) {
-      const int e = min(tid + k * T, kSplitWeights - 1), tj = e / 192;
-      rw[k] = wsrc[((long)tj * cpt + cc) * 192 + (e - tj * 192)];
+      const int e = min(tid + k * T, K::WG - 1), tj = e / 192, kyx = tj >> 1;
+      const int tap = K::WK == 3 ? kyx : kyx * 3 + kx;
+      rw[k] = wsrc[((long)(tap * 2 + (tj & 1)) * cpt + cc) * 192 + (e - tj * 192)];
     }
   };
   auto store = [&]() {
 #pragma unroll
     for (int k = 0; k < K::UNITS; k++) {
-      const int q = p0 + k * (T / 4);
+      const int q = p0 + k * (T / 4), py = q / PC, px = q - py * PC;
       if (q < NPX) {
         split_u4 v[3];
         split8(rp[k][0], rp[k][1], v[0], v[1], v[2]);
 #pragma unroll
-        for (int p = 0; p < 3; p++) P[(p * NPX + q) * 4 + g] = v[p];
+        for (int p = 0; p < 3; p++) P[(p * NPX + py * PC + place(px)) * 4 + g] = v[p];
       }
     }
+  };
+  auto store_w = [&]() {
 #pragma unroll
     for (int k = 0; k < K::WUNITS; k++)
-      if (tid + k * T < kSplitWeights) B[tid + k * T] = rw[k];
+      if (tid + k * T < K::WG) B[tid + k * T] = rw[k];
   };
   const float *bsrc = a.bias ? a.bias : kPatchZeros;
   float bcol[2];
@@ -975,17 +991,25 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
   SplitAcc acc[WR][2] = {};
 
   fetch(0);
+  fetch_w(0, 0);
   for (int cc = 0; cc < cpt; cc++) {
-    if (cc) __syncthreads();  // every wave is done with the previous block
-    store();
-    __syncthreads();
-    if (cc + 1 < cpt) fetch(cc + 1);
-    // The next block's loads stay ahead of this block's multiply-adds.
-    asm volatile("" ::: "memory");
     // Window column by window column: its taps' weights in registers, then
     // every input row of the wave's output rows once.
 #pragma unroll
     for (int kx = 0; kx < 3; kx++) {
+      if (kx == 0 || K::WK == 1) {
+        if (cc || kx) __syncthreads();  // every wave is done with the weights before
+        if (kx == 0) store();
+        store_w();
+        __syncthreads();
+        if (kx == 0 && cc + 1 < cpt) fetch(cc + 1);
+        if (K::WK == 1 && kx < 2)
+          fetch_w(cc, kx + 1);
+        else if (cc + 1 < cpt)
+          fetch_w(cc + 1, 0);
+        // The next loads stay ahead of these multiply-adds.
+        asm volatile("" ::: "memory");
+      }
       bf16x8 bv[3][2][3];
 #pragma unroll
       for (int ky = 0; ky < 3; ky++)
@@ -993,10 +1017,10 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
         for (int j = 0; j < 2; j++)
 #pragma unroll
           for (int p = 0; p < 3; p++)
-            bv[ky][j][p] = __builtin_bit_cast(bf16x8, B[(((ky * 3 + kx) * 2 + j) * 3 + p) * 64 + lane]);
+            bv[ky][j][p] = __builtin_bit_cast(bf16x8, B[((((K::WK == 3 ? ky * 3 + kx : ky) * 2 + j) * 3) + p) * 64 + lane]);
 #pragma unroll
-      for (int r = 0; r < WR + 2; r++) {
-        const int pix = (wave * WR + r) * PC + kx + li;
+      for (int r = 0; r < (WR - 1) * S + 3; r++) {
+        const int pix = (wave * WR * S + r) * PC + place(kx) + li;
         bf16x8 av[3];
 #pragma unroll
         for (int p = 0; p < 3; p++) av[p] = __builtin_bit_cast(bf16x8, P[(p * NPX + pix) * 4 + lg]);
@@ -1004,7 +1028,7 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
         for (int s = 0; s < 6; s++)
 #pragma unroll
           for (int i = 0; i < WR; i++) {
-            const int ky = r - i;
+            const int ky = r - i * S;
             if (ky < 0 || ky > 2) continue;
 #pragma unroll
             for (int j = 0; j < 2; j++) {
@@ -1031,7 +1055,7 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
   while (__builtin_expect(odd != 0, 0)) {
     const int b = __builtin_ctz(odd);
     odd &= odd - 1;
-    const float v = conv_f32(a, ln, ty0 + wave * WR + (b >> 3), tx0 + lg * 4 + (b & 3), (b >> 2 & 1) * 16 + li);
+    const float v = conv_f32<S>(a, ln, ty0 + wave * WR + (b >> 3), tx0 + lg * 4 + (b & 3), (b >> 2 & 1) * 16 + li);
 #pragma unroll
     for (int k = 0; k < WR * 8; k++)
       if (k == b) sum[k >> 3][k >> 2 & 1][k & 3] = v;
@@ -1062,23 +1086,19 @@ __global__ __launch_bounds__(64 * NW) void conv_patch_split(Group<ConvArgs, GN> 
   }
 }
 
-// Stride 1 alone: a stride-2 patch is four times its outputs, one workgroup of
-// it and the weights fills a CU's LDS, and its staging costs what the products
-// save. It won on one small image (48 -> 32 at 56 x 80: 13.3 -> 10.8 us) and
-// lost where there are more tiles than CUs (two such images even, sixteen 37.9
-// -> 50.5 us; 8 channels 19.5 -> 30.2), and the choice cannot follow the number
-// of lanes, whose bits must not depend on each other. From 16 channels on, so
-// that padding them to 32 at most doubles the products: 8 -> 17 at 240 x 184
-// took 8.8 us in f32 and 9.5 split, 16 -> 17 9.3 and 9.2.
+// From 16 channels on at stride 1 and 24 at stride 2, so that what padding them
+// to 32 adds costs less than the bf16 products save: 8 -> 17 at 240 x 184 took
+// 8.8 us in f32 and 9.5 split, 16 -> 17 9.3 and 9.2; at stride 2 16 -> 32 over
+// sixteen maps of 127 x 127 48.6 and 52.4, 24 -> 32 74.4 and 53.7.
 bool patch_split_shape(int kh, int kw, int sh, int sw, int ctot, int n) {
-  return kh == 3 && kw == 3 && sh == 1 && sw == 1 && ctot >= 16 && n > 16 && n <= 32;
+  return kh == 3 && kw == 3 && sh == sw && ((sh == 1 && ctot >= 16) || (sh == 2 && ctot >= 24)) && n > 16 && n <= 32;
 }
 
 size_t patch_split_floats(int ctot) { return size_t(kSplitTaps) * split_pack_floats((ctot + 31) / 32 * 32, 32); }
 
-template <int NW, int WR>
+template <int NW, int WR, int S>
 static hipError_t go_patch_split(const ConvArgs *as, int n, hipStream_t s) {
-  typedef SplitTile<NW, WR> K;
+  typedef SplitTile<NW, WR, S> K;
   Group<ConvArgs> g{};
   long blocks = 0;
   for (int p = 0; p < n; p++) {
@@ -1095,8 +1115,8 @@ static hipError_t go_patch_split(const ConvArgs *as, int n, hipStream_t s) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(K::T), K::LDS, s, gr);
     return hipGetLastError();
   };
-  if (n == 1) return go(conv_patch_split<NW, WR, 1>, group_of<1>(g));
-  return go(conv_patch_split<NW, WR, kGroupStep>, group_of<kGroupStep>(g));
+  if (n == 1) return go(conv_patch_split<NW, WR, S, 1>, group_of<1>(g));
+  return go(conv_patch_split<NW, WR, S, kGroupStep>, group_of<kGroupStep>(g));
 }
 
 hipError_t launch_conv_patch_split_group(const ConvArgs *as, int n, hipStream_t s) {
@@ -1104,7 +1124,7 @@ hipError_t launch_conv_patch_split_group(const ConvArgs *as, int n, hipStream_t 
   long tiles16 = 0, tiles8 = 0, tiles4 = 0;
   for (int p = 0; p < n; p++) {
     const ConvArgs &a = as[p];
-    if (!patch_split_shape(a.kh, a.kw, a.sh, a.sw, a.ctot, a.n) || a.mode != GEMM_STORE || a.gate || a.pw_w ||
+    if (!patch_split_shape(a.kh, a.kw, a.sh, a.sw, a.ctot, a.n) || a.sh != as[0].sh || a.mode != GEMM_STORE || a.gate || a.pw_w ||
         !a.split_wt || a.nsrc < 1 || a.nsrc > 4)
       return hipErrorInvalidValue;
     for (int k = 0; k < a.nsrc; k++)
@@ -1112,12 +1132,13 @@ hipError_t launch_conv_patch_split_group(const ConvArgs *as, int n, hipStream_t 
     const long across = (long)a.lanes * ((a.ow + 15) / 16);
     tiles16 += across * ((a.oh + 15) / 16), tiles8 += across * ((a.oh + 7) / 8), tiles4 += across * ((a.oh + 3) / 4);
   }
+  if (as[0].sh == 2) return go_patch_split<4, 1, 2>(as, n, s);
   auto rounds = [](long tiles) { return (tiles + 255) / 256; };
   const long t16 = rounds(tiles16) * kSplitRound16, t8 = rounds(tiles8) * kSplitRound8;
   const long t4 = rounds(tiles4) / 2 * kSplitRound4x2 + rounds(tiles4) % 2 * kSplitRound4;
-  if (t16 <= t8 && t16 <= t4) return go_patch_split<8, 2>(as, n, s);
-  if (t8 <= t4) return go_patch_split<8, 1>(as, n, s);
-  return go_patch_split<4, 1>(as, n, s);
+  if (t16 <= t8 && t16 <= t4) return go_patch_split<8, 2, 1>(as, n, s);
+  if (t8 <= t4) return go_patch_split<8, 1, 1>(as, n, s);
+  return go_patch_split<4, 1, 1>(as, n, s);
 }
 
 // One wave per row: join the row's tile partials, then y = (best, 1 / sum).

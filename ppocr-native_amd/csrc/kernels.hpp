@@ -208,8 +208,8 @@ hipError_t launch_conv_patch(const ConvArgs &a, int wr, int bk, int bn, hipStrea
 hipError_t launch_conv_patch_group(const ConvArgs *a, int n, int wr, int bk, int bn, hipStream_t s);
 
 // The 3 x 3 window on halo tiles with its products on the bf16 matrix cores
-// (split.hpp): stride 1, 17 to 32 outputs of 16 channels or more, sources of
-// channels a multiple of 8, no gate. n <= kGroupStep problems.
+// (split.hpp): stride 1 or 2, 17 to 32 outputs of enough channels, sources of
+// channels a multiple of 8, no gate. n <= kGroupStep problems of one stride.
 bool patch_split_shape(int kh, int kw, int sh, int sw, int ctot, int n);
 size_t patch_split_floats(int ctot);  // of the weights' parts
 hipError_t launch_conv_patch_split_group(const ConvArgs *a, int n, hipStream_t s);

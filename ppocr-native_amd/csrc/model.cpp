@@ -1374,7 +1374,7 @@ void Model::build_launches(Batch &b) {
             a.wt = W + op.w0, a.wt_k = 0;
             b.launches.push_back({"conv_patch_split", s.op, [a](hipStream_t st) { return launch_conv_patch_split_group(&a, 1, st); }});
             Launch &l = b.launches.back();
-            l.gk = GK_PATCH, l.gkey = -1, l.conv = a, l.bk = bk, l.bn = bn;
+            l.gk = GK_PATCH, l.gkey = -a.sh, l.conv = a, l.bk = bk, l.bn = bn;
             break;
           }
           b.launches.push_back({"conv_patch", s.op, [a, wr, bk, bn](hipStream_t st) {

@@ -140,7 +140,7 @@ def conv_plan(rng, h, w, cs, n, s, act, res):
 
 # Tiles of 4, 8 and 16 rows (few tiles, more, enough for 160 of 16 rows over
 # the lanes), edges that cut them, channels within and past a block of 32, 17
-# to 32 outputs, two sources, a folded Add; 8 channels and stride 2 run in f32.
+# to 32 outputs, both strides, two sources, a folded Add; 8 channels run in f32.
 @pytest.mark.parametrize("h,w,cs,n,s,act,res", [
     (1, 1, (8,), 17, 1, "none", False), (1, 1, (16,), 17, 1, "none", False), (5, 17, (40,), 24, 1, "hardswish", True), (33, 31, (96,), 32, 1, "relu", False),
     (66, 130, (32, 24), 24, 1, "relu", True), (150, 220, (24, 72), 20, 1, "none", False),
@@ -183,15 +183,15 @@ def test_conv_patch_split_near_overflow(oracle, s):
     """An output within 2^-7 of f32's largest value stays finite, its
     neighbours keep their bits."""
     rng = np.random.default_rng(9)
-    b = PlanBuilder(20, 24, 16)
-    wt = rng.normal(0, 0.1, (3, 3, 16, 24)).astype(np.float32)
+    b = PlanBuilder(20, 24, 24)
+    wt = rng.normal(0, 0.1, (3, 3, 24, 24)).astype(np.float32)
     wt[1, 1, 3, 20] = NEAR_W
     plan = b.to_bytes([b.conv(b.input, wt, None, k=(3, 3), s=(s, s), pad=(1, 1, 1, 1))])
-    x = rng.uniform(-1, 1, (20, 24, 16)).astype(np.float32)
+    x = rng.uniform(-1, 1, (20, 24, 24)).astype(np.float32)
     y = x.copy()
     y[8, 10, 3], y[18, 2, 3] = NEAR_X, -NEAR_X
     want = oracle.OracleModel(plan).run(y)[0].reshape(20 // s, 24 // s, 24)
-    a, c = (v.reshape(want.shape) for v in gpu(plan, (20, 24, 16), [x, y]))
+    a, c = (v.reshape(want.shape) for v in gpu(plan, (20, 24, 24), [x, y]))
     assert np.isfinite(want).all() and want[8 // s, 10 // s, 20] > 3.3e38 and want[18 // s, 2 // s, 20] < -3.3e38
     # Sums in another order: 1e-5 of the largest product.
     np.testing.assert_allclose(c, want, rtol=1e-5, atol=1e-5)
@@ -202,10 +202,11 @@ def test_conv_patch_split_near_overflow(oracle, s):
 
 
 @pytest.mark.parametrize("c,n,s,split", [(8, 24, 1, False), (16, 16, 1, False), (16, 17, 1, True), (24, 32, 1, True),
-                                         (24, 33, 1, False), (48, 32, 2, False), (96, 24, 1, True)])
+                                         (24, 33, 1, False), (96, 24, 1, True), (16, 24, 2, False), (24, 17, 2, True),
+                                         (48, 32, 2, True)])
 def test_conv_patch_split_rule(c, n, s, split):
-    """Which layers run split: not stride 2, which is slower on more tiles than
-    CUs, nor channels that padding to 32 more than doubles."""
+    """Which layers run split: not channels so few that padding them to 32
+    costs more than the products save."""
     b = PlanBuilder(20, 24, c)
     wt = np.zeros((3, 3, c, n), np.float32)
     g = GpuModel.load(b.to_bytes([b.conv(b.input, wt, None, k=(3, 3), s=(s, s), pad=(1, 1, 1, 1))]))
@@ -214,19 +215,20 @@ def test_conv_patch_split_rule(c, n, s, split):
     assert names == ["conv_patch_split" if split else "conv_patch"]
 
 
-@pytest.mark.parametrize("h,w,lanes", [(1, 352, 8), (4, 352, 8), (8, 300, 5), (9, 150, 16), (51, 130, 8), (143, 254, 1)])
-def test_conv_patch_split_tiles(oracle, h, w, lanes):
+@pytest.mark.parametrize("h,w,lanes,s", [(1, 352, 8, 1), (4, 352, 8, 1), (8, 300, 5, 1), (9, 150, 16, 1), (51, 130, 8, 1),
+                                         (143, 254, 1, 1), (3, 5, 1, 2), (65, 31, 9, 2), (112, 160, 16, 2)])
+def test_conv_patch_split_tiles(oracle, h, w, lanes, s):
     """Maps of few rows and of rows either side of a tile's, with as many tiles
     as take one round of the CUs and more: a lane's bits are those of the lane
     alone, whichever tiles each takes."""
     rng = np.random.default_rng(h)
-    b = PlanBuilder(h, w, 32)
-    wt = rng.normal(0, 0.06, (3, 3, 32, 24)).astype(np.float32)
-    plan = b.to_bytes([b.conv(b.input, wt, None, k=(3, 3), pad=(1, 1, 1, 1), fused="relu")])
-    xs = [rng.uniform(-1, 1, (h, w, 32)).astype(np.float32) for _ in range(lanes)]
-    got = gpu(plan, (h, w, 32), xs)
+    b = PlanBuilder(h, w, 40)
+    wt = rng.normal(0, 0.06, (3, 3, 40, 24)).astype(np.float32)
+    plan = b.to_bytes([b.conv(b.input, wt, None, k=(3, 3), s=(s, s), pad=(1, 1, 1, 1), fused="relu")])
+    xs = [rng.uniform(-1, 1, (h, w, 40)).astype(np.float32) for _ in range(lanes)]
+    got = gpu(plan, (h, w, 40), xs)
     m = oracle.OracleModel(plan)
     for i in (0, lanes - 1):
-        assert np.array_equal(gpu(plan, (h, w, 32), [xs[i]])[0].view(np.uint32), got[i].view(np.uint32))
+        assert np.array_equal(gpu(plan, (h, w, 40), [xs[i]])[0].view(np.uint32), got[i].view(np.uint32))
         want = m.run(xs[i])[0].reshape(-1).astype(np.float64)
         assert (np.abs(got[i] - want) <= 1e-5 * np.abs(want) + 1e-5).all()
