@@ -833,6 +833,18 @@ static RingTile ring_tile(const std::vector<ConvArgs> &as, long M) {
   return ring_rounds(tiles, lds2) < ring_rounds(tiles, lds3) ? t2 : t;
 }
 
+// `t` where it fits every layer of `as` in LDS, else the 32-column tile with
+// the most stages that does: two at least, since each layer fits a tile of its
+// own. (A gated layer's LDS grows with the lanes that 32 rows span, so a batch
+// of tiny maps may not fit the tile of a large one that shares its launch.)
+static RingTile ring_tile_fitting(const std::vector<ConvArgs> &as, RingTile t) {
+  auto fits = [&](const RingTile &x) {
+    return std::all_of(as.begin(), as.end(), [&](const ConvArgs &a) { return ring_fits(a, x); });
+  };
+  for (int st = 4; !fits(t) && st >= 2; st--) t = RingTile{1, 1, st, 32};
+  return t;
+}
+
 // row n of the packed matrix holds column n's reduction in the kernel's chunk
 // order, zero where the padding of a chunk lies.
 //  - channel layout (every source's channels a multiple of 4): per tap, the
@@ -1397,9 +1409,7 @@ void Model::build_launches(Batch &b) {
             std::vector<ConvArgs> as;
             long M = 0;
             for (const Launch *x : ls) as.push_back(x->conv), M += long(x->conv.lanes) * x->conv.oh * x->conv.ow;
-            RingTile t = ring_tile(as, M);
-            for (const ConvArgs &c : as)
-              if (!ring_fits(c, t)) t = ls[0]->rt;
+            const RingTile t = ring_tile_fitting(as, ring_tile(as, M));
             return [as, t](hipStream_t st) { return launch_conv_ring_group(as.data(), int(as.size()), t, st); };
           };
           break;
@@ -1870,9 +1880,7 @@ void Model::group(Batch &b) const {
           M += long(a.lanes) * a.oh * a.ow;
           same_n = same_n && a.n == as[0].n;
         }
-        RingTile t = same_n ? ring_tile(as, M) : gl.rt;
-        for (const ConvArgs &a : as)
-          if (!ring_fits(a, t)) t = gl.rt;
+        const RingTile t = ring_tile_fitting(as, same_n ? ring_tile(as, M) : gl.rt);
         gl.fn = [as, t](hipStream_t st) { return launch_conv_ring_group(as.data(), int(as.size()), t, st); };
         break;
       }

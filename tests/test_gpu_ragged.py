@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from ppocr_native_amd import GpuModel, nets
+from ppocr_native_amd.planfile import PlanBuilder
 
 pytestmark = pytest.mark.gpu
 
@@ -60,3 +61,18 @@ def test_launch_count():
     plan = nets.recognizer_plan(vocab=500, init="scaled")
     one, two = (check(plan, [[(48, w) for w in ws]], line, times=1) for ws in ([320, 320], [320, 330, 340]))
     assert one == two
+
+
+def test_wide_gate_of_tiny_maps():
+    """A gated 1x1 layer of many channels over one large map and many maps of
+    one pixel: the tile that the large map's rows ask for leaves no room for the
+    gates of the 32 small maps that 32 rows span."""
+    rng = np.random.default_rng(2)
+    w = lambda i, o: rng.normal(0, 1 / np.sqrt(i), (1, 1, i, o)).astype(np.float32)
+    b = PlanBuilder(96, 128, 8)
+    x = b.conv(b.input, w(8, 800), None)
+    g = b.conv(b.mean(x), w(800, 16), None, fused="relu")
+    g = b.conv(g, w(16, 800), None, fused="hardsigmoid")
+    plan = b.to_bytes([b.conv(b.channelmul(x, g), w(800, 96), None)])
+    lane = lambda s, i: np.random.default_rng(100 * i + s[0]).uniform(-1, 1, (*s, 8)).astype(np.float32)
+    check(plan, [[(96, 128)] + [(1, 1)] * 32], lane, times=2)
