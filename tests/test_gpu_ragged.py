@@ -52,6 +52,14 @@ def test_recogniser_widths(logits):
     check(plan, sizes[:1] if logits else sizes, line, times=3)
 
 
+def test_recogniser_widths_many_classes():
+    """Joined heads of so many classes that each line's records cover runs of
+    tiles, its tiles' maxima behind them, where a line alone has a record a
+    tile."""
+    plan = nets.recognizer_plan(vocab=18385, init="scaled")
+    check(plan, [[(48, w) for w in (320, 640, 1100, 801, 960, 333)]], line, times=2)
+
+
 def test_detector_sizes():
     plan = nets.detector_plan(h=64, w=64, init="scaled")
     check(plan, [[(64, 96), (160, 64), (96, 96), (64, 96)]], line)

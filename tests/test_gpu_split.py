@@ -29,10 +29,13 @@ def ctc_plan(rng, t, c, vocab):
 
 
 # Rows below, at and past the 128 of a workgroup; one input group of 32 and
-# four, whole and not; one column, one tile, tiles that do not fill a run; and
-# (4160 rows, 48 tiles) enough workgroups that each walks whole runs.
+# four, whole and not; one column, one tile, tiles that do not fill a run;
+# (4160 rows, 48 tiles) enough workgroups that each walks a whole run, (1280
+# rows, 313 tiles) so many that each walks two, its last a short one; and (640
+# rows, 288 tiles) few enough for single tiles, three a workgroup.
 @pytest.mark.parametrize("lanes,t,c,vocab", [(1, 1, 4, 1), (1, 5, 32, 64), (3, 43, 36, 65), (1, 128, 64, 400),
-                                             (2, 80, 128, 385), (26, 160, 100, 3050)])
+                                             (2, 80, 128, 385), (26, 160, 100, 3050),
+                                             (8, 160, 32, 20000), (4, 160, 64, 18385)])
 def test_ctc_panel(oracle, lanes, t, c, vocab):
     rng = np.random.default_rng(c + vocab)
     plan = ctc_plan(rng, t, c, vocab)
