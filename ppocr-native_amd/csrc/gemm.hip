@@ -1094,8 +1094,6 @@ bool patch_split_shape(int kh, int kw, int sh, int sw, int ctot, int n) {
   return kh == 3 && kw == 3 && sh == sw && ((sh == 1 && ctot >= 16) || (sh == 2 && ctot >= 24)) && n > 16 && n <= 32;
 }
 
-size_t patch_split_floats(int ctot) { return size_t(kSplitTaps) * split_pack_floats((ctot + 31) / 32 * 32, 32); }
-
 template <int NW, int WR, int S>
 static hipError_t go_patch_split(const ConvArgs *as, int n, hipStream_t s) {
   typedef SplitTile<NW, WR, S> K;

@@ -211,7 +211,6 @@ hipError_t launch_conv_patch_group(const ConvArgs *a, int n, int wr, int bk, int
 // (split.hpp): stride 1 or 2, 17 to 32 outputs of enough channels, sources of
 // channels a multiple of 8, no gate. n <= kGroupStep problems of one stride.
 bool patch_split_shape(int kh, int kw, int sh, int sw, int ctot, int n);
-size_t patch_split_floats(int ctot);  // of the weights' parts
 hipError_t launch_conv_patch_split_group(const ConvArgs *a, int n, hipStream_t s);
 
 // The CTC head over rows of ci inputs, rows_per_lane of them per lane:

@@ -1004,6 +1004,8 @@ bool Model::pack(std::string &err) {
     s.ctot = ctot;
     s.cpt = cpt;
     s.wt_k = size_t(s.chunks) * bk;
+    // (A split layer reads its parts, and in f32 the plan's own weights.)
+    if (s.patch_split) continue;
     int n_pad = (N + bn - 1) / bn * bn;
     size_t start = round_up(packed.size(), 64);
     packed.resize(start + size_t(n_pad) * s.wt_k, 0.0f);
@@ -1068,10 +1070,11 @@ bool Model::pack(std::string &err) {
       steps.erase(steps.begin() + long(k) + 1);
     }
   }
-  if (packed.empty()) return true;
-  HIPTRY(hipMalloc(&dpacked, packed.size() * sizeof(float)), "allocating packed weights");
-  HIPTRY(hipMemcpy(dpacked, packed.data(), packed.size() * sizeof(float), hipMemcpyHostToDevice),
-         "uploading packed weights");
+  if (!packed.empty()) {
+    HIPTRY(hipMalloc(&dpacked, packed.size() * sizeof(float)), "allocating packed weights");
+    HIPTRY(hipMemcpy(dpacked, packed.data(), packed.size() * sizeof(float), hipMemcpyHostToDevice),
+           "uploading packed weights");
+  }
   // The bf16 parts of the layers that run on them, made on the GPU.
   if (split_floats) HIPTRY(hipMalloc(&dsplit, split_floats * sizeof(float)), "allocating the weights' parts");
   for (size_t i = 0; i < split_jobs.size(); i++) {
@@ -1372,6 +1375,14 @@ void Model::build_launches(Batch &b) {
           a.pw_n = int(q.oc), a.pw_act = q.fused;
         }
         GemmTile t = s.tile;
+        if (s.patch_split) {
+          a.split_wt = dsplit + s.split_w;
+          a.wt = W + op.w0, a.wt_k = 0;
+          b.launches.push_back({"conv_patch_split", s.op, [a](hipStream_t st) { return launch_conv_patch_split_group(&a, 1, st); }});
+          Launch &l = b.launches.back();
+          l.gk = GK_PATCH, l.gkey = -a.sh, l.conv = a;
+          break;
+        }
         if (s.patch) {
           // Tiles of 8 rows (each wave two MFMA row blocks: half the LDS reads
           // per MFMA) when there is about one per CU or more, else of 4.
@@ -1381,14 +1392,6 @@ void Model::build_launches(Batch &b) {
           const int wr = patch_rows(tiles4, tiles8, patch_fits(a.kh, a.kw, a.sh, 2, t.bk, t.bn),
                                     patch_lds_bytes(a, 1, t.bk, t.bn), patch_lds_bytes(a, 2, t.bk, t.bn));
           const int bk = t.bk, bn = t.bn;
-          if (s.patch_split) {
-            a.split_wt = dsplit + s.split_w;
-            a.wt = W + op.w0, a.wt_k = 0;
-            b.launches.push_back({"conv_patch_split", s.op, [a](hipStream_t st) { return launch_conv_patch_split_group(&a, 1, st); }});
-            Launch &l = b.launches.back();
-            l.gk = GK_PATCH, l.gkey = -a.sh, l.conv = a, l.bk = bk, l.bn = bn;
-            break;
-          }
           b.launches.push_back({"conv_patch", s.op, [a, wr, bk, bn](hipStream_t st) {
                                   return launch_conv_patch(a, wr, bk, bn, st);
                                 }});
@@ -1886,22 +1889,21 @@ void Model::group(Batch &b) const {
       }
       case GK_PATCH: {
         std::vector<ConvArgs> as;
-        long tiles8 = 0, tiles4 = 0;
-        size_t lds4 = 0, lds8 = 0;
-        bool fits2 = true;
-        for (int m : mem) {
-          const Launch &x = b.launches[size_t(m)];
-          as.push_back(x.conv);
-          const long cols = long(x.conv.lanes) * ((x.conv.ow + 15) / 16) * ((x.conv.n + x.bn - 1) / x.bn);
-          tiles8 += cols * ((x.conv.oh + 7) / 8);
-          tiles4 += cols * ((x.conv.oh + 3) / 4);
-          fits2 = fits2 && patch_fits(x.conv.kh, x.conv.kw, x.conv.sh, 2, x.bk, x.bn);
-          lds4 = std::max(lds4, patch_lds_bytes(x.conv, 1, x.bk, x.bn));
-          lds8 = std::max(lds8, patch_lds_bytes(x.conv, 2, x.bk, x.bn));
-        }
+        for (int m : mem) as.push_back(b.launches[size_t(m)].conv);
         if (as[0].split_wt) {
           gl.fn = [as](hipStream_t st) { return launch_conv_patch_split_group(as.data(), int(as.size()), st); };
           break;
+        }
+        long tiles8 = 0, tiles4 = 0;
+        size_t lds4 = 0, lds8 = 0;
+        bool fits2 = true;
+        for (const ConvArgs &a : as) {
+          const long cols = long(a.lanes) * ((a.ow + 15) / 16) * ((a.n + gl.bn - 1) / gl.bn);
+          tiles8 += cols * ((a.oh + 7) / 8);
+          tiles4 += cols * ((a.oh + 3) / 4);
+          fits2 = fits2 && patch_fits(a.kh, a.kw, a.sh, 2, gl.bk, gl.bn);
+          lds4 = std::max(lds4, patch_lds_bytes(a, 1, gl.bk, gl.bn));
+          lds8 = std::max(lds8, patch_lds_bytes(a, 2, gl.bk, gl.bn));
         }
         const int wr = patch_rows(tiles4, tiles8, fits2, lds4, lds8), bk = gl.bk, bn = gl.bn;
         gl.fn = [as, wr, bk, bn](hipStream_t st) {
