@@ -71,8 +71,9 @@ struct __attribute__((packed, aligned(1))) Bytes8 {
 // divisions are paid once for its `per` pixels a thread. Two neighbouring
 // source pixels of a row come by one eight-byte load (at any alignment)
 // where that stays in the row. Bound by the integer work of a pixel.
-// Measured, 2550 x 3300 to 1536 x 1984: 28.3 us with the divisions per pixel
-// and byte loads, now 19.8; to 736 x 960 9.7 and 9.3.
+// Measured, 2550 x 3300 to 1536 x 1984: 26.4 us with the divisions per pixel
+// and byte loads, now 17.4; to 736 x 960 9.9 and 6.8; 1100 x 700 to 1024 x 512
+// 6.5 and 5.6; 331 x 223 to 320 x 224 4.1 both.
 __global__ __launch_bounds__(256) void det_input_kernel(const uint8_t *src, int sw, int sh, float *out, int dw,
                                                         int dh, int per, double xscale, double yscale, double m0,
                                                         double m1, double m2, double s0, double s1, double s2) {
@@ -275,9 +276,11 @@ hipError_t launch_resize(const uint8_t *src, int sw, int sh, uint8_t *dst, int d
 
 hipError_t launch_det_input(const uint8_t *src, int sw, int sh, float *out, int dw, int dh, const double *mean,
                             const double *sd, hipStream_t s) {
-  // Eight pixels a thread when that leaves a block a CU, else two.
+  // Two pixels a thread, four from 2^21 pixels on: the fewer, the more blocks
+  // hide the loads; the more, the fewer tables. Eight left about a block a CU
+  // at 2^19: 1100 x 700 to 1024 x 512 8.6 us, and 6.5 without tables.
   const long n = (long)dw * dh;
-  const int per = n >= 8L * 256 * 256 ? 8 : 2;
+  const int per = n >= (1L << 21) ? 4 : 2;
   hipLaunchKernelGGL(det_input_kernel, dim3(blocks((n + per - 1) / per)), dim3(256), 0, s, src, sw, sh, out, dw, dh, per,
                      tap_scale(sw, dw), tap_scale(sh, dh), mean[0], mean[1], mean[2], sd[0], sd[1], sd[2]);
   return hipGetLastError();

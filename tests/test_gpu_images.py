@@ -46,7 +46,8 @@ def test_det_input_golden():
 
 
 @pytest.mark.parametrize("src,dst", [((3300, 2550), (960, 736)), ((1100, 850), (960, 736)),
-                                     ((700, 500), (704, 512))])
+                                     ((700, 500), (704, 512)), ((30, 40), (32, 32)), ((700, 1100), (512, 1024)),
+                                     ((900, 1800), (1024, 2080))])
 def test_det_input_against_oracle(oracle, src, dst):
     # A letter page at 300 dpi to the detector's 736 x 960 input, and others.
     img = np.random.default_rng(src[0]).integers(0, 256, (*src, 3), dtype=np.uint8)
