@@ -272,8 +272,11 @@ struct Model {
   bool run(bool copy_in, bool copy_out, std::string &err, bool sync = true);
   bool set_db_mask(long output, float thresh, std::string &err);
   bool copy_out_all(std::string &err);
-  // The most bytes a kernel copies to and from the host (the rest by DMA).
-  static constexpr size_t kKernelCopyIn = size_t(1) << 20, kKernelCopyOut = size_t(64) << 20;
+  // The most bytes a kernel copies from the host, and to it per copy that DMA
+  // would take (the rest by DMA, whose copies cost about 5 us each and then
+  // run a little faster: results of 6 MB 151 us by kernel and 156 by DMA, 12
+  // MB 284 and 280, 24 MB 547 and 535, 47 MB 1051 and 1021).
+  static constexpr size_t kKernelCopyIn = size_t(1) << 20, kKernelCopyOut = size_t(8) << 20;
   bool host_copy(const std::vector<CopyArgs> &cs, hipMemcpyKind kind, const char *what, std::string &err);
   std::vector<size_t> step_reads(const Step &s) const;
   int enc_hidden(const Step &s) const { return s.kind == S_ENC_BLOCK ? int(plan.ops[s.m_fc1].oc) : 0; }
@@ -2315,11 +2318,11 @@ bool Model::copy_out_all(std::string &err) {
 }
 
 // Copies between the lanes and their pinned host memory, on the model's
-// stream: by launch_copy, all in one launch.
+// stream: by launch_copy, all in one launch, or, when they are large, by DMA.
 bool Model::host_copy(const std::vector<CopyArgs> &cs, hipMemcpyKind kind, const char *what, std::string &err) {
   size_t bytes = 0;
   for (const CopyArgs &c : cs) bytes += size_t(c.n) * size_t(c.lanes) * sizeof(float);
-  if (bytes <= (kind == hipMemcpyHostToDevice ? kKernelCopyIn : kKernelCopyOut)) {
+  if (bytes <= (kind == hipMemcpyHostToDevice ? kKernelCopyIn : kKernelCopyOut * cs.size())) {
     HIPTRY(launch_copy(cs.data(), int(cs.size()), stream), what);
     return true;
   }

@@ -637,3 +637,20 @@ def test_ctc_argmax_near_ties(oracle):
         assert np.array_equal(a[:, 0], b[:, 0]), np.flatnonzero(a[:, 0] != b[:, 0])
         np.testing.assert_allclose(a[:, 1], b[:, 1], rtol=1e-5, atol=1e-5)
     assert 401 not in {int(v) for gl in got for v in gl[0].reshape(-1, 2)[:, 0]}
+
+
+@pytest.mark.parametrize("lanes,floats", [(1, (2 << 20) - 32), (1, (2 << 20) + 33), (3, (2 << 20) // 3 + 1)])
+def test_results_by_kernel_and_by_dma(lanes, floats):
+    """Results of up to 8 MB come by a copy kernel, larger ones by DMA; odd
+    counts by single floats."""
+    from ppocr_native_amd import GpuModel
+    from ppocr_native_amd.planfile import PlanBuilder
+    b = PlanBuilder(1, floats, 1)
+    g = GpuModel.load(b.to_bytes([b.conv(b.input, np.full((1, 1, 1, 1), 2, np.float32), None)]))
+    g.set_sizes([(1, floats)] * lanes)
+    for i in range(lanes):
+        g.lane_input_mut(i)[:] = np.arange(floats, dtype=np.float32) + i
+    g.run()
+    for i in range(lanes):
+        assert np.array_equal(g.lane_output(i), 2 * (np.arange(floats, dtype=np.float32) + i))
+    g.close()
