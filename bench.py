@@ -33,6 +33,10 @@ if int(os.environ.get("GPU_MAX_HW_QUEUES", "4")) < 8:
     os.environ["GPU_MAX_HW_QUEUES"] = "8"
 PEAK_HBM_GBS = 8000.0
 PEAK_FP32_MFMA_TFLOPS = 157.3
+# Launches whose f32 products run as six bf16 ones (csrc/split.hpp): a sixth of
+# the dense bf16 rate.
+PEAK_SPLIT_TFLOPS = round(2500.0 / 6, 1)
+SPLIT_LAUNCHES = {"conv_patch_split", "ctc_gemm"}
 GEMM_LAUNCHES = {"pointwise_gemm", "conv_gemm", "conv_patch", "conv_patch_split", "convt_gemm", "ctc_gemm"}
 # Launches whose products run as FP32 fused multiply-adds on the vector ALUs
 # (in the CPU engine's order), scored against the unpacked FP32 vector rate:
@@ -43,8 +47,8 @@ VALU_LAUNCHES = {"stem_block"}
 # scaled by a plain copy kernel's counters (x2.0 / x1.0), for the launches
 # the bench reports a roofline of: (kernel, plan operations) -> (read, write)
 # KiB and the profile summary the numbers come from.
-MEASURED_TRAFFIC = {("conv_patch_split", (65, 71, 77, 83)): (31904, 7172, "profiles/hbm_counters_detector_recognizer.md"),
-                    ("conv_patch_split", (94,)): (9420, 5400, "profiles/hbm_counters_detector_recognizer.md")}
+MEASURED_TRAFFIC = {("conv_patch_split", (65, 71, 77, 83)): (31817, 7172, "profiles/hbm_counters_detector_recognizer.md"),
+                    ("conv_patch_split", (94,)): (9428, 5400, "profiles/hbm_counters_detector_recognizer.md")}
 
 
 def package():
@@ -63,14 +67,16 @@ def log(*a):
 
 def roofline(name: str, flops: float, nbytes: float, ms: float) -> dict:
     """A launch's achieved rate against MI355X's peak for its class. A GEMM
-    is also scored against its attainable roof, min(FP32-MFMA peak,
-    arithmetic intensity x HBM peak): a thin 1x1 layer cannot reach the MFMA
-    peak whatever the kernel does."""
+    is also scored against its attainable roof, min(MFMA peak, arithmetic
+    intensity x HBM peak): a thin 1x1 layer cannot reach the MFMA peak
+    whatever the kernel does. The MFMA peak is the one of the products a
+    launch runs: FP32's, or a sixth of bf16's."""
     if name in GEMM_LAUNCHES and flops > 0:
         ach = flops / (ms * 1e-3) / 1e12
-        roof = min(PEAK_FP32_MFMA_TFLOPS, flops / max(nbytes, 1.0) * PEAK_HBM_GBS / 1e3)
-        return {"bound": "mfma", "achieved": round(ach, 3), "peak": PEAK_FP32_MFMA_TFLOPS,
-                "unit": "TFLOP/s", "frac": round(ach / PEAK_FP32_MFMA_TFLOPS, 4),
+        peak = PEAK_SPLIT_TFLOPS if name in SPLIT_LAUNCHES else PEAK_FP32_MFMA_TFLOPS
+        roof = min(peak, flops / max(nbytes, 1.0) * PEAK_HBM_GBS / 1e3)
+        return {"bound": "mfma", "achieved": round(ach, 3), "peak": peak,
+                "unit": "TFLOP/s", "frac": round(ach / peak, 4),
                 "attainable": round(roof, 3), "frac_attainable": round(ach / roof, 4)}
     if name in VALU_LAUNCHES and flops > 0:
         ach = flops / (ms * 1e-3) / 1e12
