@@ -863,11 +863,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void c
 // rows. Reduction order: channel block, window column, input row.
 //
 // What bounds it: the matrix cores, two waves a SIMD that wait together at
-// the block's barriers (LDS holds one workgroup a CU), and on small maps the
-// first loads and the three blocks in turn. Measured against f32 MFMA
-// (conv_patch): 96 -> 24 over four upsampled sources at 496 x 384 98.9 -> 58.6
-// us, the neck's four maps 129.6 -> 79.3; at 240 x 184 28.3 -> 20.8 and 34.3
-// -> 22.0; at 56 x 80 16.3 -> 11.6 and 16.4 -> 13.1. Stride 2, 48 -> 32 to 56 x 80 13.4 -> 10.9, to
+// the block's barriers, and on small maps the first loads and the blocks in
+// turn. Measured against f32 MFMA (conv_patch): 96 -> 24 over four upsampled
+// sources at 496 x 384 97.3 -> 59.8 us, the neck's four maps 126.5 -> 83.3; at
+// 240 x 184 28.7 -> 21.1 and 34.9 -> 22.3; at 56 x 80 16.4 -> 12.2 and 15.8 ->
+// 13.0. Stride 2, 48 -> 32 to 496 x 384 82.2 -> 73.1, to 56 x 80 14.2 -> 11.3, to
 // sixteen of them 37.5 -> 35.3.
 constexpr int kSplitTaps = 9;
 // At stride 1 tiles of 16 rows (eight waves of two), 8 (eight waves of one) or 4 (four
@@ -1326,13 +1326,15 @@ __global__ __launch_bounds__(256) void ctc_merge(Group<CtcArgs, GN> grp, int nti
 // the run's weights meet in that XCD's L2.
 //
 // What bounds it: the matrix cores (the six products of 1280 x 18385 x 120
-// take 17 us at the 2.0 PFLOP/s that bf16 steps reach here) and the epilogue's
-// vector work beside them, two waves a SIMD. Measured on 1280 x 18385 x 120:
-// 45 us; on f32 MFMA 68 us. On 80 rows (one row tile): 11.4 us as 288
+// take 16 us at the 2.08 PFLOP/s that bf16 steps reach here at two waves a
+// SIMD) and the epilogue's vector work beside them. Measured on 1280 x 18385 x
+// 120: 45 us; on f32 MFMA 68 us. On 80 rows (one row tile): 11.3 us as 288
 // workgroups of a tile, 38 us on f32 as 48 of a run. Statistics kept per lane
 // over a run and joined across lanes at its end (less epilogue work, 40 us
 // with runs of three tiles) left the few-row launch at 18 us; three stages
-// instead of two took 44 us.
+// instead of two took 44 us. Both blocks of a half at once, the three
+// accumulators' 48 registers with them, spilled (7 lines of 55 steps 61 us
+// against 59).
 constexpr int kCtcRows = 128;             // rows a workgroup
 constexpr int kCtcWaves = 4;              // waves a workgroup, 128 / (16 * kCtcWaves) row blocks each
 constexpr int kCtcTarget = 512;           // workgroups a launch aims at
@@ -2119,10 +2121,12 @@ hipError_t launch_conv_patch(const ConvArgs &a, int wr, int bk, int bn, hipStrea
 
 hipError_t launch_conv_patch_group(const ConvArgs *as, int n, int wr, int bk, int bn, hipStream_t s) {
   if (n < 1 || n > kGroupStep) return hipErrorInvalidValue;
-  // 17 to 24 columns on 32-column tiles: the 8-column remainder (R8); the
-  // detector head's 3 x 3 (two row blocks a wave) went from 40 to 35 us, the
-  // neck's group (one row block a wave, its patch within four float4s a
-  // thread and the kernel held to three waves per SIMD) from 51 to 46 us.
+  // 17 to 24 columns on 32-column tiles: the 8-column remainder (R8). Measured
+  // on 96 -> 24 at 240 x 240 (two row blocks a wave) 40 -> 35 us, and on four
+  // such layers of 30 to 240 a side (one row block a wave, its patch within
+  // four float4s a thread and the kernel held to three waves per SIMD) 51 ->
+  // 46; layers like those now run split, and gated ones, ones of few or odd
+  // channels run here.
   bool r8 = bn == 32;
   for (int p = 0; p < n; p++) {
     if (!patch_supported(as[p], wr, bk, bn)) return hipErrorInvalidValue;
