@@ -706,8 +706,27 @@ static DwTile dwpw_tile(const DwArgs &d, int p) {
   return DwTile{0, tr, tw, (d.ow + tw - 1) / tw, (d.oh + tr - 1) / tr};
 }
 
-// Pixels of the tiles of n layers (0: not taken).
-static int dwpw_pixels(const DwPwArgs *as, int n) {
+constexpr size_t kDwPwMaxLds = 64 * 1024;
+
+static size_t dwpw_lds_bytes(const DwPwArgs &a, const DwTile &t, int p) {
+  return size_t(dwpw_lds(a.d, a.n, t.tr, t.tw, p, a.res != nullptr).total) * 4;
+}
+
+// dwpw_tile, and of the smallest tile as many rows as LDS takes: a map of one
+// column or row makes it a strip, whose window is several times a square's.
+static DwTile dwpw_tile_cut(const DwPwArgs &a, int p) {
+  DwTile t = dwpw_tile(a.d, p);
+  if (p == 16) {
+    while (t.tr > 1 && dwpw_lds_bytes(a, t, p) > kDwPwMaxLds) t.tr--;
+    while (t.tw > 1 && dwpw_lds_bytes(a, t, p) > kDwPwMaxLds) t.tw--;
+    t.tiles_x = (a.d.ow + t.tw - 1) / t.tw, t.tiles_y = (a.d.oh + t.tr - 1) / t.tr;
+  }
+  return t;
+}
+
+// Pixels of the tiles of n layers (0: not taken). `cut`: tiles may be cut to
+// LDS, for layers that a plan already runs fused and a lane's size does not fit.
+static int dwpw_pixels(const DwPwArgs *as, int n, bool cut) {
   int best = 0;
   for (int p : {64, 32, 16}) {
     long tiles = 0;
@@ -715,9 +734,9 @@ static int dwpw_pixels(const DwPwArgs *as, int n) {
     for (int i = 0; i < n; i++) {
       const DwArgs &d = as[i].d;
       if (!dwpw_shape_ok(d, as[i].n)) return 0;
-      const DwTile t = dwpw_tile(d, p);
+      const DwTile t = cut ? dwpw_tile_cut(as[i], p) : dwpw_tile(d, p);
       tiles += long(d.lanes) * t.tiles_x * t.tiles_y;
-      fits = fits && size_t(dwpw_lds(d, as[i].n, t.tr, t.tw, p, as[i].res != nullptr).total) * 4 <= 64 * 1024;
+      fits = fits && dwpw_lds_bytes(as[i], t, p) <= kDwPwMaxLds;
     }
     if (!fits) continue;
     best = p;
@@ -730,7 +749,7 @@ bool dwpw_supported(const DwArgs &d, int n, bool res) {
   static const float some = 0.0f;
   DwPwArgs a{};
   a.d = d, a.n = n, a.res = res ? &some : nullptr;
-  return dwpw_pixels(&a, 1) > 0;
+  return dwpw_pixels(&a, 1, false) > 0;
 }
 
 template <int K, int S, int RB>
@@ -753,7 +772,7 @@ static hipError_t go_dwpw(const Group<DwPwTileArgs> &g, size_t lds, dim3 grid, h
 
 hipError_t launch_dwpw_group(const DwPwArgs *as, int n, hipStream_t s) {
   if (n < 1 || n > kGroupMax) return hipErrorInvalidValue;
-  const int p = dwpw_pixels(as, n);
+  const int p = dwpw_pixels(as, n, true);
   if (!p) return hipErrorInvalidValue;
   Group<DwPwTileArgs> g{};
   long blocks = 0;
@@ -761,12 +780,12 @@ hipError_t launch_dwpw_group(const DwPwArgs *as, int n, hipStream_t s) {
   for (int i = 0; i < n; i++) {
     const DwArgs &d = as[i].d;
     if (!as[i].pw || !as[i].y || d.kh != as[0].d.kh || d.sw != as[0].d.sw || as[i].n != as[0].n) return hipErrorInvalidValue;
-    const DwTile t = dwpw_tile(d, p);
+    const DwTile t = dwpw_tile_cut(as[i], p);
     g.first[i] = (int)blocks;
     g.a[i] = DwPwTileArgs{as[i], t};
     blocks += long(d.lanes) * t.tiles_y * t.tiles_x;
     if (blocks < 1 || blocks > 0x7fffffffL) return hipErrorInvalidValue;
-    lds = std::max(lds, size_t(dwpw_lds(d, as[i].n, t.tr, t.tw, p, as[i].res != nullptr).total) * 4);
+    lds = std::max(lds, dwpw_lds_bytes(as[i], t, p));
   }
   g.n = n, g.first[n] = (int)blocks;
   const dim3 grid((unsigned)blocks);

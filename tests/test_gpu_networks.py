@@ -51,6 +51,22 @@ def test_detector(oracle, init, h, w):
     assert err.max() <= 4e-5
 
 
+@pytest.mark.parametrize("h,w", [(32, 128), (32, 416), (288, 32), (32, 32)])
+def test_detector_strips(oracle, h, w):
+    """Sides of 32, whose last maps are one row or column: the fused depthwise
+    and 1x1 layers' tiles are strips there."""
+    img = nets.page_image(h, w)
+    g = GpuModel.load(nets.detector_plan(h=64, w=64, init="scaled"))
+    g.set_sizes([(h, w), (h, w), (96, 64)])
+    for i in range(2):
+        g.lane_input_mut(i)[:] = img.reshape(-1)
+    g.run()
+    want = oracle.OracleModel(nets.detector_plan(h=h, w=w, init="scaled")).run(img)[0]
+    for i in range(2):
+        assert np.abs(g.lane_output(i).astype(np.float64) - want).max() <= 4e-5
+    g.close()
+
+
 def check_rec(got, want):
     g, o = got.reshape(-1, 2), want.reshape(-1, 2)
     assert np.array_equal(g[:, 0], o[:, 0]), np.flatnonzero(g[:, 0] != o[:, 0])
